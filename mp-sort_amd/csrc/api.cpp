@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "internal.h"
+#include "direct.h"
 #include "lsort.h"
 #include "model.h"
 #include "../../include/mpsort_gpu.h"
@@ -1626,6 +1627,211 @@ static int plain_bucket_first(DevCtx& c, const CallShape& cs, const SegSortPlan&
     return 0;
 }
 
+// ---- the sort without per-rank local sorts (direct.hip) ----------------------
+// Taken by the allocating plain path when nothing asks for another form (an
+// exchange, a FirstSort form, a fault hook): up to kDirectMaxP ranks, 8- or
+// 16-byte sort records with keys of at most 8 bytes.  One partition pass has
+// at most kLBins buckets, each at most about the in-LDS capacity of 4608
+// records: kDirectMaxRecords.
+constexpr int64_t kDirectMaxRecords = (int64_t)kLBins * 4200;
+constexpr int64_t kDirectMinRecords = 8193;
+constexpr int64_t kDirectAvg = 2048;   // records per bucket while kLBins buckets suffice
+static bool direct_eligible(const CallShape& cs) {
+    return !g_faults && !cs.exchange && cs.first_mode == 0 && cs.P <= kDirectMaxP && (cs.rw == 2 || cs.rw == 4) &&
+           cs.ks.key_bytes <= 8 && cs.ntot >= kDirectMinRecords && cs.ntot <= kDirectMaxRecords;
+}
+
+static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
+                      const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats) {
+    hipStream_t st = c.st;
+    const int P = cs.P, rw = cs.rw;
+    const int64_t n = cs.ntot;
+    const size_t recbytes = (size_t)rw * 4;
+    int rc = 0;
+
+    DirectShape sh;
+    memset(&sh, 0, sizeof sh);
+    sh.P = P;
+    sh.n = n;
+    sh.tile = lscatter_tile(rw);
+    for (int t = 0; t < P; t++) {
+        sh.begin[t + 1] = sh.begin[t] + nin[t];
+        sh.C[t + 1] = sh.C[t] + nout[t];
+        sh.tile_start[t + 1] = sh.tile_start[t] + (nin[t] + sh.tile - 1) / sh.tile;
+    }
+    sh.ntiles = sh.tile_start[P];
+    sh.W = (int)std::min<int64_t>(kLBins, std::max<int64_t>(2, (n + kDirectAvg - 1) / kDirectAvg));
+    sh.S = std::min(kDirectMaxChunks, (16 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
+    const bool small_form = false;
+
+    // ---- workspace
+    Sizer sz;
+    lay_hist(sz, P, nullptr);
+    if ((rc = c.small.ensure(sz.off + 4096))) return rc;
+    Arena ar{(char*)c.small.p};
+    HistArrays h;
+    lay_hist(ar, P, &h);
+    DirectWork w;
+    auto lay = [&](auto& a, auto take) {
+        take(a, w.begin, (size_t)P);
+        take(a, w.count, (size_t)P);
+        take(a, w.tile_start, (size_t)P + 1);
+        take(a, w.chunks, (size_t)sh.S);
+        take(a, w.raw, (size_t)kLBins);
+        take(a, w.tables, (size_t)kLBins);
+        take(a, w.tot, (size_t)kLBins);
+        take(a, w.base, (size_t)kLBins);
+        take(a, w.lists, (size_t)8);
+        take(a, w.hard, (size_t)kLBins);
+        take(a, w.medium, (size_t)kLBins);
+        take(a, w.overflow, (size_t)2 * kLBins);
+        take(a, w.cross, (size_t)kDirectMaxP * kDirectMaxP);
+        take(a, w.tile_cnt, (size_t)sh.ntiles * kLBins);
+        take(a, w.tile_off, (size_t)sh.ntiles * kLBins);
+        take(a, w.bkt, (size_t)n);
+    };
+    Sizer lz;
+    lay(lz, [](Sizer& a, auto*& p, size_t k) { a.take<std::remove_reference_t<decltype(*p)>>(k); });
+    if ((rc = c.ltile.ensure(lz.off + 4096))) return rc;
+    Arena la{(char*)c.ltile.p};
+    lay(la, [](Arena& a, auto*& p, size_t k) { p = a.take<std::remove_reference_t<decltype(*p)>>(k); });
+    w.C = h.C;
+    w.err = h.err;
+    w.checksum = h.checksum;
+    w.myclt = h.myclt;
+    w.mycle = h.mycle;
+    w.myC = h.myC;
+    w.send = h.send;
+    w.split = h.split;
+    w.pminmax = h.pminmax;
+    if ((rc = c.s1.ensure((size_t)n * recbytes))) return rc;
+    if (cs.general && ((rc = c.rbuf.ensure((size_t)n * recbytes)) || (rc = c.s0.ensure((size_t)n * recbytes)))) return rc;
+    if ((rc = ensure_rpin(c, sizeof(DirectResult) + 256))) return rc;
+    DirectResult* res = (DirectResult*)pin_take(c, sizeof(DirectResult));
+    if (!res) return fail(MPSORT_ERR_HIP, "no pinned memory for the results");
+
+    // ---- the sort
+    // (the timing events ride on the launches they bracket: an event recorded
+    // between two launches costs the GPU about 4.5 us)
+    const LKey lk = make_lkey(cs.ks);
+    const void* src = d_in;
+    void* dst = d_out;
+    if (cs.general) {
+        MPSG_CHECK(hipEventRecord(c.ev[kEvStart], st));
+        src = c.rbuf.p;
+        dst = c.s0.p;
+        if (packed_host) MPSG_CHECK(hipMemcpyAsync(c.rbuf.p, packed_host, n * recbytes, hipMemcpyHostToDevice, st));
+    }
+    // the sample launch clears the checksums, so the pack comes after it
+    // unless the sample reads packed records: then it clears them itself
+    if (cs.general && !packed_host) {
+        if ((rc = launch_fill_u32((uint32_t*)w.checksum, 0u, 4, st)) ||
+            (rc = launch_pack(d_in, n, cs.elsize, cs.key_off_user, cs.key_bytes_user, c.rbuf.p, rw, cs.iwords,
+                              cs.checksum ? w.checksum : nullptr, st)))
+            return rc;
+    }
+    const bool cs_direct = cs.checksum && !cs.general;
+    long long* cs_in = cs_direct ? w.checksum : nullptr;
+    long long* cs_out = cs_direct ? w.checksum + 1 : nullptr;
+    void* tmp = c.s1.p;
+    // single-value buckets go straight to the output unless it overlaps the
+    // records still to be read
+    const char *sa = (const char*)src, *da = (const char*)dst;
+    const bool eq_direct = sa >= da + (size_t)n * recbytes || da >= sa + (size_t)n * recbytes;
+    hipEvent_t* pe = cs.timing ? c.pass_ev[0] : nullptr;
+    auto mark = [&](int i) -> int {
+        if (pe) MPSG_CHECK(hipEventRecord(pe[i], st));
+        return 0;
+    };
+    const SegDev sd{w.begin, w.count, w.tile_start, P, 0};
+    if ((rc = mark(0)) || (rc = launch_direct_sample(rw, src, lk, sh, w, !(cs.general && !packed_host),
+                                                 cs.general ? nullptr : c.ev[kEvStart], st)) ||
+        (rc = mark(1)) || (rc = launch_direct_count(rw, src, lk, sh, w, cs_in, st)) || (rc = mark(2)) ||
+        (rc = launch_lscatter(rw, src, tmp, eq_direct ? dst : tmp, sd, sh.ntiles, w.bkt, w.tables, 0, w.tile_off,
+                              w.err + 1, st, w.tot, n, w.base)) ||
+        (rc = mark(3)) ||
+        (rc = launch_chunk_sort_small(rw, tmp, dst, lk, w.tot, w.base, w.tables, 0, sh.W, w.overflow, w.lists, kLBins,
+                                      w.hard, w.lists + 1, w.medium, w.lists + 2, cs_out, eq_direct, st, nullptr,
+                                      (uint32_t)kChunkCap, small_form, c.ev[kEvFirst])) ||
+        (rc = mark(4)))
+        return rc;
+    auto finish = [&]() -> int {
+        int r2 = 0;
+        if (cs.general &&
+            (r2 = launch_gather(d_in, n, cs.elsize, dst, rw, cs.iwords, d_out, cs.checksum ? w.checksum + 1 : nullptr,
+                                w.err, st)))
+            return r2;
+        if ((r2 = launch_direct_counts(rw, dst, tmp, lk, sh, w, eq_direct, res, c.ev[kEvEnd], st))) return r2;
+        MPSG_CHECK(hipStreamSynchronize(st));
+        return 0;
+    };
+    if ((rc = finish())) return rc;
+    DirectResult got = *res;
+    if (got.scatter_err) return fail(MPSORT_ERR_TIMEOUT, "bucket scatter: device flag 0x%x", got.scatter_err);
+    if (got.lists[0] | got.lists[1] | got.lists[2]) {
+        // buckets above the workgroup's capacity, then the crowded ones, then
+        // those above the in-LDS capacity; the counts again afterwards
+        if ((rc = launch_listed_sort(rw, tmp, dst, lk, w.medium, got.lists[2], w.tot, w.base, w.tables, kLBins, 0,
+                                     w.hard, w.lists + 1, cs_out, st)) ||
+            (rc = launch_lsd_sort(rw, tmp, dst, lk, w.tot, w.base, w.hard, w.lists + 1, sh.W, cs_out, st)))
+            return rc;
+        if (got.lists[0]) {
+            SegSortPlan plain;
+            plain.rw = rw;
+            plain.ks = cs.ks;
+            plain.d_checksum = w.checksum;
+            const TileCfg tc = default_tile(rw);
+            const int64_t nt = n / ((int64_t)tc.block * tc.items) + kMaxFallbackSegs + 1;
+            if ((rc = c.lookback.ensure((size_t)nt * kBins * sizeof(uint64_t))) ||
+                (rc = c.s2.ensure((size_t)n * recbytes)) ||
+                (rc = sort_listed_segments(c, plain, rw, w.overflow, got.lists[0], tmp, dst, c.s2.p, cs_out, st)))
+                return rc;
+        }
+        MPSG_CHECK(hipEventRecord(c.ev[kEvFirst], st));
+        // the first gather may have met records not yet in place
+        if (cs.general && ((rc = launch_fill_u32(w.err, 0u, 1, st)) ||
+                           (rc = launch_fill_u32((uint32_t*)(w.checksum + 1), 0u, 2, st))))
+            return rc;
+        if ((rc = finish())) return rc;
+        got = *res;
+    }
+
+    stats->nvranks = P;
+    stats->second_merged = P > 1 ? 1 : 0;
+    stats->buckets = sh.W;
+    stats->buckets_overflow = stats->buckets_overflow_first = (int32_t)got.lists[0];
+    stats->buckets_lds_radix = (int32_t)got.lists[1];
+    stats->buckets_listed = (int32_t)got.lists[2];
+    stats->record_bytes = (int32_t)recbytes;
+    stats->general_path = cs.general ? 1 : 0;
+    stats->nrecords = n;
+    stats->checksum_in = got.sums[0];
+    stats->checksum_out = got.sums[1];
+    stats->t_first_sort_ms = ev_ms(c.ev[kEvStart], c.ev[kEvFirst]);
+    stats->t_findp_ms = ev_ms(c.ev[kEvFirst], c.ev[kEvEnd]);  // with the layout
+    stats->t_total_ms = ev_ms(c.ev[kEvStart], c.ev[kEvEnd]);
+    if (pe) {
+        for (int i = 0; i < 4; i++) stats->pass_ms[i] = ev_ms(pe[i], pe[i + 1]);
+        stats->npass_ms = 4;
+    }
+    c.last_P = P;
+    c.C = h.C;
+    c.myclt = h.myclt;
+    c.mycle = h.mycle;
+    c.myC = h.myC;
+    c.send = h.send;
+    c.split = h.split;
+    c.pminmax = h.pminmax;
+    c.last_ntot = n;
+    if (got.err)
+        return fail(MPSORT_ERR_LAYOUT, "layout check failed (device flags 0x%x): the splitter counts or layout solve "
+                                       "is inconsistent", got.err);
+    if (cs.checksum && !packed_host && got.sums[0] != got.sums[1])
+        return fail(MPSORT_ERR_CHECKSUM, "MPSort: Data changed after sorting; checksum mismatch (%lld != %lld)",
+                    got.sums[0], got.sums[1]);
+    return 0;
+}
+
 static int run_histsort_learned(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out,
                                 const int64_t* nin, const int64_t* nout, const LearnedModel& M,
                                 mpsort_gpu_stats* stats) {
@@ -2412,6 +2618,7 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
     memset(&st, 0, sizeof st);
     remember_key(*c, key, 0, 0);
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
+        if (direct_eligible(cs)) return run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st);
         HistWork w;
         int r2 = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
         return r2 ? r2 : run_histsort(*c, cs, d_in, d_out, nin, nout, nullptr, &st, w);
@@ -2660,9 +2867,13 @@ int mpsort_gpu_newarray_radix(const void* base, const int64_t* nin, int P, void*
     // the gather's device checksum covers the output; the input sum is the
     // host's (the device sees only the packed records)
     cs.checksum = !(flags & MPSORT_GPU_NO_CHECKSUM);
-    HistWork w;
-    rc = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
-    if (!rc) rc = run_histsort(*c, cs, c->din.p, c->dout.p, nin, nout, packed, &st, w);
+    if (direct_eligible(cs)) {
+        rc = run_direct(*c, cs, c->din.p, c->dout.p, nin, nout, packed, &st);
+    } else {
+        HistWork w;
+        rc = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
+        if (!rc) rc = run_histsort(*c, cs, c->din.p, c->dout.p, nin, nout, packed, &st, w);
+    }
     mpiu_free(packed, __FILE__, __LINE__);
     if (!rc) {
         MPSG_CHECK(hipMemcpy(out, c->dout.p, bytes, hipMemcpyDeviceToHost));

@@ -1,0 +1,494 @@
+// direct.hip -- the sort of up to 64 ranks without per-rank local sorts: the
+// records of all ranks are partitioned into key buckets (boundaries from a
+// sorted sample), every bucket is sorted in LDS into the output, and the
+// splitters and counts of the histogram sort (mpsort-mpi.c:375-510) are read
+// off the result.  The reference's FirstSort, exchange and SecondSort
+// (mpsort-mpi.c:369,571-597) produce that same stable order.
+#include <hip/hip_ext.h>
+
+#include "direct.h"
+#include "lsort_dev.h"
+
+namespace mpsg {
+
+// ---------------------------------------------------------------------------
+// Sample.  Block c takes the keys at positions (2u + 1) n / 2S, u = 1024 c ..
+// 1024 c + 1023, and sorts them: one key per thread, a bitonic network whose
+// strides below 64 are lane exchanges and whose ten larger ones go through
+// LDS.  Block 0 also writes the call's tables and clears its counters (every
+// later kernel of the call reads them).
+__device__ __forceinline__ uint64_t bitonic1024(uint64_t v, uint64_t* s_k) {
+    const int tid = threadIdx.x;
+    for (int size = 2; size <= kDirectChunk; size <<= 1) {
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            uint64_t o;
+            if (stride >= 64) {
+                s_k[tid] = v;
+                __syncthreads();
+                o = s_k[tid ^ stride];
+                __syncthreads();
+            } else {
+                o = __shfl_xor(v, stride, 64);
+            }
+            const bool lower = (tid & stride) == 0, up = (tid & size) == 0;
+            v = (lower == up) ? (o < v ? o : v) : (o > v ? o : v);
+        }
+    }
+    return v;
+}
+
+// boundary q (1 .. W - 1) is the smallest sample rank r with (r + 1) W >= q S
+__device__ __forceinline__ void put_boundary(uint64_t key, int rank, int S, int W, uint64_t* raw) {
+    const int64_t x = (int64_t)(rank + 1) * W;
+    const int q = (int)(x / S);
+    if (q >= 1 && q < W && x - (int64_t)q * S < W) raw[q - 1] = key;
+}
+
+template <int RW>
+__global__ __launch_bounds__(kDirectChunk) void direct_sample_kernel(const uint32_t* __restrict__ src, LKey lk,
+                                                                     DirectShape sh, DirectWork w,
+                                                                     int clear_sums) {
+    __shared__ uint64_t s_k[kDirectChunk];
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0) {
+        if (tid <= sh.P) {
+            w.C[tid] = sh.C[tid];
+            w.tile_start[tid] = sh.tile_start[tid];
+            if (tid < sh.P) {
+                w.begin[tid] = sh.begin[tid];
+                w.count[tid] = sh.begin[tid + 1] - sh.begin[tid];
+            }
+        }
+        if (tid < 8) w.lists[tid] = 0;
+        if (tid < 4) w.err[tid] = 0;
+        if (tid < 2 && clear_sums) w.checksum[tid] = 0;
+    }
+    const int64_t u = (int64_t)blockIdx.x * kDirectChunk + tid;
+    const int64_t pos = ((2 * u + 1) * sh.n) / (2 * (int64_t)sh.S);
+    uint32_t r[RW];
+    RecIO<RW>::load(src, pos, r);
+    const uint64_t v = bitonic1024(lkey<RW>(r, lk), s_k);
+    if (sh.S == kDirectChunk) put_boundary(v, tid, sh.S, sh.W, w.raw);
+    else w.chunks[u] = v;
+}
+
+// The rank of every sample key among all chunks (equal keys in chunk order):
+// its index in its own chunk plus a binary search in each other chunk, 16
+// chunks staged in LDS at a time so that 16 searches advance together
+// (8 loads of a thread in flight while a stage is copied in).
+constexpr int kRankBlock = 256, kRankStage = 16;
+__global__ __launch_bounds__(kRankBlock) void direct_rank_kernel(int S, int W, const uint64_t* __restrict__ chunks,
+                                                                 uint64_t* __restrict__ raw) {
+    __shared__ __attribute__((aligned(16))) uint64_t s_k[kRankStage * kDirectChunk];
+    const int nch = S / kDirectChunk, tid = threadIdx.x;
+    const int g = blockIdx.x * kRankBlock + tid;
+    const int mine = g / kDirectChunk;
+    const uint64_t key = chunks[g];
+    int rank = g % kDirectChunk;
+    for (int c0 = 0; c0 < nch; c0 += kRankStage) {
+        const int m = min(kRankStage, nch - c0);
+        __syncthreads();
+        const uint4* from = reinterpret_cast<const uint4*>(chunks + (int64_t)c0 * kDirectChunk);
+        uint4* to = reinterpret_cast<uint4*>(s_k);
+        constexpr int U = 8;
+        const int words = m * kDirectChunk / 2;  // a multiple of kRankBlock
+        for (int i = tid; i < words; i += U * kRankBlock) {
+            uint4 x[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) x[u] = from[min(i + u * kRankBlock, words - 1)];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (i + u * kRankBlock < words) to[i + u * kRankBlock] = x[u];
+        }
+        __syncthreads();
+        int lo[kRankStage];
+#pragma unroll
+        for (int c = 0; c < kRankStage; c++) lo[c] = 0;
+#pragma unroll
+        for (int step = kDirectChunk / 2; step > 0; step >>= 1) {
+#pragma unroll
+            for (int c = 0; c < kRankStage; c++) {
+                if (c < m) {
+                    const uint64_t x = s_k[c * kDirectChunk + lo[c] + step - 1];
+                    // chunks before this one: #{<= key}; after it: #{< key}
+                    if (c0 + c < mine ? x <= key : x < key) lo[c] += step;
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < kRankStage; c++) {
+            if (c < m && c0 + c != mine) {
+                const uint64_t x = s_k[c * kDirectChunk + lo[c]];
+                rank += lo[c] + ((c0 + c < mine ? x <= key : x < key) ? 1 : 0);
+            }
+        }
+    }
+    put_boundary(key, rank, S, W, raw);
+}
+
+// ---------------------------------------------------------------------------
+// Bucket of every record and the tiles' bucket counts.  The boundary table is
+// made from the raw sample keys by every block (block 0 keeps it): where
+// boundaries repeat a key v, the first of them becomes v - 1, so that
+// (v - 1, v] holds that key alone; entries past W - 2 are the largest key.
+// The searches of a thread's U records advance together.
+template <int RW>
+__global__ __launch_bounds__(512) void direct_hist_kernel(const uint32_t* __restrict__ src, SegDev seg, int64_t ntiles,
+                                                          int64_t tpb, int tile_recs, LKey lk, int W, int step0,
+                                                          const uint64_t* __restrict__ raw,
+                                                          uint64_t* __restrict__ tables,
+                                                          uint16_t* __restrict__ tile_cnt, uint16_t* __restrict__ bkt,
+                                                          long long* __restrict__ checksum) {
+    constexpr int BLOCK = 512, U = RW == 2 ? 4 : 3;
+    __shared__ uint64_t s_tab[kLBins];
+    __shared__ uint32_t s_th[kLBins];
+    __shared__ long long s_sum[BLOCK / 64];
+    const int tid = threadIdx.x;
+    for (int e = tid; e < kLBins; e += BLOCK) {
+        uint64_t t = ~0ull;
+        if (e < W - 1) {
+            const uint64_t v = raw[e];
+            const bool first = e == 0 || raw[e - 1] < v;
+            const bool repeated = e + 1 < W - 1 && raw[e + 1] == v;
+            t = first && repeated && v > 0 ? v - 1 : v;
+        }
+        s_tab[e] = t;
+        s_th[e] = 0;
+        if (blockIdx.x == 0 && e < kLBounds) tables[e] = t;
+    }
+    __syncthreads();
+    const int64_t t0 = (int64_t)blockIdx.x * tpb, t1 = min(ntiles, t0 + tpb);
+    long long csum = 0;
+    for (int64_t tile = t0; tile < t1; tile++) {
+        const int s = seg_of_tile(seg, tile);
+        const int64_t sbeg = seg.begin[s];
+        const int64_t begin = sbeg + (tile - seg.tile_start[s]) * tile_recs;
+        const int64_t end = min(sbeg + seg.count[s], begin + (int64_t)tile_recs);
+        for (int64_t i0 = begin + tid; i0 < end; i0 += U * BLOCK) {
+            uint32_t r[U][RW];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int64_t i = i0 + (int64_t)u * BLOCK;
+                RecIO<RW>::load(src, i < end ? i : end - 1, r[u]);
+            }
+            uint64_t k[U];
+            int lo[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                k[u] = lkey<RW, true>(r[u], lk);
+                lo[u] = 0;
+            }
+            for (int step = step0; step > 0; step >>= 1) {
+                uint64_t v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) v[u] = s_tab[min(lo[u] + step - 1, kLBounds)];
+#pragma unroll
+                for (int u = 0; u < U; u++) lo[u] += (v[u] < k[u] && lo[u] + step <= kLBounds) ? step : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int64_t i = i0 + (int64_t)u * BLOCK;
+                if (i < end) {
+                    if (checksum) {
+#pragma unroll
+                        for (int q = 0; q < RW; q++) csum += sbyte_sum(r[u][q]);
+                    }
+                    bkt[i] = (uint16_t)lo[u];
+                    atomicAdd(&s_th[lo[u]], 1u);
+                }
+            }
+        }
+        __syncthreads();
+        for (int b = tid; b < kLBins; b += BLOCK) {
+            tile_cnt[tile * kLBins + b] = (uint16_t)s_th[b];
+            s_th[b] = 0;
+        }
+        __syncthreads();
+    }
+    if (checksum) {
+        csum = wave_sum_ll(csum);
+        if ((tid & 63) == 0) s_sum[tid >> 6] = csum;
+        __syncthreads();
+        if (tid == 0) {
+            long long a = 0;
+            for (int q = 0; q < BLOCK / 64; q++) a += s_sum[q];
+            atomicAdd((unsigned long long*)checksum, (unsigned long long)a);
+        }
+    }
+}
+
+// tile_off[t][b] = bucket b's records in the tiles before t, and the totals:
+// a block per 64 buckets, its 16 waves over equal runs of tiles (counts
+// summed, prefixed over the waves, then walked again)
+__global__ __launch_bounds__(1024) void direct_scan_kernel(const uint16_t* __restrict__ tile_cnt, int64_t ntiles,
+                                                           uint32_t* __restrict__ tile_off, uint32_t* __restrict__ tot) {
+    __shared__ uint32_t s_part[16][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int b = blockIdx.x * 64 + lane;
+    const int64_t per = (ntiles + 15) / 16;
+    const int64_t t0 = min(ntiles, wave * per), t1 = min(ntiles, t0 + per);
+    constexpr int U = 16;
+    uint32_t sum = 0;
+    for (int64_t t = t0; t < t1; t += U) {
+        uint32_t c[U];
+#pragma unroll
+        for (int q = 0; q < U; q++) c[q] = t + q < t1 ? tile_cnt[(t + q) * kLBins + b] : 0u;
+#pragma unroll
+        for (int q = 0; q < U; q++) sum += c[q];
+    }
+    s_part[wave][lane] = sum;
+    __syncthreads();
+    uint32_t run = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const uint32_t c = s_part[q][lane];
+        run += q < wave ? c : 0u;
+        all += c;
+    }
+    if (wave == 0) tot[b] = all;
+    for (int64_t t = t0; t < t1; t += U) {
+        uint32_t c[U];
+#pragma unroll
+        for (int q = 0; q < U; q++) c[q] = t + q < t1 ? tile_cnt[(t + q) * kLBins + b] : 0u;
+#pragma unroll
+        for (int q = 0; q < U; q++) {
+            if (t + q < t1) tile_off[(t + q) * kLBins + b] = run;
+            run += c[q];
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Splitters, counts and layout.  Splitter i = key of output record C[i+1] - 1
+// (the smallest key when C[i+1] is 0, where the reference's bisection ends).
+// Block j counts rank j's records below every splitter: its records in the
+// buckets before the splitter's (a prefix over the buckets of its tiles'
+// offsets: a rank's run in a bucket starts where its first tile's does), plus
+// those of its run in that bucket that are smaller (or equal), a wave per
+// splitter.  The block that finishes last solves the layout
+// (_solve_for_layout_mpi mpsort-mpi.c:663-727): a wave per receiver, a lane
+// per sender (the greedy fill from sender 0 as a prefix over the senders'
+// supplies), then the send counts and the call's results.  Block j reads two
+// rows of offsets; a block per splitter, which read 2 P rows each, took 43
+// instead of 12 us at 64 ranks, and the layout in a launch of its own 13 more.
+__device__ __forceinline__ uint32_t incl_scan_u32(uint32_t v) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(v, off, 64);
+        if (lane >= off) v += o;
+    }
+    return v;
+}
+
+template <int RW>
+__global__ __launch_bounds__(1024) void direct_counts_kernel(const uint32_t* __restrict__ out,
+                                                             const uint32_t* __restrict__ part, LKey lk, int P,
+                                                             int64_t n, int64_t ntiles, DirectWork w, int eq_done,
+                                                             DirectResult* __restrict__ res) {
+    constexpr int BLOCK = 1024, NW = BLOCK / 64, Q = kDirectMaxP / NW;  // splitters (receivers) per wave
+    __shared__ uint64_t s_tab[kLBins];
+    __shared__ uint32_t s_pref[kLBins];
+    __shared__ uint32_t s_tmp[NW];
+    __shared__ uint64_t s_v[kDirectMaxP];
+    __shared__ int s_b[kDirectMaxP];
+    __shared__ uint32_t s_c[kDirectMaxP + 1][kDirectMaxP];  // [receiver edge][sender]
+    __shared__ uint32_t s_err;
+    __shared__ int s_last;
+    const int j = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int P1 = P + 1;
+    if (tid == 0) s_err = 0;
+    if (P > 1) {
+        s_tab[tid] = tid < kLBounds ? w.tables[tid] : ~0ull;
+        const int64_t ta = w.tile_start[j], tb = w.tile_start[j + 1];
+        const uint32_t* oa = w.tile_off + ta * kLBins;
+        const uint32_t* ob = tb >= ntiles ? w.tot : w.tile_off + tb * kLBins;
+        const uint32_t mine = ta < tb ? ob[tid] - oa[tid] : 0u;
+        s_pref[tid] = scan_block<BLOCK>(mine, s_tmp);
+        if (tid < P - 1) {
+            const int64_t Ci = w.C[tid + 1];
+            uint32_t r[RW];
+            RecIO<RW>::load(out, Ci > 0 ? Ci - 1 : 0, r);
+            const uint64_t v = lkey<RW>(r, lk);
+            s_v[tid] = v;
+            s_b[tid] = (int)bucket_of(v, s_tab);  // s_tab is complete: scan_block has barriers
+            if (j == 0) {
+                w.split[4 * tid] = v;
+                w.split[4 * tid + 1] = w.split[4 * tid + 2] = w.split[4 * tid + 3] = 0;
+            }
+        } else if (j == 0 && tid >= BLOCK - 2) {
+            uint32_t r[RW];
+            const int q = tid - (BLOCK - 2);
+            RecIO<RW>::load(out, q ? n - 1 : 0, r);
+            w.pminmax[4 * q] = lkey<RW>(r, lk);
+            for (int k = 1; k < 4; k++) w.pminmax[4 * q + k] = 0;
+        }
+        __syncthreads();
+        // this wave's splitters: bounds of the runs first, then the records
+        uint32_t r0[Q], r1[Q], lt[Q], le[Q];
+        int64_t base[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int i = q * NW + wave;
+            r0[q] = r1[q] = lt[q] = le[q] = 0;
+            base[q] = 0;
+            if (i < P - 1 && ta < tb) {
+                const int b = s_b[i];
+                r0[q] = oa[b];
+                r1[q] = ob[b];
+                base[q] = w.base[b];
+                lt[q] = le[q] = s_pref[b];
+                if (eq_done && single_bucket(s_tab, b)) {
+                    le[q] += r1[q] - r0[q];
+                    r1[q] = r0[q];
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int i = q * NW + wave;
+            const uint64_t v = s_v[min(i, kDirectMaxP - 1)];
+            for (uint32_t x = r0[q]; x < r1[q]; x += 64) {
+                uint32_t r[RW];
+                const bool in = x + lane < r1[q];
+                RecIO<RW>::load(part, base[q] + (in ? x + lane : r0[q]), r);
+                const uint64_t k = lkey<RW>(r, lk);
+                lt[q] += (uint32_t)__popcll(__ballot(in && k < v));
+                le[q] += (uint32_t)__popcll(__ballot(in && k <= v));
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int i = q * NW + wave;
+            if (i < P - 1 && lane == 0) {
+                w.myclt[(int64_t)j * P1 + i + 1] = lt[q];
+                w.mycle[(int64_t)j * P1 + i + 1] = le[q];
+                store_agent(w.cross + i * kDirectMaxP + j, ((uint64_t)le[q] << 32) | lt[q]);
+            }
+        }
+        // the block's agent-scope stores to cross are complete before it is
+        // counted (a fence by every wave would write back its L2 each time)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0)
+            s_last = __hip_atomic_fetch_add(&w.lists[7], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+                     (uint32_t)(P - 1);
+        __syncthreads();
+        if (!s_last) return;
+        if (tid == 0) w.lists[7] = 0;  // the counts may run again in this call
+        if (tid < kDirectMaxP) s_c[0][tid] = 0;
+        const uint32_t cnt = lane < P ? (uint32_t)w.count[lane] : 0u;
+        uint64_t x[Q];
+        int64_t C1[Q], C0[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int r = min(q * NW + wave, P - 1);
+            x[q] = lane < P && r < P - 1 ? load_agent(w.cross + r * kDirectMaxP + lane) : ((uint64_t)cnt << 32) | cnt;
+            C0[q] = w.C[r];
+            C1[q] = w.C[r + 1];
+        }
+        // counts fit 32 bits: the ranks hold less than 2^31 records together
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int r = q * NW + wave;
+            const uint32_t a = (uint32_t)x[q], e = (uint32_t)(x[q] >> 32);
+            const uint32_t sure = __shfl(incl_scan_u32(a), 63, 64);
+            const long long deficit = C1[q] - (long long)sure;
+            const uint32_t sp = e > a ? e - a : 0u;
+            long long rem = deficit - (long long)(incl_scan_u32(sp) - sp);
+            rem = rem > 0 ? rem : 0;
+            if (r < P) {
+                if (deficit < 0 || (rem > 0 && e < a)) atomicOr(&s_err, 4u);
+                if (lane < P) {
+                    const uint32_t c = a + (uint32_t)((long long)sp < rem ? (long long)sp : rem);
+                    s_c[r + 1][lane] = c;
+                    w.myC[(int64_t)lane * P1 + r + 1] = c;
+                }
+            }
+        }
+        if (tid < P) {
+            w.myC[(int64_t)tid * P1] = 0;
+            w.myclt[(int64_t)tid * P1] = w.mycle[(int64_t)tid * P1] = 0;
+            w.myclt[(int64_t)tid * P1 + P] = w.mycle[(int64_t)tid * P1 + P] = w.count[tid];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int r = q * NW + wave;
+            if (r < P) {
+                const uint32_t a = lane < P ? s_c[r][lane] : 0u, e = lane < P ? s_c[r + 1][lane] : 0u;
+                if (e < a) atomicOr(&s_err, 8u);
+                if (lane < P) w.send[(int64_t)lane * P + r] = (int64_t)e - (int64_t)a;
+                const uint32_t sum = incl_scan_u32(e - a);
+                if (lane == 63 && (int64_t)sum != C1[q] - C0[q]) atomicOr(&s_err, 16u);
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < 4) res->lists[tid] = w.lists[tid];
+    if (tid < 2) res->sums[tid] = w.checksum[tid];
+    if (tid == 2) res->err = w.err[0] | s_err;
+    if (tid == 3) res->scatter_err = w.err[1];
+}
+
+// ---------------------------------------------------------------------------
+// host launchers
+int launch_direct_sample(int rw, const void* src, const LKey& lk, const DirectShape& sh, const DirectWork& w,
+                         bool clear_sums, hipEvent_t start, hipStream_t st) {
+    const uint32_t* s = (const uint32_t*)src;
+    const unsigned g = (unsigned)(sh.S / kDirectChunk);
+    switch (rw) {
+        case 2: hipExtLaunchKernelGGL(direct_sample_kernel<2>, dim3(g), dim3(kDirectChunk), 0, st, start, nullptr, 0, s, lk, sh, w, clear_sums ? 1 : 0); break;
+        case 4: hipExtLaunchKernelGGL(direct_sample_kernel<4>, dim3(g), dim3(kDirectChunk), 0, st, start, nullptr, 0, s, lk, sh, w, clear_sums ? 1 : 0); break;
+        default: return -1;
+    }
+    MPSG_CHECK(hipGetLastError());
+    if (g > 1) {
+        hipLaunchKernelGGL(direct_rank_kernel, dim3((unsigned)(sh.S / kRankBlock)), dim3(kRankBlock), 0, st, sh.S, sh.W,
+                           w.chunks, w.raw);
+        MPSG_CHECK(hipGetLastError());
+    }
+    return 0;
+}
+
+int launch_direct_count(int rw, const void* src, const LKey& lk, const DirectShape& sh, const DirectWork& w,
+                        long long* checksum, hipStream_t st) {
+    const SegDev sd{w.begin, w.count, w.tile_start, sh.P, 0};
+    const uint32_t* s = (const uint32_t*)src;
+    int step0 = 1;
+    while (2 * step0 < sh.W) step0 *= 2;
+    const int64_t slots = rw == 2 ? resident_blocks(direct_hist_kernel<2>, 512) : resident_blocks(direct_hist_kernel<4>, 512);
+    const int64_t tpb = (sh.ntiles + slots - 1) / slots;
+    const unsigned g = (unsigned)((sh.ntiles + tpb - 1) / tpb);
+    switch (rw) {
+        case 2:
+            hipLaunchKernelGGL(direct_hist_kernel<2>, dim3(g), dim3(512), 0, st, s, sd, sh.ntiles, tpb, sh.tile, lk, sh.W,
+                               step0, w.raw, w.tables, w.tile_cnt, w.bkt, checksum);
+            break;
+        case 4:
+            hipLaunchKernelGGL(direct_hist_kernel<4>, dim3(g), dim3(512), 0, st, s, sd, sh.ntiles, tpb, sh.tile, lk, sh.W,
+                               step0, w.raw, w.tables, w.tile_cnt, w.bkt, checksum);
+            break;
+        default: return -1;
+    }
+    MPSG_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(direct_scan_kernel, dim3(kLBins / 64), dim3(1024), 0, st, w.tile_cnt, sh.ntiles, w.tile_off, w.tot);
+    MPSG_CHECK(hipGetLastError());
+    return 0;
+}
+
+int launch_direct_counts(int rw, const void* out, const void* part, const LKey& lk, const DirectShape& sh,
+                         const DirectWork& w, bool eq_done, DirectResult* res, hipEvent_t stop, hipStream_t st) {
+    const uint32_t *o = (const uint32_t*)out, *p = (const uint32_t*)part;
+    const dim3 g((unsigned)sh.P), b(1024);
+    const int ed = eq_done ? 1 : 0;
+    switch (rw) {
+        case 2: hipExtLaunchKernelGGL(direct_counts_kernel<2>, g, b, 0, st, nullptr, stop, 0, o, p, lk, sh.P, sh.n, sh.ntiles, w, ed, res); break;
+        case 4: hipExtLaunchKernelGGL(direct_counts_kernel<4>, g, b, 0, st, nullptr, stop, 0, o, p, lk, sh.P, sh.n, sh.ntiles, w, ed, res); break;
+        default: return -1;
+    }
+    MPSG_CHECK(hipGetLastError());
+    return 0;
+}
+
+}  // namespace mpsg

@@ -82,10 +82,13 @@ int lscatter_tile(int rw);
 int launch_ltile_scan(const uint16_t* tile_cnt, const SegDev& sd, const int64_t* bucket_base, uint32_t* tile_off,
                       hipStream_t st);
 // records of single-value buckets go to eq_dst, the rest to dst; bkt: the
-// buckets written by launch_lhist
+// buckets written by launch_lhist.  tot (optional): the segments share one
+// bucket space over records [0, gend) -- tot[b] records in bucket b,
+// tile_off counted from the bucket's start, the starts written to base_out
 int launch_lscatter(int rw, const void* src, void* dst, void* eq_dst, const SegDev& sd, int64_t ntiles,
                     const uint16_t* bkt, const uint64_t* tables, int64_t tstride, const uint32_t* tile_off,
-                    uint32_t* err, hipStream_t st);
+                    uint32_t* err, hipStream_t st, const uint32_t* tot = nullptr, int64_t gend = 0,
+                    int64_t* base_out = nullptr);
 // Sorts every bucket (src -> dst, same slots).  eq_done: the scatter already
 // wrote the single-value buckets to dst.  Buckets above kChunkCap go to the
 // overflow list (*noverflow entries of {base, count}); hard (one uint32 per
@@ -162,14 +165,15 @@ int launch_listed_sort(int rw, const void* src, void* dst, const LKey& lk, const
                        const uint32_t* hist, const int64_t* bucket_base, const uint64_t* tables, int nbins,
                        int64_t tstride, uint32_t* hard, uint32_t* nhard, long long* checksum, hipStream_t st,
                        const EntryOut* eo = nullptr);
-// launch_chunk_sort with 512-thread workgroups (two per CU): buckets above
-// 4096 records (up to kChunkCap) are listed in medium (*nmedium entries) for
-// launch_listed_sort; no LDS radix pass is launched
+// launch_chunk_sort with 512-thread workgroups: two per CU, or with small
+// three (buckets up to kMergeCap records); larger buckets (up to kChunkCap)
+// are listed in medium (*nmedium entries) for launch_listed_sort; no LDS
+// radix pass is launched
 int launch_chunk_sort_small(int rw, const void* src, void* dst, const LKey& lk, const uint32_t* hist,
                             const int64_t* bucket_base, const uint64_t* tables, int64_t tstride, int64_t nbuckets,
                             int64_t* overflow, uint32_t* noverflow, int max_overflow, uint32_t* hard, uint32_t* nhard,
                             uint32_t* medium, uint32_t* nmedium, long long* checksum, bool eq_done, hipStream_t st,
-                            const EntryOut* eo = nullptr, uint32_t ovf_cap = (uint32_t)kChunkCap);
+                            const EntryOut* eo = nullptr, uint32_t ovf_cap = (uint32_t)kChunkCap, bool small = false, hipEvent_t stop = nullptr);
 // independent segments (the batched sort) in LDS, one workgroup each:
 // segments [0, na) of the lists cnt / base by the form chosen -- 0: 1024
 // threads x 9 records (one workgroup per CU), 1: 512 x 9 (two per CU), 2:

@@ -22,45 +22,15 @@
 // -- non-decreasing in the key.  A bucket with t[b-1] + 1 == t[b] (or b == 0
 // with t[0] == 0) holds the single key value t[b]: duplicate-heavy keys get
 // such a bucket of their own, and its records are final after the scatter.
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 
 #include "device.h"
 #include "lsort.h"
+#include "lsort_dev.h"
 
 namespace mpsg {
-
-// FAST: the common layout (the key in the record's first words, no bit
-// shift) is taken without the word selection when the key has it (the
-// condition is the same for the whole kernel; used where the registers
-// allow the second code path)
-template <int RW, bool FAST = false>
-__device__ __forceinline__ uint64_t lkey(const uint32_t (&r)[RW], const LKey& k) {
-    if (FAST && k.w0 == 0 && k.sh == 0) {
-        uint64_t v = r[0];
-        if constexpr (RW > 1) v |= (uint64_t)r[1] << 32;
-        return (v & k.mask) ^ k.xmask;
-    }
-    const uint32_t a = pick_word<RW>(r, k.w0), b = pick_word<RW>(r, k.w0 + 1),
-                   c = pick_word<RW>(r, k.w0 + 2);
-    const uint64_t lo = (uint64_t)a | ((uint64_t)b << 32);
-    const uint64_t v = k.sh ? ((lo >> k.sh) | ((uint64_t)c << (64 - k.sh))) : lo;
-    return (v & k.mask) ^ k.xmask;
-}
-
-__device__ __forceinline__ uint32_t bucket_of(uint64_t key, const uint64_t* __restrict__ t) {
-    int lo = 0;
-#pragma unroll
-    for (int step = 512; step > 0; step >>= 1)
-        if (lo + step <= kLBounds && t[lo + step - 1] < key) lo += step;
-    return (uint32_t)lo;
-}
-
-// bucket b of table t holds one key value only
-__device__ __forceinline__ bool single_bucket(const uint64_t* __restrict__ t, int b) {
-    if (b == 0) return t[0] == 0;
-    if (b >= kLBounds) return false;
-    return t[b - 1] + 1 == t[b];
-}
 
 // ---------------------------------------------------------------------------
 template <int RW>
@@ -213,24 +183,6 @@ __global__ __launch_bounds__(kBlock) void lhist_kernel(const uint32_t* __restric
     }
 }
 
-// exclusive scan of B values, one per thread of a B-thread block
-template <int B>
-__device__ __forceinline__ uint32_t scan_block(uint32_t v, uint32_t* s_tmp /*B / 64*/) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, 64);
-        if (lane >= off) x += y;
-    }
-    if (lane == 63) s_tmp[wave] = x;
-    __syncthreads();
-    uint32_t pre = 0;
-#pragma unroll
-    for (int w = 0; w < B / 64; w++) pre += (w < wave) ? s_tmp[w] : 0u;
-    __syncthreads();
-    return pre + x - v;
-}
 __device__ __forceinline__ uint32_t scan1024(uint32_t v, uint32_t* s_tmp /*16*/) { return scan_block<1024>(v, s_tmp); }
 
 // per segment: absolute base of every bucket (nb buckets per segment, a
@@ -289,12 +241,15 @@ __global__ __launch_bounds__(256) void ltile_scan_kernel(const uint16_t* __restr
 
 // ---------------------------------------------------------------------------
 // the bucket scatter: a onesweep pass with 1024 bins.  BLOCK = 512: a tile
-// fits 80 KiB of LDS, so two workgroups share a CU.
-template <int RW, int ITEMS, int BLOCK>
+// fits 80 KiB of LDS, so two workgroups share a CU.  ONE: one bucket space for
+// all segments (offsets from the bucket's start over records [0, gend), the
+// bucket starts summed here from tot and kept in base_out).
+template <int RW, int ITEMS, int BLOCK, bool ONE = false>
 __global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void lscatter_kernel(
     const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, SegDev seg, int64_t ntiles,
     const uint16_t* __restrict__ bkt, const uint64_t* __restrict__ tables, int64_t tstride,
-    const uint32_t* __restrict__ tile_off, uint32_t* __restrict__ error_flag, uint32_t* __restrict__ eq_dst) {
+    const uint32_t* __restrict__ tile_off, uint32_t* __restrict__ error_flag, uint32_t* __restrict__ eq_dst,
+    const uint32_t* __restrict__ tot, int64_t gend, int64_t* __restrict__ base_out) {
     constexpr int NW = BLOCK / 64, BPT = kLBins / BLOCK;  // waves, buckets per thread
     constexpr int TILE = BLOCK * ITEMS;
     constexpr int WAVE_TILE = 64 * ITEMS;
@@ -316,13 +271,14 @@ __global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void lscatter_kernel(
     const int64_t per = gridDim.x / 8;
     const int64_t tile = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
     if (tile >= ntiles) return;
-    const int s = upper_index<int64_t>(seg.tile_start, seg.nseg, tile);
+    const int s = ONE ? seg_of_tile(seg, tile) : upper_index<int64_t>(seg.tile_start, seg.nseg, tile);
     const int64_t t = tile - seg.tile_start[s];
     const int64_t sbeg = seg.begin[s];
     const int64_t send = sbeg + seg.count[s];
     const int64_t begin = sbeg + t * TILE;
     const int64_t end = min(send, begin + (int64_t)TILE);
     const int count = (int)(end - begin);
+    const int64_t dbeg = ONE ? 0 : sbeg, dend = ONE ? gend : send;
 
     // records and their buckets (computed by the histogram pass)
     uint32_t r[ITEMS][RW];
@@ -376,6 +332,21 @@ __global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void lscatter_kernel(
     uint32_t toff[BPT];
 #pragma unroll
     for (int q = 0; q < BPT; q++) toff[q] = tile_off[tile * kLBins + BPT * tid + q];
+    if constexpr (ONE) {
+        uint32_t bt[BPT], bs = 0;
+#pragma unroll
+        for (int q = 0; q < BPT; q++) {
+            bt[q] = tot[BPT * tid + q];
+            bs += bt[q];
+        }
+        uint32_t bx = scan_block<BLOCK>(bs, s_tmp);
+#pragma unroll
+        for (int q = 0; q < BPT; q++) {
+            toff[q] += bx;
+            if (tile == 0) base_out[BPT * tid + q] = (int64_t)bx;
+            bx += bt[q];
+        }
+    }
 #pragma unroll
     for (int q = 0; q < BPT; q++) {
         const int d = BPT * tid + q;
@@ -419,8 +390,8 @@ __global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void lscatter_kernel(
 #pragma unroll
             for (int w = 0; w < RW; w++) rr[w] = s_rec[i * RW + w];
             const uint32_t dd = s_dig[i];
-            const int64_t o = sbeg + (int64_t)s_gdelta[dd] + i;
-            if (o < sbeg || o >= send) {
+            const int64_t o = dbeg + (int64_t)s_gdelta[dd] + i;
+            if (o < dbeg || o >= dend) {
                 atomicOr(error_flag, 4u);
                 continue;
             }
@@ -2046,17 +2017,23 @@ int launch_ltile_scan(const uint16_t* tile_cnt, const SegDev& sd, const int64_t*
 
 int launch_lscatter(int rw, const void* src, void* dst, void* eq_dst, const SegDev& sd, int64_t ntiles,
                     const uint16_t* bkt, const uint64_t* tables, int64_t tstride, const uint32_t* tile_off,
-                    uint32_t* err, hipStream_t st) {
+                    uint32_t* err, hipStream_t st, const uint32_t* tot, int64_t gend, int64_t* base_out) {
     if (ntiles <= 0) return 0;
     const unsigned grid = (unsigned)(8 * ((ntiles + 7) / 8));
     const uint32_t* s = (const uint32_t*)src;
     uint32_t* d = (uint32_t*)dst;
     uint32_t* e = (uint32_t*)eq_dst;
-    switch (rw) {
-        case 2: hipLaunchKernelGGL((lscatter_kernel<2, 8, 1024>), dim3(grid), dim3(1024), 0, st, s, d, sd, ntiles, bkt, tables, tstride, tile_off, err, e); break;
-        case 4: hipLaunchKernelGGL((lscatter_kernel<4, 6, 512>), dim3(grid), dim3(512), 0, st, s, d, sd, ntiles, bkt, tables, tstride, tile_off, err, e); break;
+#define MPSG_SCATTER(R, I, B, ONE) \
+    hipLaunchKernelGGL((lscatter_kernel<R, I, B, ONE>), dim3(grid), dim3(B), 0, st, s, d, sd, ntiles, bkt, tables, \
+                       tstride, tile_off, err, e, tot, gend, base_out)
+    switch (rw * 2 + (tot ? 1 : 0)) {
+        case 4: MPSG_SCATTER(2, 8, 1024, false); break;
+        case 5: MPSG_SCATTER(2, 8, 1024, true); break;
+        case 8: MPSG_SCATTER(4, 6, 512, false); break;
+        case 9: MPSG_SCATTER(4, 6, 512, true); break;
         default: return -1;
     }
+#undef MPSG_SCATTER
     MPSG_CHECK(hipGetLastError());
     return 0;
 }
@@ -2140,26 +2117,25 @@ int launch_chunk_sort_small(int rw, const void* src, void* dst, const LKey& lk, 
                             const int64_t* bucket_base, const uint64_t* tables, int64_t tstride, int64_t nbuckets,
                             int64_t* overflow, uint32_t* noverflow, int max_overflow, uint32_t* hard, uint32_t* nhard,
                             uint32_t* medium, uint32_t* nmedium, long long* checksum, bool eq_done, hipStream_t st,
-                            const EntryOut* eop, uint32_t ovf_cap) {
+                            const EntryOut* eop, uint32_t ovf_cap, bool small, hipEvent_t stop) {
     if (nbuckets <= 0) return 0;
     const EntryOut eo = eop ? *eop : EntryOut{};
     const uint32_t* s = (const uint32_t*)src;
     uint32_t* d = (uint32_t*)dst;
     const int ed = eq_done ? 1 : 0;
     const unsigned grid = (unsigned)nbuckets;
-    switch (rw) {
-        case 2:
-            hipLaunchKernelGGL((interp_sort_kernel<2, kMergeBlock, kSmallItems>), dim3(grid), dim3(kMergeBlock), 0, st, s, d, lk, hist,
-                               bucket_base, tables, tstride, nbuckets, overflow, noverflow, max_overflow, hard, nhard,
-                               medium, nmedium, checksum, ed, eo, ovf_cap);
-            break;
-        case 4:
-            hipLaunchKernelGGL((interp_sort_kernel<4, kMergeBlock, kSmallItems>), dim3(grid), dim3(kMergeBlock), 0, st, s, d, lk, hist,
-                               bucket_base, tables, tstride, nbuckets, overflow, noverflow, max_overflow, hard, nhard,
-                               medium, nmedium, checksum, ed, eo, ovf_cap);
-            break;
+#define MPSG_CHUNKFORM(R, I) \
+    hipExtLaunchKernelGGL((interp_sort_kernel<R, kMergeBlock, I>), dim3(grid), dim3(kMergeBlock), 0, st, nullptr, stop, 0, s, d, lk, hist, \
+                       bucket_base, tables, tstride, nbuckets, overflow, noverflow, max_overflow, hard, nhard, medium, \
+                       nmedium, checksum, ed, eo, ovf_cap)
+    switch (rw * 2 + (small ? 1 : 0)) {
+        case 4: MPSG_CHUNKFORM(2, kSmallItems); break;
+        case 5: MPSG_CHUNKFORM(2, kMergeItems); break;
+        case 8: MPSG_CHUNKFORM(4, kSmallItems); break;
+        case 9: MPSG_CHUNKFORM(4, kMergeItems); break;
         default: return -1;
     }
+#undef MPSG_CHUNKFORM
     MPSG_CHECK(hipGetLastError());
     return 0;
 }

@@ -1,0 +1,99 @@
+"""The sort of up to 64 ranks without per-rank local sorts: one partition over
+all ranks, in-LDS bucket sorts, the counts read off the result.  Held to the
+oracle's bytes and counts at the edges of its sizes (one tile, one bucket more,
+the largest single partition), of ranks and tiles, and on keys that strain the
+sampled boundaries."""
+import sys
+
+import numpy
+import pytest
+
+from gpu_util import even
+from mpsort import _lib, workloads
+from mpsort._lib import lib
+from test_gpu_histsort import check_parity
+from test_gpu_plain_merged import keys
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def no_options():
+    lib.mpsort_mpi_unset_options(-1)
+
+
+def note(*a):
+    print(*a, flush=True)
+    sys.stdout.flush()
+
+
+def ragged(n, P, seed):
+    cut = numpy.sort(numpy.random.default_rng(seed).integers(0, n + 1, P - 1))
+    return numpy.diff(numpy.concatenate([[0], cut, [n]]))
+
+
+@pytest.mark.parametrize("n", [8193, 3072 * 3, 2 * 8192, 2048 * 16 + 1, 2048 * 512 + 1, 2048 * 1024 + 1, 4300800, 4300801])
+def test_sizes(n):
+    P = 5
+    a = workloads.records16(keys("random", n, n % 97))
+    note("direct n=%d" % n)
+    check_parity(a, ragged(n, P, 1), ragged(n, P, 2), 'key', device=True)
+
+
+@pytest.mark.parametrize("shape", ["heavy", "few", "zero_heavy", "sorted", "reversed", "narrow", "two_scales"])
+@pytest.mark.parametrize("P", [1, 63, 64])
+def test_shapes(shape, P):
+    n = 300007
+    a = workloads.records16(keys(shape, n, 5 + P))
+    note("direct shape=%s P=%d" % (shape, P))
+    check_parity(a, ragged(n, P, 3), ragged(n, P, 4), 'key', device=True)
+
+
+@pytest.mark.parametrize("P", [2, 64])
+@pytest.mark.parametrize("value", [0, 1, 2 ** 64 - 1])
+def test_one_key_value(value, P):
+    """every record one key, the smallest and the largest value among them;
+    and one other key in front of, or behind, the heavy one"""
+    n = 50021
+    k = numpy.full(n, value, numpy.uint64)
+    check_parity(workloads.records16(k), ragged(n, P, 5), ragged(n, P, 6), 'key', device=True)
+    k[n // 2] = numpy.uint64(value - 1 if value > 1 else value + 1)
+    check_parity(workloads.records16(k), ragged(n, P, 5), ragged(n, P, 6), 'key', device=True)
+
+
+@pytest.mark.parametrize("dt", ["u8", "i8", "i4pair", "u4pair", "keytail"])
+def test_record_types(dt):
+    n, P = 61001, 9
+    g = numpy.random.default_rng(8)
+    if dt in ("u8", "i8"):
+        i = numpy.iinfo(dt)
+        a, f = g.integers(i.min, i.max, n, dtype=dt, endpoint=True), None
+    elif dt == "keytail":
+        a, f = numpy.zeros(n, [('v', 'i8'), ('key', 'i8')]), 'key'
+        a['key'], a['v'] = g.integers(-300, 300, n), numpy.arange(n)
+    else:
+        a, f = numpy.zeros(n, [('key', dt[:2]), ('v', 'f4')]), 'key'
+        i = numpy.iinfo(dt[:2])
+        a['key'], a['v'] = g.integers(i.min, i.max, n, dtype=dt[:2], endpoint=True), numpy.arange(n)
+    check_parity(a, ragged(n, P, 7), ragged(n, P, 8), f, device=True)
+
+
+def test_overlapping_output():
+    """input and output overlap without being equal: the input is read whole
+    before the output is written"""
+    import ctypes
+    from gpu_util import key_desc
+    n, P, shift = 70001, 3, 1024
+    a = workloads.records16(keys("heavy", n, 3))
+    want = a[numpy.argsort(a['key'], kind='stable')]
+    d = lib.mpsort_gpu_dmalloc((n + shift) * 16)
+    try:
+        _lib.check(lib.mpsort_gpu_memcpy_h2d(d, a.ctypes.data, a.nbytes))
+        c = (ctypes.c_int64 * P)(*even(n, P))
+        k = key_desc(a.dtype, 'key')
+        _lib.check(lib.mpsort_gpu_newarray(d, c, P, d + shift * 16, c, 16, ctypes.byref(k), _lib.DEVICE_PTRS))
+        out = numpy.empty_like(a)
+        _lib.check(lib.mpsort_gpu_memcpy_d2h(out.ctypes.data, d + shift * 16, a.nbytes))
+    finally:
+        lib.mpsort_gpu_dfree(d)
+    assert numpy.array_equal(out, want)
