@@ -173,6 +173,7 @@ struct DevCtx {
     int64_t fsplan_key = 0;  // segments and tile shape those arrays were made for (0: none)
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
+    Buf sacc;           // small sorts: splitters, and counters that are zero between calls
     Buf hmirror;        // device copy of staged host tables (Upload)
     Buf gstage;         // small device results gathered for one download (Readback)
     void* rpin = nullptr;  // pinned: per-call staging and small reads (pin_take), reset per call
@@ -222,6 +223,7 @@ static int get_ctx(DevCtx** out) {
             for (int i = 0; i < 2 * kMaxPasses; i++)
                 MPSG_CHECK(hipEventCreateWithFlags(&c.pass_ev[a][i], hipEventDisableSystemFence));
         c.lookback.zero_on_grow = true;
+        c.sacc.zero_on_grow = true;
         // the device address of this GPU's scratch array (the device is
         // current); only the allocation-free entry point uses it
         c.scratch_err = hipGetSymbolAddress(&c.scratch, HIP_SYMBOL(scratch));
@@ -1634,11 +1636,106 @@ static int plain_bucket_first(DevCtx& c, const CallShape& cs, const SegSortPlan&
 // at most kLBins buckets, each at most about the in-LDS capacity of 4608
 // records: kDirectMaxRecords.
 constexpr int64_t kDirectMaxRecords = (int64_t)kLBins * 4200;
-constexpr int64_t kDirectMinRecords = 8193;
 constexpr int64_t kDirectAvg = 2048;   // records per bucket while kLBins buckets suffice
+static bool direct_asked(const CallShape& cs) {
+    return !g_faults && !cs.exchange && cs.first_mode == 0 && cs.P <= kDirectMaxP && cs.ks.key_bytes <= 8;
+}
 static bool direct_eligible(const CallShape& cs) {
-    return !g_faults && !cs.exchange && cs.first_mode == 0 && cs.P <= kDirectMaxP && (cs.rw == 2 || cs.rw == 4) &&
-           cs.ks.key_bytes <= 8 && cs.ntot >= kDirectMinRecords && cs.ntot <= kDirectMaxRecords;
+    return direct_asked(cs) && (cs.rw == 2 || cs.rw == 4) && cs.ntot > kSmallRecords && cs.ntot <= kDirectMaxRecords;
+}
+// One workgroup sorts everything, any record size (a packed call's records
+// directly, without packing).
+static bool small_eligible(const CallShape& cs) {
+    return direct_asked(cs) && cs.ntot >= 1 && cs.ntot <= kSmallRecords && cs.elsize <= (1 << 16);
+}
+
+// the rank tables and the counts' device arrays of the two forms
+static void direct_shape(const CallShape& cs, const int64_t* nin, const int64_t* nout, int tile, DirectShape* sh) {
+    memset(sh, 0, sizeof *sh);
+    sh->P = cs.P;
+    sh->n = cs.ntot;
+    sh->tile = tile;
+    for (int t = 0; t < cs.P; t++) {
+        sh->begin[t + 1] = sh->begin[t] + nin[t];
+        sh->C[t + 1] = sh->C[t] + nout[t];
+        sh->tile_start[t + 1] = sh->tile_start[t] + (nin[t] + tile - 1) / tile;
+    }
+    sh->ntiles = sh->tile_start[cs.P];
+}
+static int direct_counts_arrays(DevCtx& c, int P, DirectWork* w, DirectResult** res) {
+    int rc = 0;
+    Sizer sz;
+    lay_hist(sz, P, nullptr);
+    if ((rc = c.small.ensure(sz.off + 4096))) return rc;
+    Arena ar{(char*)c.small.p};
+    HistArrays h;
+    lay_hist(ar, P, &h);
+    w->C = h.C;
+    w->err = h.err;
+    w->checksum = h.checksum;
+    w->myclt = h.myclt;
+    w->mycle = h.mycle;
+    w->myC = h.myC;
+    w->send = h.send;
+    w->split = h.split;
+    w->pminmax = h.pminmax;
+    if ((rc = ensure_rpin(c, sizeof(DirectResult) + 256))) return rc;
+    *res = (DirectResult*)pin_take(c, sizeof(DirectResult));
+    return *res ? 0 : fail(MPSORT_ERR_HIP, "no pinned memory for the results");
+}
+// the statistics and recorded counts both forms leave, and their checks
+static int direct_results(DevCtx& c, const CallShape& cs, const DirectWork& w, const DirectResult& got, bool host_sum,
+                          mpsort_gpu_stats* stats) {
+    stats->nvranks = cs.P;
+    stats->second_merged = cs.P > 1 ? 1 : 0;
+    stats->record_bytes = (int32_t)(cs.rw * 4);
+    stats->general_path = cs.general ? 1 : 0;
+    stats->nrecords = cs.ntot;
+    stats->checksum_in = got.sums[0];
+    stats->checksum_out = got.sums[1];
+    c.last_P = cs.P;
+    c.C = w.C;
+    c.myclt = w.myclt;
+    c.mycle = w.mycle;
+    c.myC = w.myC;
+    c.send = w.send;
+    c.split = w.split;
+    c.pminmax = w.pminmax;
+    c.last_ntot = cs.ntot;
+    if (got.err)
+        return fail(MPSORT_ERR_LAYOUT, "layout check failed (device flags 0x%x): the splitter counts or layout solve "
+                                       "is inconsistent", got.err);
+    if (cs.checksum && !host_sum && got.sums[0] != got.sums[1])
+        return fail(MPSORT_ERR_CHECKSUM, "MPSort: Data changed after sorting; checksum mismatch (%lld != %lld)",
+                    (long long)got.sums[0], (long long)got.sums[1]);
+    return 0;
+}
+
+static int run_small(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
+                     const int64_t* nout, mpsort_gpu_stats* stats) {
+    int rc = 0;
+    DirectShape sh;
+    direct_shape(cs, nin, nout, kSmallRecords, &sh);
+    DirectWork w;
+    memset(&w, 0, sizeof w);
+    DirectResult* res = nullptr;
+    if ((rc = direct_counts_arrays(c, cs.P, &w, &res))) return rc;
+    constexpr size_t kCross = sizeof(uint64_t) * kDirectMaxP;
+    if ((rc = c.sacc.ensure(kCross + 4 * sizeof(uint64_t)))) return rc;
+    w.cross = (uint64_t*)c.sacc.p;
+    w.acc = (unsigned long long*)((char*)c.sacc.p + kCross);
+    const LKey lk = make_lkey(cs.ks);
+    const char *a = (const char*)d_in, *b = (const char*)d_out;
+    const size_t bytes = (size_t)cs.ntot * (size_t)cs.elsize;
+    const bool apart = a >= b + bytes || b >= a + bytes;
+    if ((rc = launch_small_sort(cs.general ? 0 : cs.rw, d_in, d_out, lk, (int)cs.elsize, (int)cs.key_off_user,
+                                cs.key_bytes_user, sh, w, cs.checksum, apart, res, c.ev[kEvStart], c.ev[kEvEnd], c.st)))
+        return rc;
+    MPSG_CHECK(hipStreamSynchronize(c.st));
+    const DirectResult got = *res;
+    stats->first_passes = (int32_t)got.lists[3];
+    stats->t_first_sort_ms = stats->t_total_ms = ev_ms(c.ev[kEvStart], c.ev[kEvEnd]);
+    return direct_results(c, cs, w, got, false, stats);
 }
 
 static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
@@ -1650,28 +1747,15 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     int rc = 0;
 
     DirectShape sh;
-    memset(&sh, 0, sizeof sh);
-    sh.P = P;
-    sh.n = n;
-    sh.tile = lscatter_tile(rw);
-    for (int t = 0; t < P; t++) {
-        sh.begin[t + 1] = sh.begin[t] + nin[t];
-        sh.C[t + 1] = sh.C[t] + nout[t];
-        sh.tile_start[t + 1] = sh.tile_start[t] + (nin[t] + sh.tile - 1) / sh.tile;
-    }
-    sh.ntiles = sh.tile_start[P];
+    direct_shape(cs, nin, nout, lscatter_tile(rw), &sh);
     sh.W = (int)std::min<int64_t>(kLBins, std::max<int64_t>(2, (n + kDirectAvg - 1) / kDirectAvg));
     sh.S = std::min(kDirectMaxChunks, (16 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
     const bool small_form = false;
 
     // ---- workspace
-    Sizer sz;
-    lay_hist(sz, P, nullptr);
-    if ((rc = c.small.ensure(sz.off + 4096))) return rc;
-    Arena ar{(char*)c.small.p};
-    HistArrays h;
-    lay_hist(ar, P, &h);
     DirectWork w;
+    DirectResult* res = nullptr;
+    if ((rc = direct_counts_arrays(c, P, &w, &res))) return rc;
     auto lay = [&](auto& a, auto take) {
         take(a, w.begin, (size_t)P);
         take(a, w.count, (size_t)P);
@@ -1695,21 +1779,8 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     if ((rc = c.ltile.ensure(lz.off + 4096))) return rc;
     Arena la{(char*)c.ltile.p};
     lay(la, [](Arena& a, auto*& p, size_t k) { p = a.take<std::remove_reference_t<decltype(*p)>>(k); });
-    w.C = h.C;
-    w.err = h.err;
-    w.checksum = h.checksum;
-    w.myclt = h.myclt;
-    w.mycle = h.mycle;
-    w.myC = h.myC;
-    w.send = h.send;
-    w.split = h.split;
-    w.pminmax = h.pminmax;
     if ((rc = c.s1.ensure((size_t)n * recbytes))) return rc;
     if (cs.general && ((rc = c.rbuf.ensure((size_t)n * recbytes)) || (rc = c.s0.ensure((size_t)n * recbytes)))) return rc;
-    if ((rc = ensure_rpin(c, sizeof(DirectResult) + 256))) return rc;
-    DirectResult* res = (DirectResult*)pin_take(c, sizeof(DirectResult));
-    if (!res) return fail(MPSORT_ERR_HIP, "no pinned memory for the results");
-
     // ---- the sort
     // (the timing events ride on the launches they bracket: an event recorded
     // between two launches costs the GPU about 4.5 us)
@@ -1796,17 +1867,10 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         got = *res;
     }
 
-    stats->nvranks = P;
-    stats->second_merged = P > 1 ? 1 : 0;
     stats->buckets = sh.W;
     stats->buckets_overflow = stats->buckets_overflow_first = (int32_t)got.lists[0];
     stats->buckets_lds_radix = (int32_t)got.lists[1];
     stats->buckets_listed = (int32_t)got.lists[2];
-    stats->record_bytes = (int32_t)recbytes;
-    stats->general_path = cs.general ? 1 : 0;
-    stats->nrecords = n;
-    stats->checksum_in = got.sums[0];
-    stats->checksum_out = got.sums[1];
     stats->t_first_sort_ms = ev_ms(c.ev[kEvStart], c.ev[kEvFirst]);
     stats->t_findp_ms = ev_ms(c.ev[kEvFirst], c.ev[kEvEnd]);  // with the layout
     stats->t_total_ms = ev_ms(c.ev[kEvStart], c.ev[kEvEnd]);
@@ -1814,22 +1878,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         for (int i = 0; i < 4; i++) stats->pass_ms[i] = ev_ms(pe[i], pe[i + 1]);
         stats->npass_ms = 4;
     }
-    c.last_P = P;
-    c.C = h.C;
-    c.myclt = h.myclt;
-    c.mycle = h.mycle;
-    c.myC = h.myC;
-    c.send = h.send;
-    c.split = h.split;
-    c.pminmax = h.pminmax;
-    c.last_ntot = n;
-    if (got.err)
-        return fail(MPSORT_ERR_LAYOUT, "layout check failed (device flags 0x%x): the splitter counts or layout solve "
-                                       "is inconsistent", got.err);
-    if (cs.checksum && !packed_host && got.sums[0] != got.sums[1])
-        return fail(MPSORT_ERR_CHECKSUM, "MPSort: Data changed after sorting; checksum mismatch (%lld != %lld)",
-                    got.sums[0], got.sums[1]);
-    return 0;
+    return direct_results(c, cs, w, got, packed_host != nullptr, stats);
 }
 
 static int run_histsort_learned(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out,
@@ -2618,6 +2667,7 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
     memset(&st, 0, sizeof st);
     remember_key(*c, key, 0, 0);
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
+        if (small_eligible(cs)) return run_small(*c, cs, d_in, d_out, nin, nout, &st);
         if (direct_eligible(cs)) return run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st);
         HistWork w;
         int r2 = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
@@ -2977,6 +3027,7 @@ int mpsort_gpu_release(void) {
     c.fsamp.release();
     c.fsplan.release();
     c.fsplan_key = 0;
+    c.sacc.release();
     c.hmirror.release();
     c.gstage.release();
     c.last_P = 0;

@@ -11,6 +11,8 @@
 namespace mpsg {
 
 constexpr int kDirectMaxP = 64;         // ranks: one lane each
+constexpr int kSmallRecords = 8192;     // sorted by one launch
+constexpr int kRankRecords = 4096;      // of those, by counting every record's rank
 constexpr int kDirectChunk = 1024;      // sample keys sorted by one workgroup
 constexpr int kDirectMaxChunks = 16;    // sample chunks
 constexpr int kDirectMaxBuckets = kLBins;
@@ -47,12 +49,13 @@ struct DirectWork {
     int64_t *myclt, *mycle, *myC, *send;
     uint64_t* cross;      // kDirectMaxP^2: CLE << 32 | CLT by splitter and rank, for the layout
     uint64_t *split, *pminmax;
+    unsigned long long* acc;  // 4, zero between calls: a small sort's blocks done and sums
 };
 
 // what the host reads at the end, written to pinned memory by the last kernel
 struct DirectResult {
     uint32_t err, scatter_err;
-    uint32_t lists[4];
+    uint32_t lists[4];    // [3]: digit passes of the one-workgroup sort
     long long sums[2];
 };
 
@@ -70,5 +73,13 @@ int launch_direct_count(int rw, const void* src, const LKey& lk, const DirectSha
 // instead), and the call's results into res (pinned host memory)
 int launch_direct_counts(int rw, const void* out, const void* part, const LKey& lk, const DirectShape& sh,
                          const DirectWork& w, bool eq_done, DirectResult* res, hipEvent_t stop, hipStream_t st);
+
+// at most kSmallRecords records sorted by one launch, with the splitters,
+// counts and layout (w: C, myclt, mycle, myC, send, split, pminmax, cross,
+// acc).  rw = 0: records of elsize bytes with key_bytes key bytes at key_off.
+// apart: in and out do not overlap (otherwise they are the same)
+int launch_small_sort(int rw, const void* src, void* dst, const LKey& lk, int elsize, int key_off, int key_bytes,
+                      const DirectShape& sh, const DirectWork& w, bool checksum, bool apart, DirectResult* res,
+                      hipEvent_t start, hipEvent_t stop, hipStream_t st);
 
 }  // namespace mpsg

@@ -97,3 +97,47 @@ def test_overlapping_output():
     finally:
         lib.mpsort_gpu_dfree(d)
     assert numpy.array_equal(out, want)
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 8192])
+@pytest.mark.parametrize("P", [1, 2, 64])
+def test_one_workgroup_sizes(n, P):
+    a = workloads.records16(keys("random", n, n))
+    out, st = check_parity(a, ragged(n, P, 9), ragged(n, P, 10), 'key', device=True)
+    assert st.first_passes <= 8
+
+
+@pytest.mark.parametrize("shape", ["heavy", "few", "zero_heavy", "sorted", "narrow", "two_scales"])
+def test_one_workgroup_shapes(shape):
+    P = 17
+    for n in (3001, 5003):
+        check_parity(workloads.records16(keys(shape, n, 12)), ragged(n, P, 11), ragged(n, P, 12), 'key')
+
+
+@pytest.mark.parametrize("dt", ["u4", "i4", "u8", "i8", "particle32", "rec24", "rec13", "keytail"])
+@pytest.mark.parametrize("n, inplace", [(2003, False), (2003, True), (6007, False), (6007, True)])
+def test_one_workgroup_record_types(dt, n, inplace):
+    """4-, 8-, 16- and 32-byte records directly, others (24 bytes; 13 bytes
+    with a key at an odd offset) from their bytes; in place too"""
+    import oracle
+    from gpu_util import gpu_sort_device, last_counts
+    from test_gpu_histsort import _device_inplace
+    P = 6
+    g = numpy.random.default_rng(14)
+    if dt in ("u4", "i4", "u8", "i8"):
+        i = numpy.iinfo(dt)
+        a, f = g.integers(i.min, i.max, n, dtype=dt, endpoint=True), None
+    else:
+        t = {"particle32": workloads.PARTICLE32, "rec24": [('x', 'f8'), ('id', 'i8'), ('w', 'u8')],
+             "rec13": [('b', 'u1'), ('id', 'i4'), ('w', 'u8')], "keytail": [('v', 'i8'), ('id', 'i8')]}[dt]
+        a, f = numpy.zeros(n, t), 'id'
+        a.view(numpy.uint8).reshape(n, -1)[:] = g.integers(0, 256, (n, a.dtype.itemsize))
+        a['id'] = g.integers(0, 900, n)
+    note("one workgroup %s n=%d inplace=%s" % (dt, n, inplace))
+    ref, info = oracle.histogram_sort(a, even(n, P), even(n, P), oracle.key_for(a.dtype, f))
+    out, st = _device_inplace(a, even(n, P), f) if inplace else gpu_sort_device(a, even(n, P), even(n, P), f)
+    assert numpy.array_equal(out.view(numpy.uint8), ref.view(numpy.uint8))
+    c = last_counts(P, 8)
+    for k in ("P", "C", "myCLT", "myCLE", "myC", "send"):
+        assert numpy.array_equal(c[k], info[k]), k
+    assert st.checksum_in == info['checksum_in'] == st.checksum_out
