@@ -461,9 +461,14 @@ def _device_copy(recs):
     return d
 
 
+PLAIN_LEVELS = ("sample", "level1", "level2", "bucket_sort")
+
+
 def plain_first_form(st):
     """(FirstSort form, entries of pass_ms before the SecondSort's) of a
     plain-path call's statistics"""
+    if st["first_passes"] == 0 and len(st["pass_ms"]) == 4 and st["second_passes"] == 0:
+        return "levels", 4  # two partition levels over all ranks, no SecondSort
     nsec = 4 if st["second_merged"] else st["second_passes"]
     if st["first_passes"] == 0 and len(st["pass_ms"]) - nsec == 6:
         return "buckets", 6
@@ -475,6 +480,8 @@ def plain_stages(st):
     form, k0 = plain_first_form(st)
     ms = st["pass_ms"]
     out = {}
+    if form == "levels":
+        return {name: round(ms[i], 4) for i, name in enumerate(PLAIN_LEVELS)}
     if form == "buckets":
         for i, name in enumerate(("sample_tables", "hist", "scatter", "bucket_sort", "lds_radix", "fallback")):
             out["first_" + name] = round(ms[i], 4)
@@ -689,6 +696,10 @@ def bench_histsort(args):
         plain_roof = roof([x for st in st_plain for x in st["pass_ms"][:st["first_passes"] + st["second_passes"]]],
                           "onesweep_kernel<4,1024,8> (one 8-bit digit pass, 2*n*16 B per launch)", TRAFFIC_ONESWEEP,
                           ROCPROF_MS.get("onesweep"))
+    elif first_form == "levels":
+        plain_roof = roof([st["pass_ms"][3] for st in st_plain],
+                          "wide_sort_kernel<4> (fine buckets gathered and sorted in LDS, one launch per step over all n "
+                          "records, with the listed buckets' launches: 2*n*16 B)", None, None)
     else:
         plain_roof = roof([st["pass_ms"][3] for st in st_plain],
                           "interp_sort_kernel<4,512,9> (the plain FirstSort's in-LDS bucket sort, sampled tables, "
@@ -722,10 +733,19 @@ def bench_histsort(args):
                                                     "fallback"))},
             "buckets_overflow": last["buckets_overflow_first"]}
         log("plain bucket FirstSort: %s" % json.dumps(plain_first))
+    elif first_form == "levels":
+        plain_first = {"form": "two partition levels over all ranks, in-LDS sorts of the fine buckets",
+                       "stages_ms": {name: round(sum(st["pass_ms"][i] for st in st_plain) / len(st_plain), 4)
+                                     for i, name in enumerate(PLAIN_LEVELS)},
+                       "buckets": last["buckets"], "buckets_listed": last["buckets_listed"],
+                       "buckets_lds_radix": last["buckets_lds_radix"], "buckets_overflow": last["buckets_overflow"]}
+        log("plain partition levels: %s" % json.dumps(plain_first))
     else:
         plain_first = {"form": "%d digit passes" % last["first_passes"]}
     plain_second = None
-    if last["second_merged"]:
+    if first_form == "levels":
+        plain_second = {"form": "none (the fine buckets' sorts write the output)"}
+    elif last["second_merged"]:
         # the SecondSort without an exchange: its stages after the FirstSort's
         plain_second = {
             "form": "merged (receiver buckets gathered from the senders' sorted segments, sampled tables)",

@@ -18,6 +18,7 @@
 #include "direct.h"
 #include "lsort.h"
 #include "model.h"
+#include "wide.h"
 #include "../../include/mpsort_gpu.h"
 #include "../../include/mp-mpiu.h"
 #include "../../include/mpsort.h"
@@ -1881,6 +1882,174 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     return direct_results(c, cs, w, got, packed_host != nullptr, stats);
 }
 
+// ---- the same in two partition levels (wide.hip), above one level's sizes
+constexpr int64_t kWideCoarse = (int64_t)1 << 17;  // records per coarse bucket while 512 suffice
+constexpr int kWideAvg = 1843;                     // records per fine bucket: 3072 less 2.7 deviations
+                                                   // of a size estimated from 16 sample keys
+static bool wide_eligible(const CallShape& cs) {
+    return direct_asked(cs) && (cs.rw == 2 || cs.rw == 4) && cs.ntot > kDirectMaxRecords &&
+           cs.ntot <= kWideMaxRecords;
+}
+// *again: nothing was written, the call takes the general path (the sample
+// missed the sizes of the coarse buckets by far)
+static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
+                    const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats, bool* again) {
+    hipStream_t st = c.st;
+    const int P = cs.P, rw = cs.rw;
+    const int64_t n = cs.ntot;
+    const size_t bytes = (size_t)n * rw * 4;
+    int rc = 0;
+
+    DirectShape sh;
+    direct_shape(cs, nin, nout, kWideTile, &sh);
+    sh.W = (int)std::min<int64_t>(kWideBuckets, std::max<int64_t>(2, (n + kWideCoarse - 1) / kWideCoarse));
+    sh.S = std::min(kDirectMaxChunks, (32 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
+
+    // ---- workspace
+    DirectWork d;
+    memset(&d, 0, sizeof d);
+    DirectResult* res = nullptr;
+    if ((rc = direct_counts_arrays(c, P, &d, &res))) return rc;
+    WideWork w;
+    memset(&w, 0, sizeof w);
+    w.W = sh.W;
+    w.avg = kWideAvg;
+    w.n = n;
+    w.nt = sh.ntiles;
+    w.ntpad = (w.nt + 64) / 64 * 64;
+    w.nt2 = n / kWideTile + w.W;
+    w.nfine = n / w.avg + w.W;
+    w.ncopy = n / kWideCopy + w.nfine;
+    w.max_overflow = (int)(n / kChunkCap + 1);
+    auto lay = [&](auto& a, auto take) {
+        take(a, d.begin, (size_t)P);
+        take(a, d.count, (size_t)P);
+        take(a, d.tile_start, (size_t)P + 1);
+        take(a, d.chunks, (size_t)sh.S);
+        take(a, d.raw, (size_t)kLBins);
+        take(a, d.lists, (size_t)8);
+        take(a, d.cross, (size_t)kDirectMaxP * kDirectMaxP);
+        take(a, w.tables, (size_t)kWideBuckets);
+        take(a, w.tables2, (size_t)w.W * kWideBuckets);
+        take(a, w.tile_beg, (size_t)w.nt);
+        take(a, w.ex1, (size_t)w.nt * kWideStride);
+        take(a, w.ex2, (size_t)w.nt2 * kWideStride);
+        take(a, w.part, (size_t)(w.ntpad / 64) * kWideBuckets);
+        take(a, w.off, (size_t)w.W * w.ntpad);
+        take(a, w.loc, (size_t)w.W * w.ntpad);
+        take(a, w.tot, (size_t)kWideBuckets);
+        take(a, w.cbase, (size_t)kWideBuckets + 1);
+        take(a, w.ctile, (size_t)kWideBuckets + 1);
+        take(a, w.cfine, (size_t)kWideBuckets + 1);
+        take(a, w.cw, (size_t)kWideBuckets);
+        take(a, w.first, (size_t)w.nt2);
+        take(a, w.desc, (size_t)w.nfine);
+        take(a, w.fcnt, (size_t)w.nfine);
+        take(a, w.fbase, (size_t)w.nfine);
+        take(a, w.medium, (size_t)w.nfine);
+        take(a, w.hard, (size_t)w.nfine);
+        take(a, w.copy, (size_t)w.ncopy);
+        take(a, w.overflow, (size_t)2 * w.max_overflow);
+        take(a, w.tally, (size_t)2 * kDirectMaxP * kDirectMaxP);
+    };
+    Sizer lz;
+    lay(lz, [](Sizer& a, auto*& p, size_t k) { a.take<std::remove_reference_t<decltype(*p)>>(k); });
+    if ((rc = c.ltile.ensure(lz.off + 4096)) || (rc = c.s1.ensure(bytes)) || (rc = c.s2.ensure(bytes))) return rc;
+    if (cs.general && ((rc = c.rbuf.ensure(bytes)) || (rc = c.s0.ensure(bytes)))) return rc;
+    Arena la{(char*)c.ltile.p};
+    lay(la, [](Arena& a, auto*& p, size_t k) { p = a.take<std::remove_reference_t<decltype(*p)>>(k); });
+    w.raw = d.raw;
+    w.lists = d.lists;
+
+    // ---- the sort
+    const LKey lk = make_lkey(cs.ks);
+    const void* src = d_in;
+    void* dst = d_out;
+    if (cs.general) {
+        MPSG_CHECK(hipEventRecord(c.ev[kEvStart], st));
+        src = c.rbuf.p;
+        dst = c.s0.p;
+        if (packed_host) {
+            MPSG_CHECK(hipMemcpyAsync(c.rbuf.p, packed_host, bytes, hipMemcpyHostToDevice, st));
+        } else if ((rc = launch_fill_u32((uint32_t*)d.checksum, 0u, 4, st)) ||
+                   (rc = launch_pack(d_in, n, cs.elsize, cs.key_off_user, cs.key_bytes_user, c.rbuf.p, rw, cs.iwords,
+                                     cs.checksum ? d.checksum : nullptr, st))) {
+            return rc;
+        }
+    }
+    const bool cs_direct = cs.checksum && !cs.general;
+    long long* cs_in = cs_direct ? d.checksum : nullptr;
+    long long* cs_out = cs_direct ? d.checksum + 1 : nullptr;
+    void *a = c.s1.p, *b = c.s2.p;
+    hipEvent_t* pe = cs.timing ? c.pass_ev[0] : nullptr;
+    auto mark = [&](int i) -> int {
+        if (pe) MPSG_CHECK(hipEventRecord(pe[i], st));
+        return 0;
+    };
+    const SegDev sd{d.begin, d.count, d.tile_start, P, 0};
+    if ((rc = mark(0)) ||
+        (rc = launch_direct_sample(rw, src, lk, sh, d, !(cs.general && !packed_host),
+                                   cs.general ? nullptr : c.ev[kEvStart], st)) ||
+        (rc = mark(1)) || (rc = launch_wide_level1(rw, src, a, lk, sd, w, cs_in, st)) || (rc = mark(2)) ||
+        (rc = launch_wide_level2(rw, a, b, dst, lk, w, cs_out, st)) || (rc = mark(3)) ||
+        (rc = launch_wide_sort(rw, b, dst, lk, w, cs_out, st)) || (rc = mark(4)))
+        return rc;
+    MPSG_CHECK(hipEventRecord(c.ev[kEvFirst], st));
+    auto finish = [&]() -> int {
+        int r2 = 0;
+        if (cs.general &&
+            (r2 = launch_gather(d_in, n, cs.elsize, dst, rw, cs.iwords, d_out, cs.checksum ? d.checksum + 1 : nullptr,
+                                d.err, st)))
+            return r2;
+        if ((r2 = launch_wide_counts(rw, dst, a, lk, sh, d, w, res, c.ev[kEvEnd], st))) return r2;
+        MPSG_CHECK(hipStreamSynchronize(st));
+        return 0;
+    };
+    if ((rc = finish())) return rc;
+    DirectResult got = *res;
+    if (got.lists[3]) {
+        *again = true;
+        return 0;
+    }
+    if (got.lists[0]) {
+        // oversized fine buckets of several values: radix sorted, and the
+        // counts again
+        SegSortPlan plain;
+        plain.rw = rw;
+        plain.ks = cs.ks;
+        plain.d_checksum = d.checksum;
+        const TileCfg tc = default_tile(rw);
+        const int64_t nt = n / ((int64_t)tc.block * tc.items) + kMaxFallbackSegs + 1;
+        if ((rc = c.lookback.ensure((size_t)nt * kBins * sizeof(uint64_t)))) return rc;
+        if (got.lists[0] > (uint32_t)w.max_overflow) return fail(MPSORT_ERR_LAYOUT, "oversized buckets exceed the records");
+        for (uint32_t q = 0; q < got.lists[0]; q += kMaxFallbackSegs)
+            if ((rc = sort_listed_segments(c, plain, rw, w.overflow + 2 * q,
+                                           std::min<uint32_t>(kMaxFallbackSegs, got.lists[0] - q), dst, dst, b, nullptr,
+                                           st)))
+                return rc;
+        MPSG_CHECK(hipEventRecord(c.ev[kEvFirst], st));
+        // the first gather may have met records not yet in place
+        if (cs.general && ((rc = launch_fill_u32(d.err, 0u, 1, st)) ||
+                           (rc = launch_fill_u32((uint32_t*)(d.checksum + 1), 0u, 2, st))))
+            return rc;
+        if ((rc = launch_fill_u32(w.tally, 0u, 2 * kDirectMaxP * kDirectMaxP, st)) || (rc = finish())) return rc;
+        got = *res;
+    }
+
+    stats->buckets = (int32_t)got.buckets;
+    stats->buckets_overflow = stats->buckets_overflow_first = (int32_t)got.lists[0];
+    stats->buckets_lds_radix = (int32_t)got.lists[1];
+    stats->buckets_listed = (int32_t)got.lists[2];
+    stats->t_first_sort_ms = ev_ms(c.ev[kEvStart], c.ev[kEvFirst]);
+    stats->t_findp_ms = ev_ms(c.ev[kEvFirst], c.ev[kEvEnd]);  // with the layout
+    stats->t_total_ms = ev_ms(c.ev[kEvStart], c.ev[kEvEnd]);
+    if (pe) {
+        for (int i = 0; i < 4; i++) stats->pass_ms[i] = ev_ms(pe[i], pe[i + 1]);
+        stats->npass_ms = 4;
+    }
+    return direct_results(c, cs, d, got, packed_host != nullptr, stats);
+}
+
 static int run_histsort_learned(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out,
                                 const int64_t* nin, const int64_t* nout, const LearnedModel& M,
                                 mpsort_gpu_stats* stats) {
@@ -2669,8 +2838,14 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
         if (small_eligible(cs)) return run_small(*c, cs, d_in, d_out, nin, nout, &st);
         if (direct_eligible(cs)) return run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st);
+        int r2 = 0;
+        if (wide_eligible(cs)) {
+            bool again = false;
+            r2 = run_wide(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again);
+            if (r2 || !again) return r2;
+        }
         HistWork w;
-        int r2 = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
+        r2 = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
         return r2 ? r2 : run_histsort(*c, cs, d_in, d_out, nin, nout, nullptr, &st, w);
     });
     g_last = st;

@@ -57,6 +57,7 @@ struct DirectResult {
     uint32_t err, scatter_err;
     uint32_t lists[4];    // [3]: digit passes of the one-workgroup sort
     long long sums[2];
+    uint32_t buckets;     // fine buckets of the two-level form
 };
 
 // start / stop (here and below, may be null): events of the launch itself

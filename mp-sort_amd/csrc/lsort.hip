@@ -29,6 +29,7 @@
 #include "device.h"
 #include "lsort.h"
 #include "lsort_dev.h"
+#include "wide.h"
 
 namespace mpsg {
 
@@ -660,6 +661,40 @@ __device__ __forceinline__ void load_items(const GatherSrc<RW>& src, const int (
     }
 #pragma unroll
     for (int k = 0; k < N; k++) RecIO<RW>::load(src.recs, src.begin[j[k]] + (idx[k] - src.pref[j[k]]), r[k]);
+}
+
+// the records of a fine bucket of the two-level partition, gathered from its
+// tiles' runs: run j (of at most kWideRuns) starts at beg[j], and records
+// [pref[j], pref[j+1]) of the bucket come from it (pref: kWideRuns entries,
+// those past the last run above every position); step0: the largest power of
+// two below the number of runs
+template <int RW>
+struct WideSrc {
+    const uint32_t* recs;
+    const uint32_t* beg;
+    const int* pref;
+    int step0;
+    __device__ __forceinline__ void load(int i, uint32_t (&r)[RW]) const {
+        int j = 0;
+        for (int step = step0; step > 0; step >>= 1) j = pref[j + step] <= i ? j + step : j;
+        RecIO<RW>::load(recs, (int64_t)(beg[j] + (uint32_t)(i - pref[j])), r);
+    }
+};
+template <int RW, int N>
+__device__ __forceinline__ void load_items(const WideSrc<RW>& src, const int (&idx)[N], uint32_t (&r)[N][RW]) {
+    int j[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) j[k] = 0;
+    for (int step = src.step0; step > 0; step >>= 1) {
+        int v[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) v[k] = src.pref[j[k] + step];
+#pragma unroll
+        for (int k = 0; k < N; k++) j[k] = v[k] <= idx[k] ? j[k] + step : j[k];
+    }
+#pragma unroll
+    for (int k = 0; k < N; k++)
+        RecIO<RW>::load(src.recs, (int64_t)(src.beg[j[k]] + (uint32_t)(idx[k] - src.pref[j[k]])), r[k]);
 }
 
 // Sorts one bucket of count (1 .. BSort<BLOCK>::CAP) records, given by src,
@@ -1809,6 +1844,140 @@ __global__ __launch_bounds__(kMergeBlock, ITEMS == kMergeItems ? 6 : 4) void mer
     if (checksum_out) block_checksum_add<C::W>(csum, s_sum2, checksum_out);
 }
 
+// ---------------------------------------------------------------------------
+// The fine buckets of the two-level partition (wide.hip): gathered from the
+// tiles of their coarse bucket, in tile order, and sorted.  s_t: the runs'
+// tables (kWideRuns starts, then kWideRuns prefixes), s_tmp: BLOCK / 64 words.
+template <int RW, int BLOCK>
+__device__ __forceinline__ WideSrc<RW> wide_runs(const WideWork& w, const WideBucket& b, const uint32_t* recs,
+                                                 uint32_t* s_t, uint32_t* s_tmp) {
+    static_assert(BLOCK >= kWideRuns, "a thread per run");
+    const int j = threadIdx.x;
+    uint32_t a = 0, len = 0;
+    if (j < b.ntiles) {
+        const uint16_t* ex = w.ex2 + (int64_t)(b.tile0 + j) * kWideStride + b.f;
+        a = ex[0];
+        len = ex[1] - a;
+    }
+    const uint32_t pre = scan_block<BLOCK>(len, s_tmp);
+    if (j < kWideRuns) {
+        s_t[j] = b.first + (uint32_t)j * kWideTile + a;
+        s_t[kWideRuns + j] = j < b.ntiles ? pre : 0x7fffffffu;
+    }
+    __syncthreads();
+    return WideSrc<RW>{recs, s_t, reinterpret_cast<const int*>(s_t + kWideRuns),
+                       b.ntiles > 1 ? 1 << (31 - __clz(b.ntiles - 1)) : 0};
+}
+// the bucket's records are to be put in their place by wide_copy_kernel
+__device__ __forceinline__ void wide_collect(const WideWork& w, uint32_t id, uint32_t cnt) {
+    const uint32_t k = (cnt + kWideCopy - 1) / kWideCopy;
+    const uint32_t at = atomicAdd(&w.lists[4], k);
+    for (uint32_t q = 0; q < k; q++)
+        if (at + q < (uint32_t)w.ncopy) w.copy[at + q] = make_uint2(id, q * kWideCopy);
+}
+
+// One workgroup of 512 threads per fine bucket of at most 3072 records (three
+// share a CU; neighbouring buckets go to one XCD, whose L2 holds the lines
+// their runs share); larger ones are listed for the 1024-thread form.
+template <int RW>
+__global__ __launch_bounds__(kMergeBlock, 6) void wide_sort_kernel(const uint32_t* __restrict__ recs,
+                                                                   uint32_t* __restrict__ dst, LKey lk, WideWork w,
+                                                                   long long* __restrict__ checksum_out) {
+    using C = BSort<kMergeBlock, kMergeItems>;
+    __shared__ uint32_t s_bins[C::BW];
+    __shared__ uint32_t s_t[2 * kWideRuns];
+    __shared__ uint32_t s_scan[C::W];
+    const int64_t per = gridDim.x / 8;
+    const int64_t id = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (w.lists[5] || id >= w.cfine[w.W]) return;
+    const uint32_t cnt = w.fcnt[id];
+    const int64_t base = w.fbase[id];
+    const WideBucket b = w.desc[id];
+    if (cnt == 0 || cnt > (uint32_t)kChunkCap) return;
+    if (cnt > (uint32_t)C::CAP) {
+        if (threadIdx.x == 0) w.medium[atomicAdd(&w.lists[2], 1u)] = (uint32_t)id;
+        return;
+    }
+    const WideSrc<RW> ws = wide_runs<RW, kMergeBlock>(w, b, recs, s_t, s_scan);
+    __builtin_assume(cnt <= (uint32_t)C::CAP && cnt > 0u);
+    const int rc = sort_bucket_lds<RW, kMergeBlock, WideSrc<RW>, kMergeItems>(ws, dst, base, (int)cnt, lk, s_bins,
+                                                                                 checksum_out);
+    if (rc && threadIdx.x == 0) {
+        if (rc == 2) {
+            w.medium[atomicAdd(&w.lists[2], 1u)] = (uint32_t)id;
+        } else {
+            w.hard[atomicAdd(&w.lists[1], 1u)] = (uint32_t)id;
+            wide_collect(w, (uint32_t)id, cnt);
+        }
+    }
+}
+
+// the listed ones, up to 9216 records: persistent blocks walk the list
+template <int RW>
+__global__ __launch_bounds__(kCBlock) void wide_medium_kernel(const uint32_t* __restrict__ recs,
+                                                              uint32_t* __restrict__ dst, LKey lk, WideWork w,
+                                                              long long* __restrict__ checksum_out) {
+    using C = BSort<kCBlock>;
+    __shared__ uint32_t s_bins[C::BW];
+    __shared__ uint32_t s_scan[C::W];
+    if (w.lists[5]) return;
+    const uint32_t nm = w.lists[2];
+    for (uint32_t q = blockIdx.x; q < nm; q += gridDim.x) {
+        const uint32_t id = w.medium[q];
+        const uint32_t cnt = w.fcnt[id];
+        const WideBucket b = w.desc[id];
+        __syncthreads();  // LDS of the previous bucket is free
+        const WideSrc<RW> ws = wide_runs<RW, kCBlock>(w, b, recs, s_bins, s_scan);
+        const int rc = sort_bucket_lds<RW, kCBlock, WideSrc<RW>>(ws, dst, w.fbase[id], (int)cnt, lk, s_bins,
+                                                                 checksum_out);
+        if (rc && threadIdx.x == 0) {
+            w.hard[atomicAdd(&w.lists[1], 1u)] = id;
+            wide_collect(w, id, cnt);
+        }
+    }
+}
+
+// records [first, first + 4096) of the fine buckets of the copy list, to their
+// places in dst: final for a bucket of one key value, otherwise the input of
+// the LDS radix sort (which takes its output's checksum) or the radix path
+template <int RW>
+__global__ __launch_bounds__(kMergeBlock) void wide_copy_kernel(const uint32_t* __restrict__ recs,
+                                                                uint32_t* __restrict__ dst, WideWork w,
+                                                                long long* __restrict__ checksum_out) {
+    constexpr int U = kWideCopy / kMergeBlock;
+    __shared__ uint32_t s_t[2 * kWideRuns];
+    __shared__ uint32_t s_scan[kMergeBlock / 64];
+    __shared__ long long s_sum[kMergeBlock / 64];
+    if (w.lists[5]) return;
+    const uint32_t n = min(w.lists[4], (uint32_t)w.ncopy);
+    long long csum = 0;
+    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
+        const uint2 task = w.copy[q];
+        const int cnt = (int)w.fcnt[task.x];
+        const int64_t base = w.fbase[task.x];
+        const WideBucket b = w.desc[task.x];
+        __syncthreads();  // LDS of the previous task is free
+        const WideSrc<RW> ws = wide_runs<RW, kMergeBlock>(w, b, recs, s_t, s_scan);
+        int idx[U];
+        uint32_t r[U][RW];
+#pragma unroll
+        for (int k = 0; k < U; k++) idx[k] = min((int)task.y + k * kMergeBlock + (int)threadIdx.x, cnt - 1);
+        load_items<RW>(ws, idx, r);
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const int i = (int)task.y + k * kMergeBlock + (int)threadIdx.x;
+            if (i < cnt) {
+                RecIO<RW>::store(dst, base + i, r[k]);
+                if (checksum_out && cnt > kChunkCap) {
+#pragma unroll
+                    for (int v = 0; v < RW; v++) csum += sbyte_sum(r[k][v]);
+                }
+            }
+        }
+    }
+    if (checksum_out) block_checksum_add<kMergeBlock / 64>(csum, s_sum, checksum_out);
+}
+
 // The listed buckets: stable LSD radix sort in LDS over the bytes of
 // (key - min) that vary.  Persistent blocks walk the list.
 template <int RW>
@@ -2339,6 +2508,24 @@ int launch_entries_fixup(int rw, const void* recs, const LKey& lk, const EntryOu
     }
     MPSG_CHECK(hipGetLastError());
     return 0;
+}
+
+int launch_wide_sort(int rw, const void* recs, void* out, const LKey& lk, const WideWork& w, long long* checksum_out,
+                     hipStream_t st) {
+    const uint32_t* s = (const uint32_t*)recs;
+    uint32_t* d = (uint32_t*)out;
+    const dim3 g((unsigned)((w.nfine + 7) / 8 * 8)), gm(256), gc(512);
+    if (rw == 2) hipLaunchKernelGGL(wide_sort_kernel<2>, g, dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
+    else if (rw == 4) hipLaunchKernelGGL(wide_sort_kernel<4>, g, dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
+    else return -1;
+    MPSG_CHECK(hipGetLastError());
+    if (rw == 2) hipLaunchKernelGGL(wide_medium_kernel<2>, gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
+    else hipLaunchKernelGGL(wide_medium_kernel<4>, gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
+    MPSG_CHECK(hipGetLastError());
+    if (rw == 2) hipLaunchKernelGGL(wide_copy_kernel<2>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);
+    else hipLaunchKernelGGL(wide_copy_kernel<4>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);
+    MPSG_CHECK(hipGetLastError());
+    return launch_lsd_sort(rw, d, d, lk, w.fcnt, w.fbase, w.hard, w.lists + 1, w.nfine, checksum_out, st);
 }
 
 }  // namespace mpsg
