@@ -3501,19 +3501,19 @@ int mpsort_gpu_model_train(mpsort_gpu_model** out, const void* sorted, int64_t n
         if (!M.linear_root) {
             // Adam, 2000 steps over 16 interleaved mini-batches, learning rate
             // cosine-annealed from 1e-2 to 1e-4
+            // (each Adam launch leaves the next step's effective weights)
             const int stride = 16, steps = 2000;
+            if ((r2 = launch_mlp_effective(M.raw, M.eff, st))) return r2;
             for (int step = 1; step <= steps; step++) {
                 const int off = (step - 1) % stride;
                 const float lr = 1e-4f + 0.5f * (1e-2f - 1e-4f) * (1.f + std::cos(3.14159265f * step / steps));
-                if ((r2 = launch_mlp_effective(M.raw, M.eff, st))) return r2;
                 if ((r2 = launch_mlp_grad(x, y, S, stride, off, M.raw, M.eff, partial, lossp, st))) return r2;
                 if ((r2 = launch_mlp_adam(M.raw, partial, mlp_grad_blocks(S, stride, off), am, av, lr, step, nullptr,
-                                          st)))
+                                          M.eff, st)))
                     return r2;
             }
             M.steps = steps;
             // loss of the final root over every sample
-            if ((r2 = launch_mlp_effective(M.raw, M.eff, st))) return r2;
             if ((r2 = launch_mlp_grad(x, y, S, 1, 0, M.raw, M.eff, partial, lossp, st))) return r2;
             std::vector<float> lp(grad_blocks);
             MPSG_CHECK(hipMemcpyAsync(lp.data(), lossp, sizeof(float) * grad_blocks, hipMemcpyDeviceToHost, st));
@@ -3643,7 +3643,7 @@ int mpsort_gpu_mlp_grad(const float* raw, const float* x, const float* y, int64_
         return done(fail(MPSORT_ERR_HIP, "copy failed"));
     if ((rc = launch_mlp_effective(d_raw, d_eff, c->st))) return done(rc);
     if ((rc = launch_mlp_grad(d_x, d_y, n, 1, 0, d_raw, d_eff, d_part, d_loss, c->st))) return done(rc);
-    if ((rc = launch_mlp_adam(d_raw, d_part, blocks, nullptr, nullptr, 0.f, 1, d_g, c->st))) return done(rc);
+    if ((rc = launch_mlp_adam(d_raw, d_part, blocks, nullptr, nullptr, 0.f, 1, d_g, nullptr, c->st))) return done(rc);
     std::vector<float> lp(blocks);
     if (hipStreamSynchronize(c->st) != hipSuccess ||
         hipMemcpy(grad, d_g, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost) != hipSuccess ||

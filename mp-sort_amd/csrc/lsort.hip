@@ -1912,12 +1912,15 @@ __global__ __launch_bounds__(kMergeBlock, 6) void wide_sort_kernel(const uint32_
     }
 }
 
-// the listed ones, up to 9216 records: persistent blocks walk the list
-template <int RW>
-__global__ __launch_bounds__(kCBlock) void wide_medium_kernel(const uint32_t* __restrict__ recs,
-                                                              uint32_t* __restrict__ dst, LKey lk, WideWork w,
-                                                              long long* __restrict__ checksum_out) {
-    using C = BSort<kCBlock>;
+// the listed ones: up to 4608 records by 512 threads (two blocks share a CU),
+// up to 9216 by 1024; persistent blocks walk the list
+template <int RW, int BLOCK>
+__global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void wide_medium_kernel(const uint32_t* __restrict__ recs,
+                                                                          uint32_t* __restrict__ dst, LKey lk,
+                                                                          WideWork w,
+                                                                          long long* __restrict__ checksum_out) {
+    using C = BSort<BLOCK>;
+    constexpr uint32_t kFrom = BLOCK == kCBlock ? (uint32_t)kMergeBigCap : 0u;
     __shared__ uint32_t s_bins[C::BW];
     __shared__ uint32_t s_scan[C::W];
     if (w.lists[5]) return;
@@ -1925,11 +1928,12 @@ __global__ __launch_bounds__(kCBlock) void wide_medium_kernel(const uint32_t* __
     for (uint32_t q = blockIdx.x; q < nm; q += gridDim.x) {
         const uint32_t id = w.medium[q];
         const uint32_t cnt = w.fcnt[id];
+        if (cnt <= kFrom || cnt > (uint32_t)C::CAP) continue;
         const WideBucket b = w.desc[id];
         __syncthreads();  // LDS of the previous bucket is free
-        const WideSrc<RW> ws = wide_runs<RW, kCBlock>(w, b, recs, s_bins, s_scan);
-        const int rc = sort_bucket_lds<RW, kCBlock, WideSrc<RW>>(ws, dst, w.fbase[id], (int)cnt, lk, s_bins,
-                                                                 checksum_out);
+        const WideSrc<RW> ws = wide_runs<RW, BLOCK>(w, b, recs, s_bins, s_scan);
+        const int rc = sort_bucket_lds<RW, BLOCK, WideSrc<RW>>(ws, dst, w.fbase[id], (int)cnt, lk, s_bins,
+                                                               checksum_out);
         if (rc && threadIdx.x == 0) {
             w.hard[atomicAdd(&w.lists[1], 1u)] = id;
             wide_collect(w, id, cnt);
@@ -2519,8 +2523,11 @@ int launch_wide_sort(int rw, const void* recs, void* out, const LKey& lk, const 
     else if (rw == 4) hipLaunchKernelGGL(wide_sort_kernel<4>, g, dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
     else return -1;
     MPSG_CHECK(hipGetLastError());
-    if (rw == 2) hipLaunchKernelGGL(wide_medium_kernel<2>, gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
-    else hipLaunchKernelGGL(wide_medium_kernel<4>, gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
+    if (rw == 2) hipLaunchKernelGGL((wide_medium_kernel<2, 512>), gc, dim3(512), 0, st, s, d, lk, w, checksum_out);
+    else hipLaunchKernelGGL((wide_medium_kernel<4, 512>), gc, dim3(512), 0, st, s, d, lk, w, checksum_out);
+    MPSG_CHECK(hipGetLastError());
+    if (rw == 2) hipLaunchKernelGGL((wide_medium_kernel<2, kCBlock>), gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
+    else hipLaunchKernelGGL((wide_medium_kernel<4, kCBlock>), gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
     MPSG_CHECK(hipGetLastError());
     if (rw == 2) hipLaunchKernelGGL(wide_copy_kernel<2>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);
     else hipLaunchKernelGGL(wide_copy_kernel<4>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);

@@ -35,7 +35,7 @@ int mlp_grad_blocks(int64_t n, int64_t stride, int64_t offset);
 int launch_mlp_grad(const float* x, const float* y, int64_t n, int64_t stride, int64_t offset,
                     const float* raw, const float* eff, float* partial, float* loss_partial, hipStream_t st);
 int launch_mlp_adam(float* raw, const float* partial, int nblocks, float* m, float* v, float lr, int step,
-                    float* grad_out, hipStream_t st);
+                    float* grad_out, float* eff, hipStream_t st);
 int launch_leaves(const float* x, const float* y, int64_t S, const float* eff, int L, int linear_root,
                   int* leaf, int64_t* start, float* leaves, hipStream_t st);
 // xstart[l] = smallest x the root routes to leaf l or beyond

@@ -28,117 +28,200 @@ __device__ __forceinline__ float softplus_f(float v) {
 }
 __device__ __forceinline__ float sigmoid_f(float v) { return 1.f / (1.f + expf(-v)); }
 
+__device__ __forceinline__ bool positive_param(int i) {
+    return (i >= kW1 && i < kW1 + kH) || (i >= kW2 && i < kW2 + kH * kH) || (i >= kW3 && i < kW3 + kH);
+}
+
 // effective (non-negative) weights from raw parameters
 __global__ void mlp_effective_kernel(const float* __restrict__ raw, float* __restrict__ eff) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= kMlpParams) return;
     const float v = raw[i];
-    const bool positive = (i >= kW1 && i < kW1 + kH) || (i >= kW2 && i < kW2 + kH * kH) ||
-                          (i >= kW3 && i < kW3 + kH);
-    eff[i] = positive ? softplus_f(v) : v;
+    eff[i] = positive_param(i) ? softplus_f(v) : v;
 }
 
-// Loss = mean over the batch of (r(x_i) - y_i)^2.  Block b computes the
-// gradient of its samples and writes it to partial[b][kMlpParams] (no float
-// atomics: the reduction order is fixed, so training is deterministic).
-constexpr int kGradBlock = 256;
-__global__ __launch_bounds__(kGradBlock) void mlp_grad_kernel(const float* __restrict__ x,
-                                                              const float* __restrict__ y, int64_t n,
-                                                              int64_t stride, int64_t offset,
-                                                              const float* __restrict__ raw,
-                                                              const float* __restrict__ eff_g,
-                                                              float* __restrict__ partial,
-                                                              float* __restrict__ loss_partial) {
-    __shared__ float e[kMlpParams];
-    __shared__ float s_h1[kGradBlock][kH + 1];
-    __shared__ float s_dz2[kGradBlock][kH + 1];
-    __shared__ float s_red[(kGradBlock / 64) * (3 * kH + 2)];
-    const int tid = threadIdx.x;
-    for (int i = tid; i < kMlpParams; i += kGradBlock) e[i] = eff_g[i];
-    __syncthreads();
-    const int64_t si = offset + ((int64_t)blockIdx.x * kGradBlock + tid) * stride;
+// Loss = mean over the batch of (r(x_i) - y_i)^2.  Blocks (b, 0 .. 3) compute
+// the gradient of samples 256 b .. 256 b + 255 and write it to
+// partial[b][kMlpParams] (no float atomics: every sum has a fixed order, so
+// training is deterministic).  A step has few samples (16384 of 262144), so
+// its time is the length of one block's chain of dependent operations: four
+// threads share a sample (part p holds hidden units 8 p .. 8 p + 7 of both
+// layers), and four blocks share 256 samples (block q repeats the forward
+// pass and takes the gradients of units 8 q .. 8 q + 7).  A training step of
+// 16384 samples took 78 us with one thread per sample, one block per 256
+// samples and the weights' transform in a launch of its own.
+constexpr int kGradBlock = 256;               // samples of a block
+constexpr int kGradThreads = 4 * kGradBlock;
+constexpr int kGradUnits = kH / 4;            // hidden units of a part
+constexpr int kGradRow = kGradBlock + 4;      // floats of a unit's LDS row (16-byte aligned)
+__global__ __launch_bounds__(kGradThreads) void mlp_grad_kernel(const float* __restrict__ x,
+                                                                const float* __restrict__ y, int64_t n,
+                                                                int64_t stride, int64_t offset,
+                                                                const float* __restrict__ raw,
+                                                                const float* __restrict__ eff_g,
+                                                                float* __restrict__ partial,
+                                                                float* __restrict__ loss_partial) {
+    constexpr int U = kGradUnits, G = kGradBlock / 64, Q = U / 4;  // units a part, waves a part, units a thread backward
+    constexpr int kSmall = 3 * U + 2;
+    __shared__ __attribute__((aligned(16))) float e[(kMlpParams + 3) / 4 * 4];
+    __shared__ __attribute__((aligned(16))) float s_h1[kH][kGradRow];
+    __shared__ __attribute__((aligned(16))) float s_d[kH][kGradRow];  // h2, then dz2
+    __shared__ float s_red[G][kSmall];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int s = tid & (kGradBlock - 1), part = __builtin_amdgcn_readfirstlane(tid / kGradBlock);
+    const int q = blockIdx.y, g = wave & (G - 1);
+    for (int i = tid; i < kMlpParams; i += kGradThreads) e[i] = eff_g[i];
+    const int64_t si = offset + ((int64_t)blockIdx.x * kGradBlock + s) * stride;
     const bool valid = si < n;
     const float inv_n = 1.f / (float)((n - offset + stride - 1) / stride);
-    float h1[kH], h2[kH];
-    float xv = valid ? x[si] : 0.f;
-    float r = mlp_forward(e, xv, h1, h2);
-    const float dy = valid ? 2.f * (r - y[si]) * inv_n : 0.f;
-    const float lv = valid ? (r - y[si]) * (r - y[si]) * inv_n : 0.f;
-    // backward
-    float dz1[kH];
+    const float xv = valid ? x[si] : 0.f;
+    const float yv = valid ? y[si] : 0.f;
+    __syncthreads();
+    const int u0 = part * U;
 #pragma unroll
-    for (int j = 0; j < kH; j++) dz1[j] = 0.f;
-#pragma unroll 4
+    for (int j = 0; j < U; j++) s_h1[u0 + j][s] = tanhf(e[kW1 + u0 + j] * xv + e[kB1 + u0 + j]);
+    __syncthreads();
+    float h2[U];
+    {
+        float h1[kH];
+#pragma unroll
+        for (int j = 0; j < kH; j++) h1[j] = s_h1[j][s];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            float z = e[kB2 + u0 + k];
+#pragma unroll
+            for (int j = 0; j < kH; j++) z += e[kW2 + (u0 + k) * kH + j] * h1[j];
+            h2[k] = tanhf(z);
+            s_d[u0 + k][s] = h2[k];
+        }
+    }
+    __syncthreads();
+    float r = e[kB3];
+#pragma unroll
+    for (int k = 0; k < kH; k++) r += e[kW3 + k] * s_d[k][s];
+    const float dy = valid ? 2.f * (r - yv) * inv_n : 0.f;
+    const float lv = valid ? (r - yv) * (r - yv) * inv_n : 0.f;
+    // this thread's units of the gradient: Q of the block's
+    const int v0 = q * U + part * Q;
+    float hv[Q];
+#pragma unroll
+    for (int j = 0; j < Q; j++) hv[j] = s_d[v0 + j][s];
+    __syncthreads();  // every h2 is read
+#pragma unroll
+    for (int k = 0; k < U; k++) s_d[u0 + k][s] = dy * e[kW3 + u0 + k] * (1.f - h2[k] * h2[k]);
+    __syncthreads();
+    float dz1[Q];
+#pragma unroll
+    for (int j = 0; j < Q; j++) dz1[j] = 0.f;
+#pragma unroll
     for (int k = 0; k < kH; k++) {
-        const float dz2 = dy * e[kW3 + k] * (1.f - h2[k] * h2[k]);
-        s_dz2[tid][k] = dz2;
+        const float dz2 = s_d[k][s];
 #pragma unroll
-        for (int j = 0; j < kH; j++) dz1[j] += dz2 * e[kW2 + k * kH + j];
+        for (int j = 0; j < Q; j++) dz1[j] += dz2 * e[kW2 + k * kH + v0 + j];
     }
-#pragma unroll
-    for (int j = 0; j < kH; j++) {
-        dz1[j] *= (1.f - h1[j] * h1[j]);
-        s_h1[tid][j] = h1[j];
-    }
-    // per-sample small gradients (w1, b1, w3: 3 x 32, b3, loss): wave
-    // shuffle sums, then a fixed-order sum over the block's waves
-    float* out = partial + (int64_t)blockIdx.x * kMlpParams;
-    const int lane = tid & 63, wv = tid >> 6;
-    constexpr int kSmall = 3 * kH + 2;
-    for (int q = 0; q < kSmall; q++) {
-        float v;
-        if (q < kH) v = dz1[q] * xv;
-        else if (q < 2 * kH) v = dz1[q - kH];
-        else if (q < 3 * kH) v = dy * h2[q - 2 * kH];
-        else if (q == 3 * kH) v = dy;
-        else v = lv;
+    // per-sample small gradients (w1, b1, w3, b3, loss): wave shuffle sums,
+    // then a fixed-order sum over the waves of 64 samples
+    auto wave_sum = [&](float v, int slot) {
+        asm volatile("" : "+v"(v));  // the product is rounded before it is summed
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (lane == 0) s_red[wv * kSmall + q] = v;
+        if (lane == 0) s_red[g][slot] = v;
+    };
+#pragma unroll
+    for (int j = 0; j < Q; j++) {
+        const float h = s_h1[v0 + j][s];
+        dz1[j] *= (1.f - h * h);
+        wave_sum(dz1[j] * xv, part * Q + j);
+        wave_sum(dz1[j], U + part * Q + j);
+        wave_sum(dy * hv[j], 2 * U + part * Q + j);
     }
+    if (part == 0) wave_sum(dy, 3 * U);
+    if (part == 1) wave_sum(lv, 3 * U + 1);
     __syncthreads();
-    if (tid < kSmall) {
+    float* out = partial + (int64_t)blockIdx.x * kMlpParams;
+    if (tid < U * kH) {
+        // W2[k][j] = sum dz2[:,k] * h1[:,j]: a thread per output, the samples
+        // in order, four read at a time
+        const int k = q * U + tid / kH, j = tid % kH;
+        const float4* a = reinterpret_cast<const float4*>(s_d[k]);
+        const float4* b = reinterpret_cast<const float4*>(s_h1[j]);
         float acc = 0.f;
-        for (int w = 0; w < kGradBlock / 64; w++) acc += s_red[w * kSmall + tid];
-        if (tid < kH) out[kW1 + tid] = acc * sigmoid_f(raw[kW1 + tid]);
-        else if (tid < 2 * kH) out[kB1 + tid - kH] = acc;
-        else if (tid < 3 * kH) out[kW3 + tid - 2 * kH] = acc * sigmoid_f(raw[kW3 + tid - 2 * kH]);
-        else if (tid == 3 * kH) out[kB3] = acc;
-        else loss_partial[blockIdx.x] = acc;
-    }
-    // b2[k] = sum dz2[:,k]; W2[k][j] = sum dz2[:,k] * h1[:,j]  (1024 + 32 outputs)
-    __syncthreads();
-    for (int o = tid; o < kH * kH + kH; o += kGradBlock) {
-        float acc = 0.f;
-        if (o < kH * kH) {
-            const int k = o / kH, j = o % kH;
-            for (int s = 0; s < kGradBlock; s++) acc += s_dz2[s][k] * s_h1[s][j];
-            out[kW2 + o] = acc * sigmoid_f(raw[kW2 + o]);
-        } else {
-            const int k = o - kH * kH;
-            for (int s = 0; s < kGradBlock; s++) acc += s_dz2[s][k];
-            out[kB2 + k] = acc;
+#pragma unroll 8
+        for (int i = 0; i < kGradBlock / 4; i++) {
+            const float4 d = a[i], h = b[i];
+            acc += d.x * h.x;
+            acc += d.y * h.y;
+            acc += d.z * h.z;
+            acc += d.w * h.w;
         }
+        out[kW2 + k * kH + j] = acc * sigmoid_f(raw[kW2 + k * kH + j]);
+    } else if (tid < U * kH + U) {
+        const int k = q * U + tid - U * kH;
+        const float4* a = reinterpret_cast<const float4*>(s_d[k]);
+        float acc = 0.f;
+#pragma unroll 8
+        for (int i = 0; i < kGradBlock / 4; i++) {
+            const float4 d = a[i];
+            acc += d.x;
+            acc += d.y;
+            acc += d.z;
+            acc += d.w;
+        }
+        out[kB2 + k] = acc;
+    } else if (tid >= 512 && tid < 512 + kSmall) {
+        const int t = tid - 512, j = q * U + t % U;
+        float acc = 0.f;
+#pragma unroll
+        for (int w = 0; w < G; w++) acc += s_red[w][t];
+        if (t < U) out[kW1 + j] = acc * sigmoid_f(raw[kW1 + j]);
+        else if (t < 2 * U) out[kB1 + j] = acc;
+        else if (t < 3 * U) out[kW3 + j] = acc * sigmoid_f(raw[kW3 + j]);
+        else if (t == 3 * U && q == 0) out[kB3] = acc;
+        else if (t == 3 * U + 1 && q == 0) loss_partial[blockIdx.x] = acc;
     }
 }
 
-// sum the per-block partial gradients (fixed order) and apply one Adam step
-__global__ void mlp_adam_kernel(float* __restrict__ raw, const float* __restrict__ partial, int nblocks,
-                                float* __restrict__ m, float* __restrict__ v, float lr, float beta1,
-                                float beta2, float eps, int step, float* __restrict__ grad_out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// sum the per-block partial gradients (fixed order) and apply one Adam step,
+// then the next step's effective weights (eff, may be null).  A thread per
+// parameter, one wave per block: the sums are latency, spread over the CUs;
+// 16 loads of a thread are in flight.
+constexpr int kAdamBlock = 64;
+__global__ __launch_bounds__(kAdamBlock) void mlp_adam_kernel(float* __restrict__ raw,
+                                                              const float* __restrict__ partial, int nblocks,
+                                                              float* __restrict__ m, float* __restrict__ v, float lr,
+                                                              float beta1, float beta2, float eps, int step,
+                                                              float* __restrict__ grad_out, float* __restrict__ eff) {
+    const int i = blockIdx.x * kAdamBlock + threadIdx.x;
     if (i >= kMlpParams) return;
+    float m0 = 0.f, v0 = 0.f, w0 = 0.f;
+    if (lr > 0.f) {
+        m0 = m[i];
+        v0 = v[i];
+        w0 = raw[i];
+    }
     float g = 0.f;
-    for (int b = 0; b < nblocks; b++) g += partial[(int64_t)b * kMlpParams + i];
+    constexpr int U = 16;
+    for (int b = 0; b < nblocks; b += U) {
+        float p[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) p[u] = partial[(int64_t)min(b + u, nblocks - 1) * kMlpParams + i];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (b + u < nblocks) g += p[u];
+    }
     if (grad_out) grad_out[i] = g;
     if (lr <= 0.f) return;  // gradient only
-    const float mi = beta1 * m[i] + (1.f - beta1) * g;
-    const float vi = beta2 * v[i] + (1.f - beta2) * g * g;
+    // (the rounding of each step is fixed: a network's weights do not depend on
+    // how the compiler pairs these products)
+    const float mi = __builtin_fmaf(1.f - beta1, g, beta1 * m0);
+    const float vi = __builtin_fmaf(g, (1.f - beta2) * g, beta2 * v0);
     m[i] = mi;
     v[i] = vi;
     const float mh = mi / (1.f - powf(beta1, (float)step));
     const float vh = vi / (1.f - powf(beta2, (float)step));
-    raw[i] -= lr * mh / (sqrtf(vh) + eps);
+    const float w = w0 - lr * mh / (sqrtf(vh) + eps);
+    raw[i] = w;
+    if (eff) eff[i] = positive_param(i) ? softplus_f(w) : w;
 }
 
 // root prediction of every sample -> leaf index, made monotone over the sorted
@@ -566,16 +649,16 @@ int mlp_grad_blocks(int64_t n, int64_t stride, int64_t offset) {
 int launch_mlp_grad(const float* x, const float* y, int64_t n, int64_t stride, int64_t offset,
                     const float* raw, const float* eff, float* partial, float* loss_partial, hipStream_t st) {
     const int blocks = mlp_grad_blocks(n, stride, offset);
-    hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(kGradBlock), 0, st, x, y, n, stride, offset, raw,
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks, 4), dim3(kGradThreads), 0, st, x, y, n, stride, offset, raw,
                        eff, partial, loss_partial);
     MPSG_CHECK(hipGetLastError());
     return 0;
 }
 
 int launch_mlp_adam(float* raw, const float* partial, int nblocks, float* m, float* v, float lr, int step,
-                    float* grad_out, hipStream_t st) {
-    hipLaunchKernelGGL(mlp_adam_kernel, dim3(nblk(kMlpParams, 256)), dim3(256), 0, st, raw, partial, nblocks,
-                       m, v, lr, 0.9f, 0.999f, 1e-8f, step, grad_out);
+                    float* grad_out, float* eff, hipStream_t st) {
+    hipLaunchKernelGGL(mlp_adam_kernel, dim3(nblk(kMlpParams, kAdamBlock)), dim3(kAdamBlock), 0, st, raw, partial,
+                       nblocks, m, v, lr, 0.9f, 0.999f, 1e-8f, step, grad_out, eff);
     MPSG_CHECK(hipGetLastError());
     return 0;
 }
