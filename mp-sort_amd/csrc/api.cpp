@@ -1884,8 +1884,6 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
 
 // ---- the same in two partition levels (wide.hip), above one level's sizes
 constexpr int64_t kWideCoarse = (int64_t)1 << 17;  // records per coarse bucket while 512 suffice
-constexpr int kWideAvg = 1843;                     // records per fine bucket: 3072 less 2.7 deviations
-                                                   // of a size estimated from 16 sample keys
 static bool wide_eligible(const CallShape& cs) {
     return direct_asked(cs) && (cs.rw == 2 || cs.rw == 4) && cs.ntot > kDirectMaxRecords &&
            cs.ntot <= kWideMaxRecords;
@@ -2397,12 +2395,14 @@ struct SegGroup {
     Buf plan_buf;  // arrays of the large-segment plan
     Buf tmp;       // record buffer for the digit passes
     Buf lookback;
-    int nsmall = 0, nlarge = 0;
-    int nsmall_form = 0;  // of the small segments, those sorted by the form chosen (the others: 1024 threads)
+    Buf wide_buf;  // arrays of the segments sorted by one partition level
+    int nsmall = 0, nlarge = 0, nwide = 0;
+    int form_n[kSegForms] = {};  // the small segments, by the form that sorts them (4, 3, the chosen one, 0)
+    WideWork wide;
     uint32_t* d_cnt = nullptr;
     int64_t* d_base = nullptr;
     uint32_t* d_hard = nullptr;
-    uint32_t* d_counters = nullptr;  // [0] oversized, [1] hard, [2] epoch, [4] hard of the 1024-thread list
+    uint32_t* d_counters = nullptr;  // [0] oversized, [2] epoch, [4 + form] hard
     int64_t* d_ovf = nullptr;
     SegSortPlan plan;
     uint64_t epoch_used = 0;  // epoch steps consumed since the last reset
@@ -2473,52 +2473,122 @@ static void seg_tune_store() {
 }
 
 // lay out the group's device arrays for its current tuning
+// the segments sorted by one partition level: their tables
+static int seg_group_wide(SegGroup& G, const std::vector<int64_t>& cnt, const std::vector<int64_t>& beg,
+                          hipStream_t st) {
+    int rc = 0;
+    WideWork& w = G.wide;
+    memset(&w, 0, sizeof w);
+    const int n = (int)cnt.size();
+    std::vector<uint32_t> tot(n), cbase(n), cw(n), ctile(n + 1), cfine(n + 1), tile_c;
+    for (int i = 0; i < n; i++) {
+        tot[i] = (uint32_t)cnt[i];
+        cbase[i] = (uint32_t)beg[i];
+        cw[i] = (uint32_t)((cnt[i] + kWideAvg - 1) / kWideAvg);
+        ctile[i + 1] = ctile[i] + (uint32_t)((cnt[i] + kWideTile - 1) / kWideTile);
+        cfine[i + 1] = cfine[i] + cw[i];
+        tile_c.insert(tile_c.end(), ctile[i + 1] - ctile[i], (uint32_t)i);
+        w.n += cnt[i];
+    }
+    w.W = n;
+    w.avg = kWideAvg;
+    w.nt2 = ctile[n];
+    w.nfine = cfine[n];
+    w.ncopy = w.n / kWideCopy + w.nfine;
+    w.max_overflow = (int)(w.n / kChunkCap + 1);
+    uint32_t* d_tile_c = nullptr;
+    auto lay = [&](auto& a, auto take) {
+        take(a, w.tot, (size_t)n);
+        take(a, w.cbase, (size_t)n);
+        take(a, w.cw, (size_t)n);
+        take(a, w.ctile, (size_t)n + 1);
+        take(a, w.cfine, (size_t)n + 1);
+        take(a, d_tile_c, (size_t)w.nt2);
+        take(a, w.tables2, (size_t)n * kWideBuckets);
+        take(a, w.ex2, (size_t)w.nt2 * kWideStride);
+        take(a, w.desc, (size_t)w.nfine);
+        take(a, w.fcnt, (size_t)w.nfine);
+        take(a, w.fbase, (size_t)w.nfine);
+        take(a, w.medium, (size_t)w.nfine);
+        take(a, w.hard, (size_t)w.nfine);
+        take(a, w.copy, (size_t)w.ncopy);
+        take(a, w.overflow, (size_t)2 * w.max_overflow);
+        take(a, w.lists, (size_t)8);
+    };
+    Sizer sz;
+    lay(sz, [](Sizer& a, auto*& p, size_t k) { a.take<std::remove_reference_t<decltype(*p)>>(k); });
+    if ((rc = G.wide_buf.ensure(sz.off + 4096)) || (rc = G.tmp.ensure((size_t)G.nrec * G.elsize))) return rc;
+    Arena ar{(char*)G.wide_buf.p};
+    lay(ar, [](Arena& a, auto*& p, size_t k) { p = a.take<std::remove_reference_t<decltype(*p)>>(k); });
+    w.tile_c = d_tile_c;
+    auto up = [&](uint32_t* d, const std::vector<uint32_t>& h) -> int {
+        MPSG_CHECK(hipMemcpyAsync(d, h.data(), sizeof(uint32_t) * h.size(), hipMemcpyHostToDevice, st));
+        return 0;
+    };
+    if ((rc = up(w.tot, tot)) || (rc = up(w.cbase, cbase)) || (rc = up(w.cw, cw)) || (rc = up(w.ctile, ctile)) ||
+        (rc = up(w.cfine, cfine)) || (rc = up(d_tile_c, tile_c)))
+        return rc;
+    MPSG_CHECK(hipStreamSynchronize(st));
+    return 0;
+}
+
 static int seg_group_prepare(SegGroup& G, hipStream_t st) {
     int rc = 0;
     const int npass = G.ks.key_bytes;
     const bool lds_ok = (G.rw == 2 || G.rw == 4) && G.ks.key_bytes <= 8;
     const int thr = lds_ok ? G.tune.threshold : 0;
-    const int fcap = segments_lds_cap(G.tune.form);
-    std::vector<uint32_t> scnt, mcnt;
-    std::vector<int64_t> sbase, mbase, lcnt, lbeg;
-    for (int i = 0; i < G.nseg; i++) {
-        if (G.count[i] == 0) continue;
-        if (G.count[i] <= thr && G.count[i] <= fcap) {
+    // a small segment takes the smallest form that holds it: 128, 256 or 512
+    // threads leave a CU eleven, six or two workgroups, where 1024 threads
+    // leave one (10,000,000 records in 20,000 segments of 110 to 1100: 445 us
+    // with 1024 threads each).  A segment above the threshold is sampled,
+    // grouped by bucket and its buckets sorted in LDS: three passes over its
+    // records, where the digit passes take one per key byte and one more to
+    // count.  Segments above kWideSegMax have more than one level's buckets.
+    std::vector<int> forms{4, 3, G.tune.form ? G.tune.form : 1, 0};
+    if (G.each) forms = G.tune.form ? std::vector<int>{G.tune.form, 0} : std::vector<int>{0};
+    std::vector<uint32_t> scnt;
+    std::vector<int64_t> sbase, lcnt, lbeg, wcnt, wbeg;
+    int64_t above = 0;
+    for (int f = 0; f < kSegForms; f++) G.form_n[f] = 0;
+    for (int form : forms) {
+        const int64_t cap = std::min<int64_t>(thr, segments_lds_cap(form));
+        for (int i = 0; i < G.nseg; i++) {
+            if (G.count[i] <= above || G.count[i] > cap) continue;
             scnt.push_back((uint32_t)G.count[i]);
             sbase.push_back(G.begin[i]);
-        } else if (G.count[i] <= thr) {
-            mcnt.push_back((uint32_t)G.count[i]);
-            mbase.push_back(G.begin[i]);
-        } else {
-            lcnt.push_back(G.count[i]);
-            lbeg.push_back(G.begin[i]);
+            G.form_n[form]++;
         }
+        above = std::max(above, cap);
     }
-    // the form's segments, then those above its capacity
-    G.nsmall_form = (int)scnt.size();
-    scnt.insert(scnt.end(), mcnt.begin(), mcnt.end());
-    sbase.insert(sbase.end(), mbase.begin(), mbase.end());
+    for (int i = 0; i < G.nseg; i++) {
+        if (G.count[i] == 0 || G.count[i] <= thr) continue;
+        const bool wide = lds_ok && !G.each && G.count[i] <= kWideSegMax && G.nrec < ((int64_t)1 << 31);
+        (wide ? wcnt : lcnt).push_back(G.count[i]);
+        (wide ? wbeg : lbeg).push_back(G.begin[i]);
+    }
     G.nsmall = (int)scnt.size();
     G.nlarge = (int)lcnt.size();
+    G.nwide = (int)wcnt.size();
     Sizer sz;
     sz.take<uint32_t>((size_t)G.nsmall + 1);
     sz.take<int64_t>((size_t)G.nsmall + 1);
     sz.take<uint32_t>((size_t)G.nsmall + 1);
-    sz.take<uint32_t>(8);
+    sz.take<uint32_t>(16);
     sz.take<int64_t>(2);
     if ((rc = G.small.ensure(sz.off + 4096))) return rc;
     Arena a{(char*)G.small.p};
     G.d_cnt = a.take<uint32_t>((size_t)G.nsmall + 1);
     G.d_base = a.take<int64_t>((size_t)G.nsmall + 1);
     G.d_hard = a.take<uint32_t>((size_t)G.nsmall + 1);
-    G.d_counters = a.take<uint32_t>(8);
+    G.d_counters = a.take<uint32_t>(16);
     G.d_ovf = a.take<int64_t>(2);
     if (G.nsmall) {
         MPSG_CHECK(hipMemcpyAsync(G.d_cnt, scnt.data(), sizeof(uint32_t) * G.nsmall, hipMemcpyHostToDevice, st));
         MPSG_CHECK(hipMemcpyAsync(G.d_base, sbase.data(), sizeof(int64_t) * G.nsmall, hipMemcpyHostToDevice, st));
     }
-    if ((rc = launch_fill_u32(G.d_counters, 0u, 8, st))) return rc;
+    if ((rc = launch_fill_u32(G.d_counters, 0u, 16, st))) return rc;
     G.epoch_used = 0;
+    if (G.nwide && (rc = seg_group_wide(G, wcnt, wbeg, st))) return rc;
 
     SegSortPlan& p = G.plan;
     p = SegSortPlan();
@@ -2583,14 +2653,17 @@ static int seg_group_enqueue_each(SegGroup& G, hipStream_t st);
 static int seg_group_enqueue(SegGroup& G, hipStream_t st) {
     int rc = 0;
     if ((rc = launch_fill_u32(G.d_counters, 0u, 2, st))) return rc;
-    if ((rc = launch_fill_u32(G.d_counters + 4, 0u, 1, st))) return rc;
+    if ((rc = launch_fill_u32(G.d_counters + 4, 0u, kSegForms, st))) return rc;
     if (G.each) return seg_group_enqueue_each(G, st);
-    if (G.nsmall) {
-        if ((rc = launch_segments_lds(G.rw, G.tune.form, G.in, G.out, G.lk, G.d_cnt, G.d_base, G.nsmall_form,
-                                      G.nsmall - G.nsmall_form, G.d_ovf, G.d_counters, G.d_hard, G.d_counters + 1,
-                                      G.d_counters + 4, st)))
+    int64_t at = 0;
+    for (int form : {4, 3, 2, 1, 0}) {
+        const int64_t n = G.form_n[form];
+        if ((rc = launch_segments_lds(G.rw, form, G.in, G.out, G.lk, G.d_cnt + at, G.d_base + at, n, G.d_ovf, G.d_counters,
+                                      G.d_hard + at, G.d_counters + 4 + form, st)))
             return rc;
+        at += n;
     }
+    if (G.nwide && (rc = launch_wide_segments(G.rw, G.in, G.tmp.p, G.out, G.lk, G.wide, st))) return rc;
     if (G.nlarge) {
         if ((rc = launch_add_u32(G.d_counters + 2, (uint32_t)kMaxPasses, st))) return rc;
         if ((rc = seg_count(G.plan, G.in, nullptr, st)))
@@ -2613,12 +2686,10 @@ static int seg_group_enqueue(SegGroup& G, hipStream_t st) {
 static int seg_group_enqueue_each(SegGroup& G, hipStream_t st) {
     int rc = 0;
     for (int i = 0; i < G.nsmall; i++) {
-        if ((rc = launch_fill_u32(G.d_counters + 1, 0u, 1, st))) return rc;
-        if ((rc = launch_fill_u32(G.d_counters + 4, 0u, 1, st))) return rc;
-        const bool in_form = i < G.nsmall_form;
-        if ((rc = launch_segments_lds(G.rw, G.tune.form, G.in, G.out, G.lk, G.d_cnt + i, G.d_base + i, in_form ? 1 : 0,
-                                      in_form ? 0 : 1, G.d_ovf, G.d_counters, G.d_hard, G.d_counters + 1,
-                                      G.d_counters + 4, st)))
+        const int form = i < G.nsmall - G.form_n[0] ? G.tune.form : 0;
+        if ((rc = launch_fill_u32(G.d_counters + 4 + form, 0u, 1, st))) return rc;
+        if ((rc = launch_segments_lds(G.rw, form, G.in, G.out, G.lk, G.d_cnt + i, G.d_base + i, 1, G.d_ovf, G.d_counters,
+                                      G.d_hard, G.d_counters + 4 + form, st)))
             return rc;
     }
     const int npass = G.ks.key_bytes;
@@ -3811,7 +3882,7 @@ int mpsort_gpu_segplan_info(const mpsort_gpu_segplan* p, int group, int* nsmall,
     if (!p || group < 0 || group >= (int)p->groups.size()) return fail(MPSORT_ERR_ARG, "no such group");
     const SegGroup* G = p->groups[group];
     if (nsmall) *nsmall = G->nsmall;
-    if (nlarge) *nlarge = G->nlarge;
+    if (nlarge) *nlarge = G->nlarge + G->nwide;
     if (block) *block = G->tune.tile.block;
     if (items) *items = G->tune.tile.items;
     if (threshold) *threshold = G->tune.threshold;
@@ -3833,6 +3904,7 @@ int mpsort_gpu_segplan_free(mpsort_gpu_segplan* p) {
     for (SegGroup* G : p->groups) {
         G->small.release();
         G->plan_buf.release();
+        G->wide_buf.release();
         G->tmp.release();
         G->lookback.release();
         delete G;

@@ -605,7 +605,8 @@ template <int BLOCK, int ITEMS = kCItems>
 struct BSort {
     static constexpr int B = BLOCK, W = BLOCK / 64, I = ITEMS, CAP = BLOCK * ITEMS;
     static constexpr int NL = CAP / (kLongMin + 1) + 1;  // bins of more than kLongMin records, at most
-    static constexpr int SUB = CAP > 3072 ? 63 : 31;             // bins per sample interval
+    // bins per sample interval: about one record a bin at the largest size
+    static constexpr int SUB = CAP > 3072 ? 63 : (CAP > 1536 ? 31 : (CAP > 768 ? 15 : 7));
     static constexpr int FINE = (kSamp + 1) * SUB;               // bins
     static constexpr int NB = (FINE + 1 + BLOCK - 1) / BLOCK * BLOCK;  // bin counters
     static constexpr int BW = NB;                                // words of the bin arrays
@@ -713,7 +714,7 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
                                                 const EntryOut eo = EntryOut{}, int ej = 0, int eb = 0) {
     using C = BSort<BLOCK, ITEMS>;
     // one-value long bins placed here (the 512 x 6 form hands them on)
-    constexpr bool DUPS = BLOCK == kCBlock || ITEMS >= 9;
+    constexpr bool DUPS = BLOCK != 512 || ITEMS >= 9;
     __shared__ uint64_t s_gkey[C::CAP + 8];  // key of each bin-order slot (+8: unrolled reads)
     __shared__ uint16_t s_sbin[C::CAP];      // bin of each bin-order slot, then the final
                                              // slot of each bucket position (s_pos)
@@ -1130,7 +1131,7 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
 // BLOCK = 512: buckets above BSort<512>::CAP (up to kChunkCap) go to the
 // medium list for the 1024-thread form (medium must then be given).
 template <int RW, int BLOCK, int ITEMS = kCItems>
-__global__ __launch_bounds__(BLOCK, ITEMS <= 6 ? 6 : 2048 / BLOCK) void interp_sort_kernel(
+__global__ __launch_bounds__(BLOCK, BLOCK < 512 ? 5 : (ITEMS <= 6 ? 6 : 2048 / BLOCK)) void interp_sort_kernel(
     const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, LKey lk,
     const uint32_t* __restrict__ hist, const int64_t* __restrict__ bucket_base,
     const uint64_t* __restrict__ tables, int64_t tstride, int64_t nbuckets, int64_t* __restrict__ overflow,
@@ -2046,6 +2047,90 @@ __global__ __launch_bounds__(kCBlock) void lsd_sort_kernel(
     if (checksum_out) block_checksum_add(csum, s_sum, checksum_out);
 }
 
+// The fine buckets of several values above the in-LDS capacity (rare: the
+// sample missed their weight), in place in dst at the positions listed: one
+// workgroup each, stable 8-bit digit passes between dst and the same
+// positions of tmp, over the key bytes that vary.  For callers that cannot
+// take a count back to the host (a captured plan).
+template <int RW>
+__global__ __launch_bounds__(kCBlock) void wide_big_kernel(uint32_t* dst, uint32_t* tmp, LKey lk, WideWork w) {
+    __shared__ uint32_t s_start[256];
+    __shared__ uint32_t s_base[kCWaves][256];
+    __shared__ uint32_t s_tmp[kCWaves];
+    __shared__ unsigned long long s_diff;
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const uint32_t n = min(w.lists[0], (uint32_t)w.max_overflow);
+    const uint64_t lt = __lanemask_lt();
+    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
+        const int64_t base = w.overflow[2 * q], cnt = w.overflow[2 * q + 1];
+        uint32_t *a = dst, *b = tmp;
+        uint32_t r[RW];
+        RecIO<RW>::load(a, base, r);
+        const uint64_t k0 = lkey<RW>(r, lk);
+        __syncthreads();
+        if (tid == 0) s_diff = 0;
+        __syncthreads();
+        uint64_t diff = 0;
+        for (int64_t i = tid; i < cnt; i += kCBlock) {
+            RecIO<RW>::load(a, base + i, r);
+            diff |= lkey<RW>(r, lk) ^ k0;
+        }
+        if (diff) atomicOr(&s_diff, (unsigned long long)diff);
+        __syncthreads();
+        diff = s_diff;
+        for (int sh = 0; sh < 64; sh += 8) {
+            if (((diff >> sh) & 0xffu) == 0) continue;
+            if (tid < 256) s_start[tid] = 0;
+            __syncthreads();
+            for (int64_t i = tid; i < cnt; i += kCBlock) {
+                RecIO<RW>::load(a, base + i, r);
+                atomicAdd(&s_start[(lkey<RW>(r, lk) >> sh) & 0xffu], 1u);
+            }
+            __syncthreads();
+            const uint32_t ex = scan_block<kCBlock>(tid < 256 ? s_start[tid] : 0u, s_tmp);
+            if (tid < 256) s_start[tid] = ex;
+            for (int64_t c0 = 0; c0 < cnt; c0 += kCBlock) {
+                for (int i = tid; i < kCWaves * 256; i += kCBlock) (&s_base[0][0])[i] = 0;
+                __syncthreads();
+                const bool in = c0 + tid < cnt;
+                RecIO<RW>::load(a, base + (in ? c0 + tid : 0), r);
+                const uint32_t d = (uint32_t)(lkey<RW>(r, lk) >> sh) & 0xffu;
+                uint64_t peers = __ballot(in);
+#pragma unroll
+                for (int bb = 0; bb < 8; bb++) {
+                    const bool bit = (d >> bb) & 1u;
+                    const uint64_t m = __ballot(bit);
+                    peers &= bit ? m : ~m;
+                }
+                const uint32_t rank = __popcll(peers & lt);
+                if (in && rank == 0) s_base[wave][d] = (uint32_t)__popcll(peers);
+                __syncthreads();
+                if (tid < 256) {
+                    uint32_t at = s_start[tid];
+                    for (int v = 0; v < kCWaves; v++) {
+                        const uint32_t c = s_base[v][tid];
+                        s_base[v][tid] = at;
+                        at += c;
+                    }
+                    s_start[tid] = at;
+                }
+                __syncthreads();
+                if (in) RecIO<RW>::store(b, base + s_base[wave][d] + rank, r);
+                __syncthreads();
+            }
+            uint32_t* t = a;
+            a = b;
+            b = t;
+        }
+        if (a != dst) {
+            for (int64_t i = tid; i < cnt; i += kCBlock) {
+                RecIO<RW>::load(a, base + i, r);
+                RecIO<RW>::store(dst, base + i, r);
+            }
+        }
+    }
+}
+
 // The listed segments ({begin, count} pairs) that hold one key value are in
 // stable order already.  one_value_check_kernel: gridDim.x workgroups per
 // segment (blockIdx.y) compare their share of its keys with its first key;
@@ -2250,40 +2335,47 @@ int launch_chunk_sort(int rw, const void* src, void* dst, const LKey& lk, const 
 }
 
 int launch_segments_lds(int rw, int form, const void* src, void* dst, const LKey& lk, const uint32_t* cnt,
-                        const int64_t* base, int64_t na, int64_t nb, int64_t* overflow, uint32_t* noverflow,
-                        uint32_t* hard, uint32_t* nhard_a, uint32_t* nhard_b, hipStream_t st) {
-    if (form == 0 || na == 0)
-        return launch_chunk_sort(rw, src, dst, lk, cnt, base, nullptr, 0, na + nb, overflow, noverflow, 1, hard,
-                                 nhard_a, nullptr, false, st);
+                        const int64_t* base, int64_t n, int64_t* overflow, uint32_t* noverflow, uint32_t* hard,
+                        uint32_t* nhard, hipStream_t st) {
+    if (n <= 0) return 0;
+    if (form == 0)
+        return launch_chunk_sort(rw, src, dst, lk, cnt, base, nullptr, 0, n, overflow, noverflow, 1, hard, nhard,
+                                 nullptr, false, st);
     const uint32_t* s = (const uint32_t*)src;
     uint32_t* d = (uint32_t*)dst;
-    const unsigned grid = (unsigned)na, persistent = (unsigned)std::min<int64_t>(na, 512);
+    const unsigned grid = (unsigned)n, persistent = (unsigned)std::min<int64_t>(n, 512);
     const uint32_t cap = (uint32_t)kChunkCap;
-#define MPSG_SEGFORM(R, I) do { \
-        hipLaunchKernelGGL((interp_sort_kernel<R, kMergeBlock, I>), dim3(grid), dim3(kMergeBlock), 0, st, s, d, lk, \
-                           cnt, base, nullptr, 0, na, overflow, noverflow, 1, hard, nhard_a, nullptr, nullptr, nullptr, \
+#define MPSG_SEGFORM(R, B, I) do { \
+        hipLaunchKernelGGL((interp_sort_kernel<R, B, I>), dim3(grid), dim3(B), 0, st, s, d, lk, \
+                           cnt, base, nullptr, 0, n, overflow, noverflow, 1, hard, nhard, nullptr, nullptr, nullptr, \
                            0, EntryOut{}, cap); \
         MPSG_CHECK(hipGetLastError()); \
         hipLaunchKernelGGL(lsd_sort_kernel<R>, dim3(persistent), dim3(kCBlock), 0, st, s, d, lk, cnt, base, \
-                           (const uint32_t*)hard, (const uint32_t*)nhard_a, nullptr); \
+                           (const uint32_t*)hard, (const uint32_t*)nhard, nullptr); \
     } while (0)
-    switch (rw * 4 + form) {
-        case 9: MPSG_SEGFORM(2, kSmallItems); break;
-        case 10: MPSG_SEGFORM(2, kMergeItems); break;
-        case 17: MPSG_SEGFORM(4, kSmallItems); break;
-        case 18: MPSG_SEGFORM(4, kMergeItems); break;
+    switch (rw * 8 + form) {
+        case 17: MPSG_SEGFORM(2, kMergeBlock, kSmallItems); break;
+        case 18: MPSG_SEGFORM(2, kMergeBlock, kMergeItems); break;
+        case 19: MPSG_SEGFORM(2, 256, 6); break;
+        case 20: MPSG_SEGFORM(2, 128, 6); break;
+        case 33: MPSG_SEGFORM(4, kMergeBlock, kSmallItems); break;
+        case 34: MPSG_SEGFORM(4, kMergeBlock, kMergeItems); break;
+        case 35: MPSG_SEGFORM(4, 256, 6); break;
+        case 36: MPSG_SEGFORM(4, 128, 6); break;
         default: return -1;
     }
 #undef MPSG_SEGFORM
     MPSG_CHECK(hipGetLastError());
-    if (nb == 0) return 0;
-    // the segments above the form's capacity: the 1024-thread form
-    return launch_chunk_sort(rw, src, dst, lk, cnt + na, base + na, nullptr, 0, nb, overflow, noverflow, 1, hard + na,
-                             nhard_b, nullptr, false, st);
+    return 0;
 }
-
 int segments_lds_cap(int form) {
-    return form == 1 ? BSort<kMergeBlock, kSmallItems>::CAP : (form == 2 ? BSort<kMergeBlock, kMergeItems>::CAP : kChunkCap);
+    switch (form) {
+        case 1: return BSort<kMergeBlock, kSmallItems>::CAP;
+        case 2: return BSort<kMergeBlock, kMergeItems>::CAP;
+        case 3: return BSort<256, 6>::CAP;
+        case 4: return BSort<128, 6>::CAP;
+        default: return kChunkCap;
+    }
 }
 
 int launch_chunk_sort_small(int rw, const void* src, void* dst, const LKey& lk, const uint32_t* hist,
@@ -2533,6 +2625,14 @@ int launch_wide_sort(int rw, const void* recs, void* out, const LKey& lk, const 
     else hipLaunchKernelGGL(wide_copy_kernel<4>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);
     MPSG_CHECK(hipGetLastError());
     return launch_lsd_sort(rw, d, d, lk, w.fcnt, w.fbase, w.hard, w.lists + 1, w.nfine, checksum_out, st);
+}
+
+int launch_wide_big(int rw, void* out, void* tmp, const LKey& lk, const WideWork& w, hipStream_t st) {
+    if (rw == 2) hipLaunchKernelGGL(wide_big_kernel<2>, dim3(256), dim3(kCBlock), 0, st, (uint32_t*)out, (uint32_t*)tmp, lk, w);
+    else if (rw == 4) hipLaunchKernelGGL(wide_big_kernel<4>, dim3(256), dim3(kCBlock), 0, st, (uint32_t*)out, (uint32_t*)tmp, lk, w);
+    else return -1;
+    MPSG_CHECK(hipGetLastError());
+    return 0;
 }
 
 }  // namespace mpsg

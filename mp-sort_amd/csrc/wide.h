@@ -56,6 +56,7 @@ struct WideWork {
     int max_overflow;
     uint32_t* lists;           // 8: [0] oversized, [1] LDS radix, [2] 1024-thread form, [4] copy tasks,
                                // [5] set: a coarse bucket of several values has too many tiles
+    const uint32_t* tile_c;    // segments: coarse bucket (segment) of every level 2 tile
     uint32_t* tally;           // 2 * kDirectMaxP^2: records below and at most each splitter, by rank
 };
 
@@ -74,6 +75,17 @@ int launch_wide_level2(int rw, const void* src, void* dst, void* out, const LKey
 // listed in overflow, for the radix path)
 int launch_wide_sort(int rw, const void* recs, void* out, const LKey& lk, const WideWork& w, long long* checksum_out,
                      hipStream_t st);
+// the listed oversized buckets of several values, in place in out, by digit
+// passes through the same positions of tmp
+int launch_wide_big(int rw, void* out, void* tmp, const LKey& lk, const WideWork& w, hipStream_t st);
+// independent segments (w.W of them, each at most kWideSegMax records, as
+// coarse buckets whose tot, cbase, ctile, cfine, cw and tile_c the caller has
+// set): src -> out through tmp (src may equal out); nothing but kernels
+constexpr int kWideAvg = 1843;  // records per fine bucket: 3072 less 2.7 deviations of a size estimated
+                                // from 16 sample keys
+constexpr int64_t kWideSegMax = (int64_t)kWideBuckets * kWideAvg;
+int launch_wide_segments(int rw, const void* src, void* tmp, void* out, const LKey& lk, const WideWork& w,
+                         hipStream_t st);
 // splitters, counts and layout (as launch_direct_counts): part is level 1's dst
 int launch_wide_counts(int rw, const void* out, const void* part, const LKey& lk, const DirectShape& sh,
                        const DirectWork& d, const WideWork& w, DirectResult* res, hipEvent_t stop, hipStream_t st);

@@ -105,12 +105,17 @@ __device__ __forceinline__ void wide_locate(const WideWork& w, int c, uint32_t t
 
 // ---------------------------------------------------------------------------
 // One tile grouped by bucket, stably, and written to its own place: records
-// loaded wave-major (16 loads of a thread in flight), their buckets searched
+// loaded wave-major (12 loads of a thread in flight), their buckets searched
 // in LDS, ranked by ballots among the lanes of a wave and by counters across
 // its items and the waves, and staged through LDS 8 bytes of a record at a
-// time so that two workgroups share a CU.  Level 1 (L2 false) reads the input
-// in place; level 2 reads the runs of its coarse bucket.
-template <int RW, bool L2>
+// time so that two workgroups share a CU.  kLevel1 reads the input in place;
+// kLevel2 reads the runs of its coarse bucket; kSegment is level 2 of a
+// segment, which lies in one piece.
+// 12 records per thread: with 16 (tiles of 8192) the registers spilled, and
+// the two levels of 2^28 x 16 B took 3.00 and 3.35 ms instead of 2.11 and 2.30
+// (8.6 GB each: 4.1 and 3.7 TB/s).
+enum { kLevel1, kLevel2, kSegment };
+template <int RW, int MODE>
 __global__ __launch_bounds__(kWBlock, 4) void wide_part_kernel(const uint32_t* __restrict__ src,
                                                                uint32_t* __restrict__ dst, uint32_t* __restrict__ out,
                                                                LKey lk, SegDev seg, WideWork w,
@@ -131,16 +136,16 @@ __global__ __launch_bounds__(kWBlock, 4) void wide_part_kernel(const uint32_t* _
     uint32_t begin;  // first record of the tile in dst
     int cnt, nw;
     uint16_t* ex;
-    if constexpr (L2) {
+    if constexpr (MODE != kLevel1) {
         if (w.lists[5] || tile >= w.ctile[w.W]) return;
-        const int c = wide_coarse_of(w, tile, s_tmp);
+        const int c = MODE == kSegment ? (int)w.tile_c[tile] : wide_coarse_of(w, tile, s_tmp);
         const uint32_t p0 = (tile - w.ctile[c]) * (uint32_t)kWideTile, n = w.tot[c];
         begin = w.cbase[c] + p0;
         cnt = (int)min((uint32_t)kWideTile, n - p0);
         nw = (int)w.cw[c];
         ex = w.ex2 + (int64_t)tile * kWideStride;
         s_tab[tid] = tid < nw - 1 ? w.tables2[(int64_t)c * kWideBuckets + tid] : ~0ull;
-        wide_locate(w, c, tile, p0, p0 + (uint32_t)cnt, s.rt, s_tmp);
+        if constexpr (MODE == kLevel2) wide_locate(w, c, tile, p0, p0 + (uint32_t)cnt, s.rt, s_tmp);
     } else {
         const int j = seg_of_tile(seg, tile);
         begin = (uint32_t)(seg.begin[j] + (int64_t)(tile - (uint32_t)seg.tile_start[j]) * kWideTile);
@@ -156,9 +161,9 @@ __global__ __launch_bounds__(kWBlock, 4) void wide_part_kernel(const uint32_t* _
 #pragma unroll
     for (int k = 0; k < kWItems; k++) {
         const uint32_t q = (uint32_t)min(wave * kWSpan + k * 64 + lane, cnt - 1);
-        RecIO<RW>::load(src, (int64_t)(L2 ? s.rt.at(q) : begin + q), r[k]);
+        RecIO<RW>::load(src, (int64_t)(MODE == kLevel2 ? s.rt.at(q) : begin + q), r[k]);
     }
-    if (!L2 || nw == 0) {
+    if (MODE == kLevel1 || (MODE == kLevel2 && nw == 0)) {
         // level 1 sums the input; a coarse bucket of one key value is in its
         // final order, and summed as output
         if (checksum) {
@@ -390,7 +395,7 @@ __global__ __launch_bounds__(256) void wide_offsets_kernel(WideWork w) {
 // ---------------------------------------------------------------------------
 // Fine boundaries: up to 4096 keys at even positions of a coarse bucket,
 // sorted in LDS by a bitonic network.
-template <int RW>
+template <int RW, bool SEG>
 __global__ __launch_bounds__(1024) void wide_sample_kernel(const uint32_t* __restrict__ src, LKey lk, WideWork w) {
     constexpr int I = kWideSamples / 1024;
     __shared__ uint64_t s_k[kWideSamples];
@@ -399,34 +404,44 @@ __global__ __launch_bounds__(1024) void wide_sample_kernel(const uint32_t* __res
     const int nw = (int)w.cw[c];
     if (w.lists[5] || nw <= 1) return;
     const uint32_t n = w.tot[c], m = min((uint32_t)kWideSamples, n);
-    const uint32_t* off = w.off + (int64_t)c * w.ntpad;
-    const uint16_t* loc = w.loc + (int64_t)c * w.ntpad;
-    const uint32_t t0 = w.ctile[c], t1 = w.ctile[c + 1];
-    uint32_t pos[I], lo[I], hi[I];
+    uint32_t pos[I], at[I];
 #pragma unroll
     for (int k = 0; k < I; k++) {
         const uint32_t u = min((uint32_t)(k * 1024 + tid), m - 1);
         pos[k] = (uint32_t)(((2 * (uint64_t)u + 1) * n) / (2 * (uint64_t)m));
-        const uint32_t t = t0 + pos[k] / kWideTile;
-        lo[k] = w.first[t];
-        hi[k] = t + 1 < t1 ? w.first[t + 1] + 1 : (uint32_t)w.nt;  // off[lo] <= pos < off[hi]
+        at[k] = w.cbase[c] + pos[k];
     }
-    for (;;) {
-        bool more = false;
+    if constexpr (!SEG) {
+        // the level 1 tile of each position: off[lo] <= pos < off[hi]
+        const uint32_t* off = w.off + (int64_t)c * w.ntpad;
+        const uint16_t* loc = w.loc + (int64_t)c * w.ntpad;
+        const uint32_t t0 = w.ctile[c], t1 = w.ctile[c + 1];
+        uint32_t lo[I], hi[I];
 #pragma unroll
         for (int k = 0; k < I; k++) {
-            if (hi[k] - lo[k] > 1) {
-                const uint32_t mid = (lo[k] + hi[k]) >> 1;
-                if (off[mid] <= pos[k]) lo[k] = mid; else hi[k] = mid;
-                more = true;
-            }
+            const uint32_t t = t0 + pos[k] / kWideTile;
+            lo[k] = w.first[t];
+            hi[k] = t + 1 < t1 ? w.first[t + 1] + 1 : (uint32_t)w.nt;
         }
-        if (!more) break;
+        for (;;) {
+            bool more = false;
+#pragma unroll
+            for (int k = 0; k < I; k++) {
+                if (hi[k] - lo[k] > 1) {
+                    const uint32_t mid = (lo[k] + hi[k]) >> 1;
+                    if (off[mid] <= pos[k]) lo[k] = mid; else hi[k] = mid;
+                    more = true;
+                }
+            }
+            if (!more) break;
+        }
+#pragma unroll
+        for (int k = 0; k < I; k++) at[k] = w.tile_beg[lo[k]] + loc[lo[k]] + (pos[k] - off[lo[k]]);
     }
 #pragma unroll
     for (int k = 0; k < I; k++) {
         uint32_t r[RW];
-        RecIO<RW>::load(src, (int64_t)(w.tile_beg[lo[k]] + loc[lo[k]] + (pos[k] - off[lo[k]])), r);
+        RecIO<RW>::load(src, (int64_t)at[k], r);
         s_k[k * 1024 + tid] = (uint32_t)(k * 1024 + tid) < m ? lkey<RW>(r, lk) : ~0ull;
     }
     __syncthreads();
@@ -661,8 +676,8 @@ int launch_wide_level1(int rw, const void* src, void* dst, const LKey& lk, const
     const uint32_t* s = (const uint32_t*)src;
     uint32_t* o = (uint32_t*)dst;
     const dim3 g((unsigned)w.nt), b(kWBlock);
-    if (rw == 2) hipLaunchKernelGGL((wide_part_kernel<2, false>), g, b, 0, st, s, o, nullptr, lk, sd, w, checksum);
-    else if (rw == 4) hipLaunchKernelGGL((wide_part_kernel<4, false>), g, b, 0, st, s, o, nullptr, lk, sd, w, checksum);
+    if (rw == 2) hipLaunchKernelGGL((wide_part_kernel<2, kLevel1>), g, b, 0, st, s, o, nullptr, lk, sd, w, checksum);
+    else if (rw == 4) hipLaunchKernelGGL((wide_part_kernel<4, kLevel1>), g, b, 0, st, s, o, nullptr, lk, sd, w, checksum);
     else return -1;
     MPSG_CHECK(hipGetLastError());
     // off and loc have an entry past the last tile (the bucket's total)
@@ -676,8 +691,8 @@ int launch_wide_level1(int rw, const void* src, void* dst, const LKey& lk, const
     MPSG_CHECK(hipGetLastError());
     hipLaunchKernelGGL(wide_offsets_kernel, dim3((unsigned)rows, cb), dim3(256), 0, st, w);
     MPSG_CHECK(hipGetLastError());
-    if (rw == 2) hipLaunchKernelGGL(wide_sample_kernel<2>, dim3((unsigned)w.W), dim3(1024), 0, st, o, lk, w);
-    else hipLaunchKernelGGL(wide_sample_kernel<4>, dim3((unsigned)w.W), dim3(1024), 0, st, o, lk, w);
+    if (rw == 2) hipLaunchKernelGGL((wide_sample_kernel<2, false>), dim3((unsigned)w.W), dim3(1024), 0, st, o, lk, w);
+    else hipLaunchKernelGGL((wide_sample_kernel<4, false>), dim3((unsigned)w.W), dim3(1024), 0, st, o, lk, w);
     MPSG_CHECK(hipGetLastError());
     return 0;
 }
@@ -688,13 +703,34 @@ int launch_wide_level2(int rw, const void* src, void* dst, void* out, const LKey
     uint32_t *d = (uint32_t*)dst, *o = (uint32_t*)out;
     const dim3 g((unsigned)w.nt2), b(kWBlock);
     const SegDev none{nullptr, nullptr, nullptr, 0, 0};
-    if (rw == 2) hipLaunchKernelGGL((wide_part_kernel<2, true>), g, b, 0, st, s, d, o, lk, none, w, checksum_out);
-    else if (rw == 4) hipLaunchKernelGGL((wide_part_kernel<4, true>), g, b, 0, st, s, d, o, lk, none, w, checksum_out);
+    if (rw == 2) hipLaunchKernelGGL((wide_part_kernel<2, kLevel2>), g, b, 0, st, s, d, o, lk, none, w, checksum_out);
+    else if (rw == 4) hipLaunchKernelGGL((wide_part_kernel<4, kLevel2>), g, b, 0, st, s, d, o, lk, none, w, checksum_out);
     else return -1;
     MPSG_CHECK(hipGetLastError());
     hipLaunchKernelGGL(wide_fine_kernel, dim3((unsigned)w.W), dim3(kWideBuckets), 0, st, w);
     MPSG_CHECK(hipGetLastError());
     return 0;
+}
+
+int launch_wide_segments(int rw, const void* src, void* tmp, void* out, const LKey& lk, const WideWork& w,
+                         hipStream_t st) {
+    const uint32_t* s = (const uint32_t*)src;
+    uint32_t* t = (uint32_t*)tmp;
+    const dim3 g((unsigned)w.nt2), b(kWBlock), gw((unsigned)w.W);
+    const SegDev none{nullptr, nullptr, nullptr, 0, 0};
+    int rc = 0;
+    if (rw != 2 && rw != 4) return -1;
+    if ((rc = launch_fill_u32(w.lists, 0u, 8, st))) return rc;
+    if (rw == 2) hipLaunchKernelGGL((wide_sample_kernel<2, true>), gw, dim3(1024), 0, st, s, lk, w);
+    else hipLaunchKernelGGL((wide_sample_kernel<4, true>), gw, dim3(1024), 0, st, s, lk, w);
+    MPSG_CHECK(hipGetLastError());
+    if (rw == 2) hipLaunchKernelGGL((wide_part_kernel<2, kSegment>), g, b, 0, st, s, t, nullptr, lk, none, w, nullptr);
+    else hipLaunchKernelGGL((wide_part_kernel<4, kSegment>), g, b, 0, st, s, t, nullptr, lk, none, w, nullptr);
+    MPSG_CHECK(hipGetLastError());
+    hipLaunchKernelGGL(wide_fine_kernel, gw, dim3(kWideBuckets), 0, st, w);
+    MPSG_CHECK(hipGetLastError());
+    if ((rc = launch_wide_sort(rw, tmp, out, lk, w, nullptr, st))) return rc;
+    return launch_wide_big(rw, out, tmp, lk, w, st);
 }
 
 int launch_wide_counts(int rw, const void* out, const void* part, const LKey& lk, const DirectShape& sh,
