@@ -1911,12 +1911,13 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     WideWork w;
     memset(&w, 0, sizeof w);
     w.W = sh.W;
-    w.avg = kWideAvg;
+    w.avg = kWideFine;
     w.n = n;
     w.nt = sh.ntiles;
     w.ntpad = (w.nt + 64) / 64 * 64;
     w.nt2 = n / kWideTile + w.W;
     w.nfine = n / w.avg + w.W;
+    w.ngrid = wide_grid(n, w.W);
     w.ncopy = n / kWideCopy + w.nfine;
     w.max_overflow = (int)(n / kChunkCap + 1);
     auto lay = [&](auto& a, auto take) {
@@ -2480,20 +2481,20 @@ static int seg_group_wide(SegGroup& G, const std::vector<int64_t>& cnt, const st
     WideWork& w = G.wide;
     memset(&w, 0, sizeof w);
     const int n = (int)cnt.size();
-    std::vector<uint32_t> tot(n), cbase(n), cw(n), ctile(n + 1), cfine(n + 1), tile_c;
+    std::vector<uint32_t> tot(n), cbase(n), cw(n), ctile(n + 1), tile_c;
     for (int i = 0; i < n; i++) {
         tot[i] = (uint32_t)cnt[i];
         cbase[i] = (uint32_t)beg[i];
-        cw[i] = (uint32_t)((cnt[i] + kWideAvg - 1) / kWideAvg);
+        cw[i] = (uint32_t)std::min<int64_t>(kWideBuckets, (cnt[i] + kWideFine - 1) / kWideFine);
         ctile[i + 1] = ctile[i] + (uint32_t)((cnt[i] + kWideTile - 1) / kWideTile);
-        cfine[i + 1] = cfine[i] + cw[i];
+        w.nfine += cw[i];
         tile_c.insert(tile_c.end(), ctile[i + 1] - ctile[i], (uint32_t)i);
         w.n += cnt[i];
     }
     w.W = n;
-    w.avg = kWideAvg;
+    w.avg = kWideFine;
     w.nt2 = ctile[n];
-    w.nfine = cfine[n];
+    w.ngrid = wide_grid(w.n, w.W);
     w.ncopy = w.n / kWideCopy + w.nfine;
     w.max_overflow = (int)(w.n / kChunkCap + 1);
     uint32_t* d_tile_c = nullptr;
@@ -2502,7 +2503,6 @@ static int seg_group_wide(SegGroup& G, const std::vector<int64_t>& cnt, const st
         take(a, w.cbase, (size_t)n);
         take(a, w.cw, (size_t)n);
         take(a, w.ctile, (size_t)n + 1);
-        take(a, w.cfine, (size_t)n + 1);
         take(a, d_tile_c, (size_t)w.nt2);
         take(a, w.tables2, (size_t)n * kWideBuckets);
         take(a, w.ex2, (size_t)w.nt2 * kWideStride);
@@ -2526,7 +2526,7 @@ static int seg_group_wide(SegGroup& G, const std::vector<int64_t>& cnt, const st
         return 0;
     };
     if ((rc = up(w.tot, tot)) || (rc = up(w.cbase, cbase)) || (rc = up(w.cw, cw)) || (rc = up(w.ctile, ctile)) ||
-        (rc = up(w.cfine, cfine)) || (rc = up(d_tile_c, tile_c)))
+        (rc = up(d_tile_c, tile_c)))
         return rc;
     MPSG_CHECK(hipStreamSynchronize(st));
     return 0;

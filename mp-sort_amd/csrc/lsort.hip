@@ -1846,9 +1846,10 @@ __global__ __launch_bounds__(kMergeBlock, ITEMS == kMergeItems ? 6 : 4) void mer
 }
 
 // ---------------------------------------------------------------------------
-// The fine buckets of the two-level partition (wide.hip): gathered from the
-// tiles of their coarse bucket, in tile order, and sorted.  s_t: the runs'
-// tables (kWideRuns starts, then kWideRuns prefixes), s_tmp: BLOCK / 64 words.
+// The groups of fine buckets of the two-level partition (wide.hip): gathered
+// from the tiles of their coarse bucket, in tile order, and sorted.  s_t: the
+// runs' tables (kWideRuns starts, then kWideRuns prefixes), s_tmp: BLOCK / 64
+// words.
 template <int RW, int BLOCK>
 __device__ __forceinline__ WideSrc<RW> wide_runs(const WideWork& w, const WideBucket& b, const uint32_t* recs,
                                                  uint32_t* s_t, uint32_t* s_tmp) {
@@ -1856,9 +1857,9 @@ __device__ __forceinline__ WideSrc<RW> wide_runs(const WideWork& w, const WideBu
     const int j = threadIdx.x;
     uint32_t a = 0, len = 0;
     if (j < b.ntiles) {
-        const uint16_t* ex = w.ex2 + (int64_t)(b.tile0 + j) * kWideStride + b.f;
-        a = ex[0];
-        len = ex[1] - a;
+        const uint16_t* ex = w.ex2 + (int64_t)(b.tile0 + j) * kWideStride;
+        a = ex[b.f];
+        len = ex[b.fe] - a;
     }
     const uint32_t pre = scan_block<BLOCK>(len, s_tmp);
     if (j < kWideRuns) {
@@ -1877,9 +1878,11 @@ __device__ __forceinline__ void wide_collect(const WideWork& w, uint32_t id, uin
         if (at + q < (uint32_t)w.ncopy) w.copy[at + q] = make_uint2(id, q * kWideCopy);
 }
 
-// One workgroup of 512 threads per fine bucket of at most 3072 records (three
-// share a CU; neighbouring buckets go to one XCD, whose L2 holds the lines
-// their runs share); larger ones are listed for the 1024-thread form.
+// One workgroup of 512 threads per group of at most 3072 records (three share
+// a CU; neighbouring groups go to one XCD, whose L2 holds the lines their runs
+// share); larger ones are listed for the larger forms.  No loop over groups:
+// it kept the kernel's arguments live across the sort, which then spilled 29
+// registers a thread (4.8 instead of 3.6 ms on 2^28 x 16 B).
 template <int RW>
 __global__ __launch_bounds__(kMergeBlock, 6) void wide_sort_kernel(const uint32_t* __restrict__ recs,
                                                                    uint32_t* __restrict__ dst, LKey lk, WideWork w,
@@ -1888,40 +1891,67 @@ __global__ __launch_bounds__(kMergeBlock, 6) void wide_sort_kernel(const uint32_
     __shared__ uint32_t s_bins[C::BW];
     __shared__ uint32_t s_t[2 * kWideRuns];
     __shared__ uint32_t s_scan[C::W];
-    const int64_t per = gridDim.x / 8;
-    const int64_t id = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-    if (w.lists[5] || id >= w.cfine[w.W]) return;
+    const uint32_t ngroups = min(w.lists[6], (uint32_t)w.ngrid), per = (ngroups + 7) / 8;
+    const uint32_t q = blockIdx.x / 8, id = (blockIdx.x % 8) * per + q;
+    if (w.lists[5] || q >= per || id >= ngroups) return;
     const uint32_t cnt = w.fcnt[id];
     const int64_t base = w.fbase[id];
     const WideBucket b = w.desc[id];
     if (cnt == 0 || cnt > (uint32_t)kChunkCap) return;
     if (cnt > (uint32_t)C::CAP) {
-        if (threadIdx.x == 0) w.medium[atomicAdd(&w.lists[2], 1u)] = (uint32_t)id;
+        if (threadIdx.x == 0) w.medium[atomicAdd(&w.lists[2], 1u)] = id;
         return;
     }
     const WideSrc<RW> ws = wide_runs<RW, kMergeBlock>(w, b, recs, s_t, s_scan);
     __builtin_assume(cnt <= (uint32_t)C::CAP && cnt > 0u);
-    const int rc = sort_bucket_lds<RW, kMergeBlock, WideSrc<RW>, kMergeItems>(ws, dst, base, (int)cnt, lk, s_bins,
-                                                                                 checksum_out);
+    const int rc = sort_bucket_lds<RW, kMergeBlock, WideSrc<RW>, kMergeItems>(
+        ws, dst, base, (int)cnt, lk, s_bins, checksum_out);
     if (rc && threadIdx.x == 0) {
         if (rc == 2) {
-            w.medium[atomicAdd(&w.lists[2], 1u)] = (uint32_t)id;
+            w.medium[atomicAdd(&w.lists[2], 1u)] = id;
         } else {
-            w.hard[atomicAdd(&w.lists[1], 1u)] = (uint32_t)id;
-            wide_collect(w, (uint32_t)id, cnt);
+            w.hard[atomicAdd(&w.lists[1], 1u)] = id;
+            wide_collect(w, id, cnt);
         }
     }
 }
 
-// the listed ones: up to 4608 records by 512 threads (two blocks share a CU),
-// up to 9216 by 1024; persistent blocks walk the list
+// The listed groups of up to 4608 records, one workgroup of 512 threads each
+// (two share a CU) for the first gridDim of them.  A loop over the list
+// spilled 38 registers a thread (Zipf keys, 10,000,019 x 8 B: 306 us, now 240).
 template <int RW, int BLOCK>
-__global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void wide_medium_kernel(const uint32_t* __restrict__ recs,
-                                                                          uint32_t* __restrict__ dst, LKey lk,
-                                                                          WideWork w,
-                                                                          long long* __restrict__ checksum_out) {
-    using C = BSort<BLOCK>;
-    constexpr uint32_t kFrom = BLOCK == kCBlock ? (uint32_t)kMergeBigCap : 0u;
+__device__ __forceinline__ void wide_medium_one(const WideWork& w, uint32_t id, uint32_t cnt, const uint32_t* recs,
+                                                uint32_t* dst, const LKey& lk, uint32_t* s_bins, uint32_t* s_scan,
+                                                long long* checksum_out) {
+    const WideBucket b = w.desc[id];
+    const WideSrc<RW> ws = wide_runs<RW, BLOCK>(w, b, recs, s_bins, s_scan);
+    const int rc = sort_bucket_lds<RW, BLOCK, WideSrc<RW>>(ws, dst, w.fbase[id], (int)cnt, lk, s_bins, checksum_out);
+    if (rc && threadIdx.x == 0) {
+        w.hard[atomicAdd(&w.lists[1], 1u)] = id;
+        wide_collect(w, id, cnt);
+    }
+}
+template <int RW>
+__global__ __launch_bounds__(kMergeBlock, 4) void wide_medium_kernel(const uint32_t* __restrict__ recs,
+                                                                     uint32_t* __restrict__ dst, LKey lk, WideWork w,
+                                                                     long long* __restrict__ checksum_out) {
+    using C = BSort<kMergeBlock>;
+    __shared__ uint32_t s_bins[C::BW];
+    __shared__ uint32_t s_scan[C::W];
+    if (w.lists[5] || blockIdx.x >= w.lists[2]) return;
+    const uint32_t id = w.medium[blockIdx.x];
+    const uint32_t cnt = w.fcnt[id];
+    if (cnt > (uint32_t)C::CAP) return;
+    wide_medium_one<RW, kMergeBlock>(w, id, cnt, recs, dst, lk, s_bins, s_scan, checksum_out);
+}
+
+// the larger ones, up to 9216 records, and those past the first nsmall: 1024
+// threads; persistent blocks walk the list
+template <int RW>
+__global__ __launch_bounds__(kCBlock) void wide_large_kernel(const uint32_t* __restrict__ recs,
+                                                             uint32_t* __restrict__ dst, LKey lk, WideWork w,
+                                                             uint32_t nsmall, long long* __restrict__ checksum_out) {
+    using C = BSort<kCBlock>;
     __shared__ uint32_t s_bins[C::BW];
     __shared__ uint32_t s_scan[C::W];
     if (w.lists[5]) return;
@@ -1929,20 +1959,13 @@ __global__ __launch_bounds__(BLOCK, 2048 / BLOCK) void wide_medium_kernel(const 
     for (uint32_t q = blockIdx.x; q < nm; q += gridDim.x) {
         const uint32_t id = w.medium[q];
         const uint32_t cnt = w.fcnt[id];
-        if (cnt <= kFrom || cnt > (uint32_t)C::CAP) continue;
-        const WideBucket b = w.desc[id];
-        __syncthreads();  // LDS of the previous bucket is free
-        const WideSrc<RW> ws = wide_runs<RW, BLOCK>(w, b, recs, s_bins, s_scan);
-        const int rc = sort_bucket_lds<RW, BLOCK, WideSrc<RW>>(ws, dst, w.fbase[id], (int)cnt, lk, s_bins,
-                                                               checksum_out);
-        if (rc && threadIdx.x == 0) {
-            w.hard[atomicAdd(&w.lists[1], 1u)] = id;
-            wide_collect(w, id, cnt);
-        }
+        if ((cnt <= (uint32_t)kMergeBigCap && q < nsmall) || cnt > (uint32_t)C::CAP) continue;
+        __syncthreads();  // LDS of the previous group is free
+        wide_medium_one<RW, kCBlock>(w, id, cnt, recs, dst, lk, s_bins, s_scan, checksum_out);
     }
 }
 
-// records [first, first + 4096) of the fine buckets of the copy list, to their
+// records [first, first + 4096) of the groups of the copy list, to their
 // places in dst: final for a bucket of one key value, otherwise the input of
 // the LDS radix sort (which takes its output's checksum) or the radix path
 template <int RW>
@@ -2610,16 +2633,18 @@ int launch_wide_sort(int rw, const void* recs, void* out, const LKey& lk, const 
                      hipStream_t st) {
     const uint32_t* s = (const uint32_t*)recs;
     uint32_t* d = (uint32_t*)out;
-    const dim3 g((unsigned)((w.nfine + 7) / 8 * 8)), gm(256), gc(512);
+    const dim3 g((unsigned)w.ngrid), gm(256), gc(512);
     if (rw == 2) hipLaunchKernelGGL(wide_sort_kernel<2>, g, dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
     else if (rw == 4) hipLaunchKernelGGL(wide_sort_kernel<4>, g, dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
     else return -1;
     MPSG_CHECK(hipGetLastError());
-    if (rw == 2) hipLaunchKernelGGL((wide_medium_kernel<2, 512>), gc, dim3(512), 0, st, s, d, lk, w, checksum_out);
-    else hipLaunchKernelGGL((wide_medium_kernel<4, 512>), gc, dim3(512), 0, st, s, d, lk, w, checksum_out);
+    // (blocks without an entry end at once: 16,384 of them take about 10 us)
+    const unsigned nm = (unsigned)std::min<int64_t>(w.ngrid, 16384);
+    if (rw == 2) hipLaunchKernelGGL(wide_medium_kernel<2>, dim3(nm), dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
+    else hipLaunchKernelGGL(wide_medium_kernel<4>, dim3(nm), dim3(kMergeBlock), 0, st, s, d, lk, w, checksum_out);
     MPSG_CHECK(hipGetLastError());
-    if (rw == 2) hipLaunchKernelGGL((wide_medium_kernel<2, kCBlock>), gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
-    else hipLaunchKernelGGL((wide_medium_kernel<4, kCBlock>), gm, dim3(kCBlock), 0, st, s, d, lk, w, checksum_out);
+    if (rw == 2) hipLaunchKernelGGL(wide_large_kernel<2>, gm, dim3(kCBlock), 0, st, s, d, lk, w, nm, checksum_out);
+    else hipLaunchKernelGGL(wide_large_kernel<4>, gm, dim3(kCBlock), 0, st, s, d, lk, w, nm, checksum_out);
     MPSG_CHECK(hipGetLastError());
     if (rw == 2) hipLaunchKernelGGL(wide_copy_kernel<2>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);
     else hipLaunchKernelGGL(wide_copy_kernel<4>, gc, dim3(kMergeBlock), 0, st, s, d, w, checksum_out);

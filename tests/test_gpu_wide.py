@@ -116,3 +116,14 @@ def test_in_place_and_overlapping():
         finally:
             lib.mpsort_gpu_dfree(d)
         assert numpy.array_equal(out, want)
+
+
+@pytest.mark.parametrize("per", [900, 1500, 3500])
+def test_groups_of_one_value(per):
+    """each key repeated about per times: most fine buckets hold one value and
+    stand alone, more of them than the grid of the groups' sorts has
+    workgroups, between groups of the values that share a boundary"""
+    n, P = N + 999, 7
+    g = numpy.random.default_rng(per)
+    v = g.integers(0, 2 ** 64, n // per, dtype=numpy.uint64)
+    check_parity(workloads.records16(v[g.integers(0, len(v), n)]), ragged(n, P, 8), ragged(n, P, 9), 'key', device=True)
