@@ -154,10 +154,13 @@ struct Buf {
 
 enum { kEvStart, kEvFirst, kEvFindP, kEvLayout, kEvExchange, kEvSecond, kEvEnd, kEvPhase };
 
+constexpr int kSideStreams = 3;  // with the main stream, the four hardware queues of a process
 struct DevCtx {
     bool init = false;
     int device = 0;
     hipStream_t st = nullptr;
+    hipStream_t side[kSideStreams] = {};  // independent parts of a batched plan (made when first needed)
+    hipEvent_t fork = nullptr, join[kSideStreams] = {};
     uint32_t epoch = 0;
     Buf din, dout;      // host staging
     Buf s0, s1, rbuf;   // sort-record buffers
@@ -2379,6 +2382,7 @@ struct SegTune {
 };
 static int form_waves_per_cu(int form) { return form == 2 ? 24 : 16; }
 
+constexpr int kSegEpoch = 12;  // counters before it are cleared in every run
 struct SegGroup {
     const void* in = nullptr;
     void* out = nullptr;
@@ -2403,7 +2407,7 @@ struct SegGroup {
     uint32_t* d_cnt = nullptr;
     int64_t* d_base = nullptr;
     uint32_t* d_hard = nullptr;
-    uint32_t* d_counters = nullptr;  // [0] oversized, [2] epoch, [4 + form] hard
+    uint32_t* d_counters = nullptr;  // [0] oversized, [4 + form] hard, [kSegEpoch] epoch
     int64_t* d_ovf = nullptr;
     SegSortPlan plan;
     uint64_t epoch_used = 0;  // epoch steps consumed since the last reset
@@ -2641,7 +2645,7 @@ static int seg_group_prepare(SegGroup& G, hipStream_t st) {
         p.d_checksum = nullptr;
         p.sparse = true;
         p.all_passes = true;
-        p.d_epoch_base = G.d_counters + 2;
+        p.d_epoch_base = G.d_counters + kSegEpoch;
     }
     MPSG_CHECK(hipStreamSynchronize(st));
     return 0;
@@ -2650,10 +2654,9 @@ static int seg_group_prepare(SegGroup& G, hipStream_t st) {
 // the device work of one group; records nothing but kernels, so it can be
 // captured (look-back epochs come from the counter bumped here)
 static int seg_group_enqueue_each(SegGroup& G, hipStream_t st);
-static int seg_group_enqueue(SegGroup& G, hipStream_t st) {
+static int seg_group_small(SegGroup& G, hipStream_t st) {
     int rc = 0;
-    if ((rc = launch_fill_u32(G.d_counters, 0u, 2, st))) return rc;
-    if ((rc = launch_fill_u32(G.d_counters + 4, 0u, kSegForms, st))) return rc;
+    if ((rc = launch_fill_u32(G.d_counters, 0u, kSegEpoch, st))) return rc;
     if (G.each) return seg_group_enqueue_each(G, st);
     int64_t at = 0;
     for (int form : {4, 3, 2, 1, 0}) {
@@ -2663,9 +2666,14 @@ static int seg_group_enqueue(SegGroup& G, hipStream_t st) {
             return rc;
         at += n;
     }
+    return 0;
+}
+static int seg_group_rest(SegGroup& G, hipStream_t st) {
+    int rc = 0;
+    if (G.each) return 0;
     if (G.nwide && (rc = launch_wide_segments(G.rw, G.in, G.tmp.p, G.out, G.lk, G.wide, st))) return rc;
     if (G.nlarge) {
-        if ((rc = launch_add_u32(G.d_counters + 2, (uint32_t)kMaxPasses, st))) return rc;
+        if ((rc = launch_add_u32(G.d_counters + kSegEpoch, (uint32_t)kMaxPasses, st))) return rc;
         if ((rc = seg_count(G.plan, G.in, nullptr, st)))
             return rc < 0 && !g_err[0] ? fail(MPSORT_ERR_UNSUPPORTED, "segmented sort: tile %d x %d not supported for "
                                               "%d-byte records", G.plan.tile.block, G.plan.tile.items, 4 * G.rw) : rc;
@@ -2675,6 +2683,81 @@ static int seg_group_enqueue(SegGroup& G, hipStream_t st) {
             return rc < 0 && !g_err[0] ? fail(MPSORT_ERR_UNSUPPORTED, "segmented sort: tile %d x %d not supported for "
                                               "%d-byte records", G.plan.tile.block, G.plan.tile.items, 4 * G.rw) : rc;
     }
+    return 0;
+}
+static int seg_group_enqueue(SegGroup& G, hipStream_t st) {
+    const int rc = seg_group_small(G, st);
+    return rc ? rc : seg_group_rest(G, st);
+}
+
+// The groups of a plan write nothing that another group reads or writes, and
+// a group's buffers are the same or apart: their parts may run side by side.
+static bool seg_groups_apart(const std::vector<SegGroup*>& groups) {
+    struct Range {
+        const char *a, *b;
+    };
+    auto meet = [](const Range& x, const Range& y) { return x.a < y.b && y.a < x.b; };
+    auto range = [](const void* p, const SegGroup* G) {
+        return Range{(const char*)p, (const char*)p + (size_t)G->nrec * G->elsize};
+    };
+    for (size_t i = 0; i < groups.size(); i++) {
+        const SegGroup* G = groups[i];
+        const Range in = range(G->in, G), out = range(G->out, G);
+        if (G->each || (G->in != G->out && meet(in, out))) return false;
+        for (size_t k = 0; k < i; k++) {
+            const SegGroup* H = groups[k];
+            const Range hin = range(H->in, H), hout = range(H->out, H);
+            if (meet(out, hin) || meet(out, hout) || meet(in, hout)) return false;
+        }
+    }
+    return true;
+}
+static int side_streams(DevCtx& c) {
+    if (c.fork) return 0;
+    for (int i = 0; i < kSideStreams; i++) {
+        if (!c.side[i]) MPSG_CHECK(hipStreamCreateWithFlags(&c.side[i], hipStreamNonBlocking));
+        if (!c.join[i]) MPSG_CHECK(hipEventCreateWithFlags(&c.join[i], hipEventDisableTiming));
+    }
+    MPSG_CHECK(hipEventCreateWithFlags(&c.fork, hipEventDisableTiming));
+    return 0;
+}
+// All groups of a plan: the in-LDS segments and the larger ones of every group
+// are chains of short launches that leave most of the chip idle, so they go
+// to streams of their own, forked from st and joined to it again.  A plan
+// with one chain, or whose buffers meet, stays on st.
+static int seg_plan_enqueue(DevCtx& c, const std::vector<SegGroup*>& groups, hipStream_t st) {
+    struct Part {
+        SegGroup* G;
+        bool small;
+    };
+    std::vector<Part> parts;
+    for (SegGroup* G : groups) {
+        if (G->nwide || G->nlarge) parts.push_back(Part{G, false});
+        if (G->nsmall) parts.push_back(Part{G, true});
+    }
+    int rc = 0;
+    if (parts.size() < 2 || !seg_groups_apart(groups)) {
+        for (SegGroup* G : groups)
+            if ((rc = seg_group_enqueue(*G, st))) return rc;
+        return 0;
+    }
+    const int used = (int)std::min<size_t>(kSideStreams, parts.size() - 1);
+    MPSG_CHECK(hipEventRecord(c.fork, st));
+    int forked = 0;
+    hipError_t e = hipSuccess;
+    for (; forked < used && e == hipSuccess; forked++) e = hipStreamWaitEvent(c.side[forked], c.fork, 0);
+    for (size_t i = 0; i < parts.size() && e == hipSuccess && !rc; i++) {
+        hipStream_t s = i % (used + 1) == 0 ? st : c.side[i % (used + 1) - 1];
+        rc = parts[i].small ? seg_group_small(*parts[i].G, s) : seg_group_rest(*parts[i].G, s);
+    }
+    // joined also after an error, so that a capture can end
+    for (int i = 0; i < forked; i++) {
+        const hipError_t a = hipEventRecord(c.join[i], c.side[i]);
+        const hipError_t b = a == hipSuccess ? hipStreamWaitEvent(st, c.join[i], 0) : a;
+        if (e == hipSuccess) e = b;
+    }
+    if (rc) return rc;
+    MPSG_CHECK(e);
     return 0;
 }
 
@@ -2694,7 +2777,7 @@ static int seg_group_enqueue_each(SegGroup& G, hipStream_t st) {
     }
     const int npass = G.ks.key_bytes;
     for (int i = 0; i < G.nlarge; i++) {
-        if ((rc = launch_add_u32(G.d_counters + 2, (uint32_t)kMaxPasses, st))) return rc;
+        if ((rc = launch_add_u32(G.d_counters + kSegEpoch, (uint32_t)kMaxPasses, st))) return rc;
         SegSortPlan v = G.plan;
         v.nseg = 1;
         v.nrec = G.lcount[i];
@@ -2724,7 +2807,7 @@ static int seg_group_epoch_guard(SegGroup& G, hipStream_t st) {
     }
     int rc = launch_fill_u32((uint32_t*)G.lookback.p, 0u, (int64_t)(G.lookback.bytes / 4), st);
     if (rc) return rc;
-    if ((rc = launch_fill_u32(G.d_counters + 2, 0u, 1, st))) return rc;
+    if ((rc = launch_fill_u32(G.d_counters + kSegEpoch, 0u, 1, st))) return rc;
     G.epoch_used = step;
     return 0;
 }
@@ -3834,6 +3917,7 @@ int mpsort_gpu_segplan_run(mpsort_gpu_segplan* p, mpsort_gpu_stats* stats) {
     if (c->device != p->device) return fail(MPSORT_ERR_ARG, "the plan belongs to device %d", p->device);
     hipStream_t st = c->st;
     if (!p->prepared) {
+        if ((rc = side_streams(*c))) return rc;
         for (SegGroup* G : p->groups) {
             if (p->flags & MPSORT_GPU_SEGPLAN_TUNE) rc = seg_group_tune(*G, *c);
             else rc = seg_group_prepare(*G, st);
@@ -3847,21 +3931,18 @@ int mpsort_gpu_segplan_run(mpsort_gpu_segplan* p, mpsort_gpu_stats* stats) {
     if (p->flags & MPSORT_GPU_SEGPLAN_GRAPH) {
         if (!p->exec) {
             MPSG_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-            for (SegGroup* G : p->groups) {
-                if ((rc = seg_group_enqueue(*G, st))) {
-                    hipGraph_t g = nullptr;
-                    (void)hipStreamEndCapture(st, &g);
-                    if (g) (void)hipGraphDestroy(g);
-                    return rc;
-                }
+            if ((rc = seg_plan_enqueue(*c, p->groups, st))) {
+                hipGraph_t g = nullptr;
+                (void)hipStreamEndCapture(st, &g);
+                if (g) (void)hipGraphDestroy(g);
+                return rc;
             }
             MPSG_CHECK(hipStreamEndCapture(st, &p->graph));
             MPSG_CHECK(hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0));
         }
         MPSG_CHECK(hipGraphLaunch(p->exec, st));
-    } else {
-        for (SegGroup* G : p->groups)
-            if ((rc = seg_group_enqueue(*G, st))) return rc;
+    } else if ((rc = seg_plan_enqueue(*c, p->groups, st))) {
+        return rc;
     }
     MPSG_CHECK(hipEventRecord(c->ev[kEvEnd], st));
     for (SegGroup* G : p->groups)

@@ -60,3 +60,28 @@ def test_the_sample_misses_the_weight(dtype):
         plan.close()
         lib.mpsort_gpu_dfree(d)
         lib.mpsort_gpu_dfree(o)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_groups_that_depend_on_each_other(graph):
+    """the second group reads what the first wrote: the parts of a plan run
+    side by side only where their buffers are apart"""
+    dtype = workloads.REC16I
+    sizes = numpy.array([300, 20000, 5, 1000, 60001], numpy.int64)
+    n = int(sizes.sum())
+    a = make(dtype, sizes, 77, key_bits=16)
+    d = [lib.mpsort_gpu_dmalloc(a.nbytes) for _ in range(3)]
+    plan = segments.SegmentPlan(graph=graph)
+    try:
+        _lib.check(lib.mpsort_gpu_memcpy_h2d(d[0], a.ctypes.data, a.nbytes))
+        plan.add(d[0], d[1], sizes, dtype, 'key')
+        plan.add(d[1], d[2], numpy.array([n], numpy.int64), dtype, 'key')
+        for _ in range(3):
+            plan.run()
+            g = numpy.empty_like(a)
+            _lib.check(lib.mpsort_gpu_memcpy_d2h(g.ctypes.data, d[2], a.nbytes))
+            assert numpy.array_equal(g, expected(a, [n]))
+    finally:
+        plan.close()
+        for p in d:
+            lib.mpsort_gpu_dfree(p)
