@@ -1830,6 +1830,19 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
                                       (uint32_t)kChunkCap, small_form, c.ev[kEvFirst])) ||
         (rc = mark(4)))
         return rc;
+    // The buckets above 4608 records (lists[2]) and the crowded ones: enqueued
+    // with the rest where some are likely.  A bucket's size is estimated from
+    // 16 sample keys (a deviation of a quarter): at 2500 records on average
+    // one bucket in a thousand is above, at 3900 one in five.  Waiting for
+    // their number and counting a second time took 40 us of 289 (4,000,000 x
+    // 16 B); where none are listed the two launches take 8.
+    const bool ahead = n > (int64_t)kLBins * 2500;
+    auto listed = [&](uint32_t most, const uint32_t* d_n) -> int {
+        int r2 = launch_listed_sort(rw, tmp, dst, lk, w.medium, most, w.tot, w.base, w.tables, kLBins, 0, w.hard,
+                                    w.lists + 1, cs_out, st, nullptr, d_n);
+        return r2 ? r2 : launch_lsd_sort(rw, tmp, dst, lk, w.tot, w.base, w.hard, w.lists + 1, sh.W, cs_out, st);
+    };
+    if (ahead && (rc = listed((uint32_t)sh.W, w.lists + 2))) return rc;
     auto finish = [&]() -> int {
         int r2 = 0;
         if (cs.general &&
@@ -1843,13 +1856,10 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     if ((rc = finish())) return rc;
     DirectResult got = *res;
     if (got.scatter_err) return fail(MPSORT_ERR_TIMEOUT, "bucket scatter: device flag 0x%x", got.scatter_err);
-    if (got.lists[0] | got.lists[1] | got.lists[2]) {
+    if (got.lists[0] || (!ahead && (got.lists[1] | got.lists[2]))) {
         // buckets above the workgroup's capacity, then the crowded ones, then
         // those above the in-LDS capacity; the counts again afterwards
-        if ((rc = launch_listed_sort(rw, tmp, dst, lk, w.medium, got.lists[2], w.tot, w.base, w.tables, kLBins, 0,
-                                     w.hard, w.lists + 1, cs_out, st)) ||
-            (rc = launch_lsd_sort(rw, tmp, dst, lk, w.tot, w.base, w.hard, w.lists + 1, sh.W, cs_out, st)))
-            return rc;
+        if (!ahead && (rc = listed(got.lists[2], nullptr))) return rc;
         if (got.lists[0]) {
             SegSortPlan plain;
             plain.rw = rw;

@@ -160,11 +160,12 @@ int launch_merge_bucket(int rw, bool big, const void* recs, void* dst, const LKe
                         long long* checksum, hipStream_t st, uint32_t ovf_cap = (uint32_t)kChunkCap);
 // in-LDS sort (1024-thread form) of the nlist listed buckets, src -> dst at
 // the same slots (src may equal dst); nbins buckets per segment, segment s
-// uses tables + s * tstride; crowded ones are appended to hard
+// uses tables + s * tstride; crowded ones are appended to hard.  d_nlist: the
+// number listed, on the device (at most nlist)
 int launch_listed_sort(int rw, const void* src, void* dst, const LKey& lk, const uint32_t* list, uint32_t nlist,
                        const uint32_t* hist, const int64_t* bucket_base, const uint64_t* tables, int nbins,
                        int64_t tstride, uint32_t* hard, uint32_t* nhard, long long* checksum, hipStream_t st,
-                       const EntryOut* eo = nullptr);
+                       const EntryOut* eo = nullptr, const uint32_t* d_nlist = nullptr);
 // launch_chunk_sort with 512-thread workgroups: two per CU, or with small
 // three (buckets up to kMergeCap records); larger buckets (up to kChunkCap)
 // are listed in medium (*nmedium entries) for launch_listed_sort; no LDS

@@ -1227,8 +1227,9 @@ __global__ __launch_bounds__(kCBlock) void listed_sort_kernel(
     const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, LKey lk, const uint32_t* __restrict__ list,
     const uint32_t* __restrict__ hist, const int64_t* __restrict__ bucket_base, const uint64_t* __restrict__ tables,
     int nbins, int64_t tstride, uint32_t* __restrict__ hard, uint32_t* __restrict__ nhard,
-    long long* __restrict__ checksum_out, EntryOut eo) {
+    long long* __restrict__ checksum_out, EntryOut eo, const uint32_t* __restrict__ nlist) {
     __shared__ uint32_t s_bins[BSort<kCBlock>::BW];
+    if (nlist && blockIdx.x >= *nlist) return;
     const uint32_t b = list[blockIdx.x];
     const uint32_t cnt32 = hist[b];
     const int64_t base = bucket_base[b];
@@ -2551,14 +2552,14 @@ int launch_merge_bucket(int rw, bool big, const void* recs, void* dst, const LKe
 int launch_listed_sort(int rw, const void* src, void* dst, const LKey& lk, const uint32_t* list, uint32_t nlist,
                        const uint32_t* hist, const int64_t* bucket_base, const uint64_t* tables, int nbins,
                        int64_t tstride, uint32_t* hard, uint32_t* nhard, long long* checksum, hipStream_t st,
-                       const EntryOut* eop) {
+                       const EntryOut* eop, const uint32_t* d_nlist) {
     if (nlist == 0) return 0;
     const EntryOut eo = eop ? *eop : EntryOut{};
     const uint32_t* s = (const uint32_t*)src;
     uint32_t* d = (uint32_t*)dst;
     switch (rw) {
-        case 2: hipLaunchKernelGGL(listed_sort_kernel<2>, dim3(nlist), dim3(kCBlock), 0, st, s, d, lk, list, hist, bucket_base, tables, nbins, tstride, hard, nhard, checksum, eo); break;
-        case 4: hipLaunchKernelGGL(listed_sort_kernel<4>, dim3(nlist), dim3(kCBlock), 0, st, s, d, lk, list, hist, bucket_base, tables, nbins, tstride, hard, nhard, checksum, eo); break;
+        case 2: hipLaunchKernelGGL(listed_sort_kernel<2>, dim3(nlist), dim3(kCBlock), 0, st, s, d, lk, list, hist, bucket_base, tables, nbins, tstride, hard, nhard, checksum, eo, d_nlist); break;
+        case 4: hipLaunchKernelGGL(listed_sort_kernel<4>, dim3(nlist), dim3(kCBlock), 0, st, s, d, lk, list, hist, bucket_base, tables, nbins, tstride, hard, nhard, checksum, eo, d_nlist); break;
         default: return -1;
     }
     MPSG_CHECK(hipGetLastError());
