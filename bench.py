@@ -464,6 +464,12 @@ def _device_copy(recs):
 PLAIN_LEVELS = ("sample", "level1", "level2", "bucket_sort")
 
 
+def learned_stages(st):
+    """names of a learned call's pass_ms: two partition levels, or the per-rank
+    form's kernels"""
+    return list(PLAIN_LEVELS) if len(st["pass_ms"]) == len(PLAIN_LEVELS) else LEARNED_KERNELS
+
+
 def plain_first_form(st):
     """(FirstSort form, entries of pass_ms before the SecondSort's) of a
     plain-path call's statistics"""
@@ -646,7 +652,7 @@ def bench_histsort(args):
             "buckets_lds_radix": L["buckets_lds_radix"],
             "buckets_listed": L["buckets_listed"],
             "phases_ms": {k2: round(L[k2], 4) for k2 in PHASES},
-            "kernels_ms": dict(zip(LEARNED_KERNELS, [round(x, 4) for x in L["pass_ms"]]))}
+            "kernels_ms": dict(zip(learned_stages(L), [round(x, 4) for x in L["pass_ms"]]))}
         log("learned phases: " + json.dumps(result_learned["phases_ms"]))
         log("learned kernels: " + json.dumps(result_learned["kernels_ms"]))
         model.close()
@@ -706,18 +712,24 @@ def bench_histsort(args):
                           "one launch per step over all n records: 2*n*16 B per launch)", TRAFFIC_PLAIN_BUCKET_SORT,
                           ROCPROF_MS.get("plain_bucket_sort"))
     if result_learned is not None:
-        ib = LEARNED_KERNELS.index
-        # the step's largest kernel: the FirstSort's in-LDS bucket sort, one
-        # launch per step over all n records (the merged SecondSort splits
-        # its records over two smaller kernels, merge_B in kernels_ms)
-        roofline = roof([st["pass_ms"][ib("bucket_sort_A")] for st in st_learned],
-                        "interp_sort_kernel<4,512,9> (FirstSort in-LDS bucket sort, one launch per step over all n "
-                        "records: 2*n*16 B per launch)", TRAFFIC_BUCKET_SORT, ROCPROF_MS.get("bucket_sort_A"))
+        names = learned_stages(st_learned[-1])
+        ib = names.index
+        # the step's largest kernel: the in-LDS sorts (per-rank form: the
+        # FirstSort's bucket sort, one launch per step over all n records)
+        if names[0] == PLAIN_LEVELS[0]:
+            roofline = roof([st["pass_ms"][ib("bucket_sort")] for st in st_learned],
+                            "wide_sort_kernel<4> (groups of fine buckets gathered and sorted in LDS, one launch per step "
+                            "over all n records, with the listed groups' launches: 2*n*16 B)", None, None)
+        else:
+            roofline = roof([st["pass_ms"][ib("bucket_sort_A")] for st in st_learned],
+                            "interp_sort_kernel<4,512,9> (FirstSort in-LDS bucket sort, one launch per step over all n "
+                            "records: 2*n*16 B per launch)", TRAFFIC_BUCKET_SORT, ROCPROF_MS.get("bucket_sort_A"))
         result_learned["roofline_by_stage"] = {
             k: {"avg_ms": round(sum(st["pass_ms"][ib(k)] for st in st_learned) / len(st_learned), 4),
                 "GB/s": round((alg_bytes / 2 if k.startswith("hist") else alg_bytes) /
                               (sum(st["pass_ms"][ib(k)] for st in st_learned) / len(st_learned) * 1e-3) / 1e9, 1)}
-            for k in ("hist_A", "scatter_A", "bucket_sort_A", "merge_B")}
+            for k in ("hist_A", "scatter_A", "bucket_sort_A", "merge_B", "level1", "level2", "bucket_sort")
+            if k in names}
     else:
         roofline = plain_roof
     log("plain phases (ms): first %.3f findP %.3f lay %.3f exch %.3f second %.3f total %.3f; passes %d+%d, "
@@ -862,7 +874,7 @@ def bench_dists(args):
                      "buckets_lds_radix": L["buckets_lds_radix"],
                      "buckets_listed": L["buckets_listed"],
                      "phases_ms": {k2: round(L[k2], 4) for k2 in PHASES},
-                     "kernels_ms": dict(zip(LEARNED_KERNELS, [round(x, 4) for x in L["pass_ms"]])),
+                     "kernels_ms": dict(zip(learned_stages(L), [round(x, 4) for x in L["pass_ms"]])),
                      "plain_stages_ms": plain_stages(st_p[-1]),
                      "plain_buckets_overflow": st_p[-1]["buckets_overflow"],
                      "plain_buckets_lds_radix": st_p[-1]["buckets_lds_radix"]}

@@ -1901,10 +1901,13 @@ static bool wide_eligible(const CallShape& cs) {
     return direct_asked(cs) && (cs.rw == 2 || cs.rw == 4) && cs.ntot > kDirectMaxRecords &&
            cs.ntot <= kWideMaxRecords;
 }
-// *again: nothing was written, the call takes the general path (the sample
-// missed the sizes of the coarse buckets by far)
+// M: the learned path; the coarse boundaries are the model's quantiles, and
+// its splitters are compared with those read off the result.
+// *again: nothing was written, the call takes another path (the sample, or the
+// model, missed the sizes of the coarse buckets by far)
 static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
-                    const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats, bool* again) {
+                    const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats, bool* again,
+                    const LearnedModel* M = nullptr) {
     hipStream_t st = c.st;
     const int P = cs.P, rw = cs.rw;
     const int64_t n = cs.ntot;
@@ -1914,7 +1917,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     DirectShape sh;
     direct_shape(cs, nin, nout, kWideTile, &sh);
     sh.W = (int)std::min<int64_t>(kWideBuckets, std::max<int64_t>(2, (n + kWideCoarse - 1) / kWideCoarse));
-    sh.S = std::min(kDirectMaxChunks, (32 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
+    sh.S = M ? kDirectChunk : std::min(kDirectMaxChunks, (32 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
 
     // ---- workspace
     DirectWork d;
@@ -1933,6 +1936,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     w.ngrid = wide_grid(n, w.W);
     w.ncopy = n / kWideCopy + w.nfine;
     w.max_overflow = (int)(n / kChunkCap + 1);
+    uint64_t* prop = nullptr;
     auto lay = [&](auto& a, auto take) {
         take(a, d.begin, (size_t)P);
         take(a, d.count, (size_t)P);
@@ -1963,6 +1967,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         take(a, w.copy, (size_t)w.ncopy);
         take(a, w.overflow, (size_t)2 * w.max_overflow);
         take(a, w.tally, (size_t)2 * kDirectMaxP * kDirectMaxP);
+        take(a, prop, (size_t)kDirectMaxP);
     };
     Sizer lz;
     lay(lz, [](Sizer& a, auto*& p, size_t k) { a.take<std::remove_reference_t<decltype(*p)>>(k); });
@@ -2001,8 +2006,17 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     const SegDev sd{d.begin, d.count, d.tile_start, P, 0};
     if ((rc = mark(0)) ||
         (rc = launch_direct_sample(rw, src, lk, sh, d, !(cs.general && !packed_host),
-                                   cs.general ? nullptr : c.ev[kEvStart], st)) ||
-        (rc = mark(1)) || (rc = launch_wide_level1(rw, src, a, lk, sd, w, cs_in, st)) || (rc = mark(2)) ||
+                                   cs.general ? nullptr : c.ev[kEvStart], st)))
+        return rc;
+    if (M) {
+        const ModelDev md = M->dev();
+        d.prop = prop;
+        if ((rc = launch_model_tables(md, M->kmax, nullptr, nullptr, 1, sh.W - 1, d.raw, M->heavy, M->heavy_q, M->nheavy,
+                                      st)) ||
+            (rc = launch_model_proposals(md, d.C, n, P, prop, st)))
+            return rc;
+    }
+    if ((rc = mark(1)) || (rc = launch_wide_level1(rw, src, a, lk, sd, w, cs_in, st)) || (rc = mark(2)) ||
         (rc = launch_wide_level2(rw, a, b, dst, lk, w, cs_out, st)) || (rc = mark(3)) ||
         (rc = launch_wide_sort(rw, b, dst, lk, w, cs_out, st)) || (rc = mark(4)))
         return rc;
@@ -2059,9 +2073,25 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         for (int i = 0; i < 4; i++) stats->pass_ms[i] = ev_ms(pe[i], pe[i + 1]);
         stats->npass_ms = 4;
     }
+    if (M) {
+        stats->learned = 1;
+        stats->splitters_exact = P > 1 ? (int32_t)got.exact : 0;
+        stats->splitters_repaired = P > 1 ? P - 1 - stats->splitters_exact : 0;
+        // one round where every proposal holds, else the result is read too
+        stats->bisect_rounds = stats->repair_rounds = P > 1 ? (stats->splitters_repaired ? 2 : 1) : 0;
+    }
     return direct_results(c, cs, d, got, packed_host != nullptr, stats);
 }
 
+// The learned path by two partition levels: per-rank bucket sorts, bounds and
+// a merge took 3.47 ms on 2^26 x 16 B, 64 ranks, the two levels 2.32.  Below one
+// level's sizes, and where a receiver's kMergeBins buckets are above the
+// in-LDS capacity on average, the per-rank form stays: its counters of
+// oversized buckets (buckets_overflow, plain_sides) are how a caller learns
+// that a model does not fit the sizes or the keys.
+static bool learned_wide_eligible(const CallShape& cs) {
+    return wide_eligible(cs) && (cs.P == 1 || cs.ntot <= (int64_t)cs.P * kMergeBins * kChunkCap);
+}
 static int run_histsort_learned(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out,
                                 const int64_t* nin, const int64_t* nout, const LearnedModel& M,
                                 mpsort_gpu_stats* stats) {
@@ -3851,6 +3881,11 @@ int mpsort_gpu_newarray_learned(const void* base, const int64_t* nin, int P, voi
     memset(&st, 0, sizeof st);
     remember_key(*c, key, 0, 0);
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
+        if (learned_wide_eligible(cs)) {
+            bool again = false;
+            const int r2 = run_wide(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again, &model->m);
+            if (r2 || !again) return r2;
+        }
         return run_histsort_learned(*c, cs, d_in, d_out, nin, nout, model->m, &st);
     });
     g_last = st;

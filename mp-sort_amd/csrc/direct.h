@@ -49,6 +49,7 @@ struct DirectWork {
     int64_t *myclt, *mycle, *myC, *send;
     uint64_t* cross;      // kDirectMaxP^2: CLE << 32 | CLT by splitter and rank, for the layout
     uint64_t *split, *pminmax;
+    const uint64_t* prop;     // a model's proposals for the splitters (may be null)
     unsigned long long* acc;  // 4, zero between calls: a small sort's blocks done and sums
 };
 
@@ -58,6 +59,7 @@ struct DirectResult {
     uint32_t lists[4];    // [3]: digit passes of the one-workgroup sort
     long long sums[2];
     uint32_t buckets;     // fine buckets of the two-level form
+    uint32_t exact;       // splitters that the model proposed
 };
 
 // start / stop (here and below, may be null): events of the launch itself

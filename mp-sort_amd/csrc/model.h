@@ -51,6 +51,7 @@ constexpr int kMaxHeavy = 16384;
 int launch_model_tables(const ModelDev& m, uint64_t kmax, const float* q0, const float* q1, int ntables,
                         int nb, uint64_t* tables, const uint64_t* heavy, const float2* heavy_q, int nheavy,
                         hipStream_t st, const int* nedge = nullptr, bool ordered = false);
+int launch_model_proposals(const ModelDev& m, const int64_t* C, int64_t n, int P, uint64_t* prop, hipStream_t st);
 // per segment of unsorted records: the quantile range of its keys and its
 // edge boundaries (see model_tables_kernel)
 int launch_seg_range(const ModelDev& m, const void* recs, int64_t elsize, int64_t key_off, int key_bytes,

@@ -347,7 +347,7 @@ __global__ void leaf_xstart_kernel(ModelDev m, float* __restrict__ xstart) {
 // Boundary tables: table t has nb boundaries for quantile targets
 // q = q0[t] + (q1[t] - q0[t]) * (i + 1) / (nb + 1).  With nedge[t] = E > 0
 // the first E targets split [0, q0) evenly, the last E split (q1, 1], and
-// the nb - 2E between them split [q0, q1]: a table for a segment whose keys
+// the nb - 2E between them split [q0, q1] (null: [0, 1]): a table for a segment whose keys
 // mostly lie in one part of the distribution that still spreads the few
 // keys outside it.  Tables are made non-decreasing afterwards.  One thread
 // per boundary.
@@ -359,7 +359,7 @@ __global__ void model_tables_kernel(ModelDev m, const float* __restrict__ q0, co
     if (g >= (int64_t)ntables * nb) return;
     const int t = (int)(g / nb), i = (int)(g % nb);
     const int E = nedge ? nedge[t] : 0;
-    const float a = q0[t], b = q1[t];
+    const float a = q0 ? q0[t] : 0.f, b = q1 ? q1[t] : 1.f;
     float q;
     if (E > 0 && i < E) {
         q = a * (float)(i + 1) / (float)(E + 1);
@@ -707,6 +707,22 @@ int launch_model_tables(const ModelDev& m, uint64_t kmax, const float* q0, const
         hipLaunchKernelGGL(tables_order_kernel, dim3(ntables - 1), dim3(256), 0, st, tables, ntables, nb);
         MPSG_CHECK(hipGetLastError());
     }
+    return 0;
+}
+
+// the model's proposal for every splitter (the value the learned search tests
+// first), 0 where C is 0
+__global__ __launch_bounds__(64) void model_proposals_kernel(ModelDev m, const int64_t* __restrict__ C, int64_t n,
+                                                             int P, uint64_t* __restrict__ prop) {
+    const int i = threadIdx.x;
+    if (i >= P - 1) return;
+    const int64_t Ci = C[i + 1];
+    prop[i] = Ci > 0 ? model_inverse_leaves(m, (float)(((double)Ci - 0.5) / (double)n)) : 0;
+}
+int launch_model_proposals(const ModelDev& m, const int64_t* C, int64_t n, int P, uint64_t* prop, hipStream_t st) {
+    if (P > 64) return -1;
+    hipLaunchKernelGGL(model_proposals_kernel, dim3(1), dim3(64), 0, st, m, C, n, P, prop);
+    MPSG_CHECK(hipGetLastError());
     return 0;
 }
 

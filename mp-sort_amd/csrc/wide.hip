@@ -668,6 +668,7 @@ __global__ __launch_bounds__(1024) void wide_counts_kernel(const uint32_t* __res
     const int j = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int P1 = P + 1;
     if (tid == 0) s_err = 0;
+    bool hit = false;
     if (P > 1 && !w.lists[5]) {
         if (tid < kWideBuckets) s_tab[tid] = w.tables[tid];
         uint32_t mine = 0;
@@ -683,6 +684,7 @@ __global__ __launch_bounds__(1024) void wide_counts_kernel(const uint32_t* __res
             uint32_t r[RW];
             RecIO<RW>::load(out, Ci > 0 ? Ci - 1 : 0, r);
             const uint64_t v = lkey<RW>(r, lk);
+            hit = d.prop && Ci > 0 && d.prop[tid] == v;
             int b = 0;
             for (int step = kWideBuckets / 2; step > 0; step >>= 1) b += s_tab[b + step - 1] < v ? step : 0;
             b = min(b, w.W - 1);
@@ -730,6 +732,8 @@ __global__ __launch_bounds__(1024) void wide_counts_kernel(const uint32_t* __res
         return;
     }
     __syncthreads();
+    const uint64_t hits = __ballot(hit);  // splitters belong to the first wave
+    if (tid == 0) res->exact = (uint32_t)__popcll(hits);
     if (tid < 3) res->lists[tid] = w.lists[tid];
     if (tid == 3) res->lists[3] = w.lists[5];
     if (tid < 2) res->sums[tid] = d.checksum[tid];

@@ -293,3 +293,34 @@ def test_merged_secondsort_with_thousands_of_oversized_buckets():
     assert st.plain_sides >= 1
     assert numpy.array_equal(out, ref)
     assert st.checksum_in == st.checksum_out
+
+
+@pytest.mark.parametrize("P", [1, 5, 64])
+@pytest.mark.parametrize("dist", ["clustered", "zipf", "nearly_sorted", "mismatch"])
+def test_learned_above_one_partition_level(dist, P):
+    """sizes sorted by two partition levels whose coarse boundaries are the
+    model's: output and counts equal the plain path's; a model of keys below
+    2^40 on keys of 64 bits leaves one coarse bucket, and the sort takes the
+    per-rank form"""
+    n = 1024 * 4200 + 4321
+    note("learned levels dist=%s P=%d" % (dist, P))
+    if dist == "mismatch":
+        t = workloads.records16(workloads.uniform(1 << 18, 3) >> numpy.uint64(24))
+        ts, _ = gpu_sort(t, [1 << 18], [1 << 18], 'key')
+        model = learned.train(ts, 'key', nsample=1 << 14, seed=7)
+        a = workloads.records16(keys_of("uniform", n, 5))
+    else:
+        model = trained(dist, n)
+        a = workloads.records16(keys_of(dist, n, 5))
+    ref, _ = gpu_sort(a, even(n, P), even(n, P), 'key')
+    ref_counts = last_counts(P, 8) if P > 1 else None
+    out = learned.sort_learned(a, model, 'key', nin=even(n, P))
+    assert numpy.array_equal(out, ref)
+    s = _lib.last_stats()
+    assert s.learned == 1 and s.checksum_in == s.checksum_out
+    assert s.splitters_exact + s.splitters_repaired == P - 1
+    if P > 1:
+        c = last_counts(P, 8)
+        for k in ("C", "P", "myCLT", "myCLE", "myC", "send"):
+            assert numpy.array_equal(c[k], ref_counts[k]), k
+    model.close()
