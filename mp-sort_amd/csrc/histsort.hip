@@ -976,6 +976,95 @@ int launch_exchange_hist(const void* src, void* dst, int64_t ntot, int rw, const
     return 0;
 }
 
+// Pack and gather of 32-byte records at 16-byte addresses with 16-byte sort
+// records: four records of a thread in flight, and at most 2048 blocks, each
+// of which adds to the checksum once.  8192 blocks of one record at a time took
+// 177 and 262 us at 12,000,017 records, these take 111 and 187 (5.2 and 4.6
+// TB/s with the index reads): bound by HBM, the gather by its
+// scattered 32-byte reads.
+constexpr int kRec32Unroll = 4;
+__device__ __forceinline__ void block_sum_add(long long csum, long long* s_sum, long long* __restrict__ checksum) {
+    csum = wave_sum_ll(csum);
+    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = csum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        long long a = 0;
+        for (int q = 0; q < kWaves; q++) a += s_sum[q];
+        atomicAdd((unsigned long long*)checksum, (unsigned long long)a);
+    }
+}
+__device__ __forceinline__ int sbyte_sum4(const uint4& x) {
+    return sbyte_sum(x.x) + sbyte_sum(x.y) + sbyte_sum(x.z) + sbyte_sum(x.w);
+}
+__global__ __launch_bounds__(kBlock) void pack32_kernel(const uint4* __restrict__ in, int64_t n, int kw0, int kwords,
+                                                        uint4* __restrict__ out, int iwords,
+                                                        long long* __restrict__ checksum) {
+    constexpr int U = kRec32Unroll;
+    __shared__ long long s_sum[kWaves];
+    long long csum = 0;
+    for (int64_t i0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x; i0 < n; i0 += (int64_t)gridDim.x * kBlock * U) {
+        uint4 a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t i = min(i0 + u * kBlock, n - 1);
+            a[u] = in[2 * i];
+            b[u] = in[2 * i + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t i = i0 + u * kBlock;
+            if (i >= n) break;
+            csum += sbyte_sum4(a[u]) + sbyte_sum4(b[u]);
+            const uint32_t r[8] = {a[u].x, a[u].y, a[u].z, a[u].w, b[u].x, b[u].y, b[u].z, b[u].w};
+            const uint32_t k0 = pick_word<8>(r, kw0), k1 = kwords > 1 ? pick_word<8>(r, kw0 + 1) : 0u;
+            out[i] = make_uint4(k0, k1, iwords == 2 ? (uint32_t)i : 0u,
+                                iwords == 2 ? (uint32_t)((uint64_t)i >> 32) : (uint32_t)i);
+        }
+    }
+    if (checksum) block_sum_add(csum, s_sum, checksum);
+}
+__global__ __launch_bounds__(kBlock) void gather32_kernel(const uint4* __restrict__ in, int64_t n,
+                                                          const uint2* __restrict__ srec, int iwords,
+                                                          uint4* __restrict__ out, long long* __restrict__ checksum,
+                                                          uint32_t* __restrict__ error_flag) {
+    constexpr int U = kRec32Unroll;
+    __shared__ long long s_sum[kWaves];
+    long long csum = 0;
+    for (int64_t o0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x; o0 < n; o0 += (int64_t)gridDim.x * kBlock * U) {
+        int64_t at[U];
+        uint4 a[U], b[U];
+        bool bad = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint2 x = srec[2 * min(o0 + u * kBlock, n - 1) + 1];
+            at[u] = iwords == 2 ? (int64_t)(((uint64_t)x.y << 32) | x.x) : (int64_t)x.y;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (at[u] < 0 || at[u] >= n) {  // only reachable with corrupted sort records
+                bad = true;
+                at[u] = -1;
+            }
+            const int64_t i = at[u] < 0 ? 0 : at[u];
+            a[u] = in[2 * i];
+            b[u] = in[2 * i + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int64_t o = o0 + u * kBlock;
+            if (o >= n || at[u] < 0) continue;
+            out[2 * o] = a[u];
+            out[2 * o + 1] = b[u];
+            csum += sbyte_sum4(a[u]) + sbyte_sum4(b[u]);
+        }
+        if (bad && error_flag) atomicOr(error_flag, 64u);
+    }
+    if (checksum) block_sum_add(csum, s_sum, checksum);
+}
+static unsigned rec32_blocks(int64_t n) {
+    return (unsigned)std::min<int64_t>((n + kBlock * kRec32Unroll - 1) / (kBlock * kRec32Unroll), 2048);
+}
+
 int launch_pack(const void* in, int64_t n, int64_t elsize, int64_t key_off, int key_bytes,
                 void* out, int rw, int iwords, long long* checksum, hipStream_t st) {
     if (n <= 0) return 0;
@@ -983,6 +1072,12 @@ int launch_pack(const void* in, int64_t n, int64_t elsize, int64_t key_off, int 
     if (blocks > 8192) blocks = 8192;
     const int vec = (elsize % 16 == 0 && (uintptr_t)in % 16 == 0) ? 1 : 0;
     const int kwords = (key_off % 4 == 0 && key_bytes % 4 == 0 && elsize % 4 == 0 && (uintptr_t)in % 4 == 0) ? 1 : 0;
+    if (elsize == 32 && vec && kwords && rw == 4 && key_bytes <= 8) {
+        hipLaunchKernelGGL(pack32_kernel, dim3(rec32_blocks(n)), dim3(kBlock), 0, st, (const uint4*)in, n,
+                           (int)(key_off >> 2), key_bytes >> 2, (uint4*)out, iwords, checksum);
+        MPSG_CHECK(hipGetLastError());
+        return 0;
+    }
     hipLaunchKernelGGL(pack_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, (const uint8_t*)in,
                        n, elsize, key_off, key_bytes, (uint32_t*)out, rw, iwords, checksum, vec, kwords);
     MPSG_CHECK(hipGetLastError());
@@ -994,6 +1089,12 @@ int launch_gather(const void* in, int64_t n, int64_t elsize, const void* srec, i
     if (n <= 0) return 0;
     int64_t blocks = (n + kBlock - 1) / kBlock;
     if (blocks > 8192) blocks = 8192;
+    if (elsize == 32 && rw == 4 && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0) {
+        hipLaunchKernelGGL(gather32_kernel, dim3(rec32_blocks(n)), dim3(kBlock), 0, st, (const uint4*)in, n,
+                           (const uint2*)srec, iwords, (uint4*)out, checksum, err);
+        MPSG_CHECK(hipGetLastError());
+        return 0;
+    }
     hipLaunchKernelGGL(gather_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, (const uint8_t*)in,
                        n, elsize, (const uint32_t*)srec, rw, iwords, (uint8_t*)out, checksum, err);
     MPSG_CHECK(hipGetLastError());

@@ -141,3 +141,18 @@ def test_one_workgroup_record_types(dt, n, inplace):
     for k in ("P", "C", "myCLT", "myCLE", "myC", "send"):
         assert numpy.array_equal(c[k], info[k]), k
     assert st.checksum_in == info['checksum_in'] == st.checksum_out
+
+
+@pytest.mark.parametrize("n", [8193, 262145, 2048 * 1024 - 1, 2048 * 1024 + 1])
+@pytest.mark.parametrize("at", [0, 12, 24])
+def test_packed_32_byte_records(n, at):
+    """32-byte records sorted as packed {key, index}: the pack and the gather
+    at the edges of their blocks and of one round of them, with the key at
+    several places"""
+    dt = numpy.dtype({"names": ["key", "a", "b"], "formats": ["<i8", "<u4", "<u4"],
+                      "offsets": [at, (at + 8) % 32, (at + 16) % 32], "itemsize": 32})
+    g = numpy.random.default_rng(n + at)
+    a = numpy.frombuffer(g.bytes(32 * n), dt).copy()
+    a['key'] >>= 30
+    P = 7
+    check_parity(a, ragged(n, P, 1), ragged(n, P, 2), 'key', flags=_lib.FORCE_GENERAL, device=True)
