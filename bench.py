@@ -255,15 +255,18 @@ def bench_batched(args):
     loop_value = nrec / loop_s / 1e6
     each_value = nrec / each_s / 1e6
     # bytes the plan's passes move: a segment up to the in-LDS threshold is
-    # read and written once; a larger one is read by the digit histogram and
-    # read and written by one onesweep pass per key byte (uniform keys leave
-    # no digit place trivial)
+    # read and written once; one of up to 512 x 1843 records (of 8 or 16
+    # bytes) is read and written by its partition level and again by the sorts
+    # of its buckets; a larger one is read by the digit histogram and read and
+    # written by one onesweep pass per key byte (uniform keys leave no digit
+    # place trivial)
     pass_bytes = 0
     for g, info in zip(groups, plan_info):
         es = g["dtype"].itemsize
         kb = g["dtype"]['key'].itemsize
         small = int(g["sizes"][g["sizes"] <= info["threshold"]].sum())
-        pass_bytes += small * 2 * es + (g["n"] - small) * es * (1 + 2 * kb)
+        level = int(g["sizes"][g["sizes"] <= 512 * 1843].sum()) - small
+        pass_bytes += small * 2 * es + level * 4 * es + (g["n"] - small - level) * es * (1 + 2 * kb)
     pass_gbs = pass_bytes / (ms * 1e-3) / 1e9
     result = {
         "metric": "Mrecords/s, batched segmented sort (10,000 segments, 2^30 records)", "value": round(value, 2),
@@ -281,7 +284,8 @@ def bench_batched(args):
                           "form": "one mpsort_gpu_newarray call per segment, each waiting for its result"},
         "sort_equivalent_GBps": round(2.0 * nbytes / (ms * 1e-3) / 1e9, 1),
         "passes": {"bytes": pass_bytes, "GBps": round(pass_gbs, 1), "frac_of_hbm_peak": round(pass_gbs / HBM_PEAK_GBS, 3),
-                   "form": "segments up to the in-LDS threshold: one read and one write; larger ones: the "
+                   "form": "segments up to the in-LDS threshold: one read and one write; up to 943,616 records: "
+                           "two of each (partition level, bucket sorts); larger ones: the "
                            "histogram read plus one read and one write per key byte (4 passes for i32 keys, "
                            "8 for i64)"},
         "tuned_plan": {"i32_f32": plan_info[0], "i64_i64": plan_info[1]},
