@@ -466,19 +466,22 @@ def _device_copy(recs):
 
 
 PLAIN_LEVELS = ("sample", "level1", "level2", "bucket_sort")
+PLAIN_ONE_LEVEL = ("sample", "counts", "scatter", "bucket_sort")
+FORM_ONE_LAUNCH, FORM_ONE_LEVEL, FORM_TWO_LEVELS = 2, 3, 4  # mpsort_gpu_last_form
+FORM_STAGES = {FORM_ONE_LAUNCH: (), FORM_ONE_LEVEL: PLAIN_ONE_LEVEL, FORM_TWO_LEVELS: PLAIN_LEVELS}
 
 
 def learned_stages(st):
     """names of a learned call's pass_ms: two partition levels, or the per-rank
     form's kernels"""
-    return list(PLAIN_LEVELS) if len(st["pass_ms"]) == len(PLAIN_LEVELS) else LEARNED_KERNELS
+    return list(PLAIN_LEVELS) if st["form"] == FORM_TWO_LEVELS else LEARNED_KERNELS
 
 
 def plain_first_form(st):
     """(FirstSort form, entries of pass_ms before the SecondSort's) of a
     plain-path call's statistics"""
-    if st["first_passes"] == 0 and len(st["pass_ms"]) == 4 and st["second_passes"] == 0:
-        return "levels", 4  # two partition levels over all ranks, no SecondSort
+    if st["form"] in FORM_STAGES:
+        return "levels", len(st["pass_ms"])  # all ranks together, no SecondSort
     nsec = 4 if st["second_merged"] else st["second_passes"]
     if st["first_passes"] == 0 and len(st["pass_ms"]) - nsec == 6:
         return "buckets", 6
@@ -491,7 +494,7 @@ def plain_stages(st):
     ms = st["pass_ms"]
     out = {}
     if form == "levels":
-        return {name: round(ms[i], 4) for i, name in enumerate(PLAIN_LEVELS)}
+        return {name: round(x, 4) for name, x in zip(FORM_STAGES[st["form"]], ms)}
     if form == "buckets":
         for i, name in enumerate(("sample_tables", "hist", "scatter", "bucket_sort", "lds_radix", "fallback")):
             out["first_" + name] = round(ms[i], 4)
@@ -707,9 +710,12 @@ def bench_histsort(args):
                           "onesweep_kernel<4,1024,8> (one 8-bit digit pass, 2*n*16 B per launch)", TRAFFIC_ONESWEEP,
                           ROCPROF_MS.get("onesweep"))
     elif first_form == "levels":
-        plain_roof = roof([st["pass_ms"][3] for st in st_plain],
-                          "wide_sort_kernel<4> (fine buckets gathered and sorted in LDS, one launch per step over all n "
-                          "records, with the listed buckets' launches: 2*n*16 B)", None, None)
+        kernel = {FORM_ONE_LAUNCH: "the sort's one launch (2*n*16 B)",
+                  FORM_ONE_LEVEL: "interp_sort_kernel<4,512,9> (the buckets sorted in LDS, one launch per step over all n "
+                                  "records: 2*n*16 B)",
+                  FORM_TWO_LEVELS: "wide_sort_kernel<4> (fine buckets gathered and sorted in LDS, one launch per step over "
+                                   "all n records, with the listed buckets' launches: 2*n*16 B)"}[st_plain[-1]["form"]]
+        plain_roof = roof([st["pass_ms"][3] if k0 else st["t_total_ms"] for st in st_plain], kernel, None, None)
     else:
         plain_roof = roof([st["pass_ms"][3] for st in st_plain],
                           "interp_sort_kernel<4,512,9> (the plain FirstSort's in-LDS bucket sort, sampled tables, "
@@ -750,9 +756,12 @@ def bench_histsort(args):
             "buckets_overflow": last["buckets_overflow_first"]}
         log("plain bucket FirstSort: %s" % json.dumps(plain_first))
     elif first_form == "levels":
-        plain_first = {"form": "two partition levels over all ranks, in-LDS sorts of the fine buckets",
+        plain_first = {"form": {FORM_ONE_LAUNCH: "one launch",
+                                FORM_ONE_LEVEL: "one partition over all ranks, in-LDS sorts of the buckets",
+                                FORM_TWO_LEVELS: "two partition levels over all ranks, in-LDS sorts of the fine "
+                                                 "buckets"}[last["form"]],
                        "stages_ms": {name: round(sum(st["pass_ms"][i] for st in st_plain) / len(st_plain), 4)
-                                     for i, name in enumerate(PLAIN_LEVELS)},
+                                     for i, name in enumerate(FORM_STAGES[last["form"]])},
                        "buckets": last["buckets"], "buckets_listed": last["buckets_listed"],
                        "buckets_lds_radix": last["buckets_lds_radix"], "buckets_overflow": last["buckets_overflow"]}
         log("plain partition levels: %s" % json.dumps(plain_first))

@@ -152,20 +152,25 @@ typedef struct {
     int32_t record_bytes;    /* sort record size actually moved */
     int32_t first_passes;    /* digit passes run by FirstSort */
     int32_t second_passes;
-    int32_t bisect_rounds;   /* max over splitters */
+    int32_t bisect_rounds;   /* max over splitters; 0 where the splitters are read off the sorted
+                                records (forms other than MPSORT_GPU_FORM_RANKS) */
     int32_t general_path;    /* 1 when packed {key, index} records were sorted */
     int64_t nrecords;
     int64_t checksum_in;
     int64_t checksum_out;
     int32_t npass_ms;        /* entries used in pass_ms */
     int32_t learned;         /* 1 when the learned path ran */
-    double pass_ms[64];      /* per digit pass kernel time (FirstSort then SecondSort) */
+    double pass_ms[64];      /* per digit pass kernel time (FirstSort then SecondSort); a sort of all
+                                ranks together in partition levels (mpsort_gpu_last_form) leaves
+                                four entries: the sample and its boundaries; then with one level the
+                                bucket counts, the scatter, the bucket sorts, with two level 1, level 2,
+                                the bucket sorts */
     /* learned path */
     int32_t splitters_exact;   /* proposals accepted without repair */
     int32_t splitters_repaired;
     int32_t buckets;
     int32_t buckets_overflow;  /* buckets that fell back to the plain sort */
-    int32_t repair_rounds;
+    int32_t repair_rounds;     /* as bisect_rounds */
     int32_t plain_sides;       /* local sorts that took the plain radix path */
     double t_model_ms;
     double t_bucket_ms;
@@ -174,11 +179,30 @@ typedef struct {
     int32_t buckets_listed;    /* buckets sorted by the 1024-thread in-LDS form from a list */
     int32_t exchange_sparse;   /* 1 when the exchange walked the non-empty runs only */
     int32_t exchange_runs;     /* runs in the table it walked (P * P when dense) */
-    int32_t second_merged;     /* 1 when the SecondSort gathered every receiver bucket from the
-                                  senders' sorted segments (no exchange, no digit passes) */
+    int32_t second_merged;     /* 1 when no exchange and no digit passes followed the FirstSort of
+                                  several ranks: every receiver bucket was gathered from the senders'
+                                  sorted segments (MPSORT_GPU_FORM_RANKS), or all ranks' records were
+                                  sorted together */
 } mpsort_gpu_stats;
 
 int mpsort_gpu_last_stats(mpsort_gpu_stats *stats);
+
+/* What sorted the records of the last mpsort_gpu_newarray* call (no
+ * counterpart in the reference; the result is the same):
+ *   RANKS       the reference's steps: FirstSort of every rank, splitter
+ *               search, layout, exchange and SecondSort (or the merged
+ *               SecondSort)
+ *   ONE_LAUNCH  all ranks together in one launch (at most 8192 records)
+ *   ONE_LEVEL   all ranks together by one partition into in-LDS buckets
+ *   TWO_LEVELS  the same in two partition levels
+ * In the last three the splitters and counts are read off the sorted records.
+ * NONE: the call failed or sorted nothing. */
+#define MPSORT_GPU_FORM_NONE 0
+#define MPSORT_GPU_FORM_RANKS 1
+#define MPSORT_GPU_FORM_ONE_LAUNCH 2
+#define MPSORT_GPU_FORM_ONE_LEVEL 3
+#define MPSORT_GPU_FORM_TWO_LEVELS 4
+int mpsort_gpu_last_form(void);
 
 /* Fault hooks, for tests of the paths that the checks of the reference
  * guard (it aborts instead, mpsort-mpi.c:324-330,496-510,707-716); no

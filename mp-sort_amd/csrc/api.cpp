@@ -65,6 +65,7 @@ static mpsort_gpu_malloc_fn g_malloc = nullptr;
 static mpsort_gpu_free_fn g_free = nullptr;
 static void* g_alloc_ud = nullptr;
 static mpsort_gpu_stats g_last;
+static int g_form = MPSORT_GPU_FORM_NONE;  // what sorted the last call's records
 
 // ---- host allocation hook (mp-mpiu.h:4-16): the library's large host
 // temporaries go through it
@@ -952,6 +953,7 @@ static int run_histsort(DevCtx& c, const CallShape& cs, const void* d_in, void* 
     if (cs.checksum && !packed_host && sums[0] != sums[1])
         return fail(MPSORT_ERR_CHECKSUM, "MPSort: Data changed after sorting; checksum mismatch (%lld != %lld)",
                     sums[0], sums[1]);
+    g_form = MPSORT_GPU_FORM_RANKS;
     return 0;
 }
 
@@ -1689,7 +1691,7 @@ static int direct_counts_arrays(DevCtx& c, int P, DirectWork* w, DirectResult** 
 }
 // the statistics and recorded counts both forms leave, and their checks
 static int direct_results(DevCtx& c, const CallShape& cs, const DirectWork& w, const DirectResult& got, bool host_sum,
-                          mpsort_gpu_stats* stats) {
+                          int form, mpsort_gpu_stats* stats) {
     stats->nvranks = cs.P;
     stats->second_merged = cs.P > 1 ? 1 : 0;
     stats->record_bytes = (int32_t)(cs.rw * 4);
@@ -1712,6 +1714,7 @@ static int direct_results(DevCtx& c, const CallShape& cs, const DirectWork& w, c
     if (cs.checksum && !host_sum && got.sums[0] != got.sums[1])
         return fail(MPSORT_ERR_CHECKSUM, "MPSort: Data changed after sorting; checksum mismatch (%lld != %lld)",
                     (long long)got.sums[0], (long long)got.sums[1]);
+    g_form = form;
     return 0;
 }
 
@@ -1739,7 +1742,7 @@ static int run_small(DevCtx& c, const CallShape& cs, const void* d_in, void* d_o
     const DirectResult got = *res;
     stats->first_passes = (int32_t)got.lists[3];
     stats->t_first_sort_ms = stats->t_total_ms = ev_ms(c.ev[kEvStart], c.ev[kEvEnd]);
-    return direct_results(c, cs, w, got, false, stats);
+    return direct_results(c, cs, w, got, false, MPSORT_GPU_FORM_ONE_LAUNCH, stats);
 }
 
 static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
@@ -1892,7 +1895,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         for (int i = 0; i < 4; i++) stats->pass_ms[i] = ev_ms(pe[i], pe[i + 1]);
         stats->npass_ms = 4;
     }
-    return direct_results(c, cs, w, got, packed_host != nullptr, stats);
+    return direct_results(c, cs, w, got, packed_host != nullptr, MPSORT_GPU_FORM_ONE_LEVEL, stats);
 }
 
 // ---- the same in two partition levels (wide.hip), above one level's sizes
@@ -2077,10 +2080,8 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         stats->learned = 1;
         stats->splitters_exact = P > 1 ? (int32_t)got.exact : 0;
         stats->splitters_repaired = P > 1 ? P - 1 - stats->splitters_exact : 0;
-        // one round where every proposal holds, else the result is read too
-        stats->bisect_rounds = stats->repair_rounds = P > 1 ? (stats->splitters_repaired ? 2 : 1) : 0;
     }
-    return direct_results(c, cs, d, got, packed_host != nullptr, stats);
+    return direct_results(c, cs, d, got, packed_host != nullptr, MPSORT_GPU_FORM_TWO_LEVELS, stats);
 }
 
 // The learned path by two partition levels: per-rank bucket sorts, bounds and
@@ -2396,6 +2397,7 @@ static int run_histsort_learned(DevCtx& c, const CallShape& cs, const void* d_in
     if (cs.checksum && sums[0] != sums[1])
         return fail(MPSORT_ERR_CHECKSUM, "MPSort: Data changed after sorting; checksum mismatch (%lld != %lld)",
                     sums[0], sums[1]);
+    g_form = MPSORT_GPU_FORM_RANKS;
     return 0;
 }
 
@@ -3004,6 +3006,7 @@ int mpsort_gpu_device_count(void) {
 int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, const int64_t* nout,
                         size_t elsize, const mpsort_key_desc* key, unsigned flags) {
     g_err[0] = 0;
+    g_form = MPSORT_GPU_FORM_NONE;
     int64_t ntot = 0;
     int rc = validate_counts(nin, P, nout, &ntot);
     if (rc) return rc;
@@ -3049,6 +3052,7 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
 int mpsort_gpu_newarray_noalloc(const void* base, const int64_t* nin, int P, void* out, const int64_t* nout,
                                 size_t elsize, const mpsort_key_desc* key, unsigned flags) {
     g_err[0] = 0;
+    g_form = MPSORT_GPU_FORM_NONE;
     int64_t ntot = 0;
     int rc = validate_counts(nin, P, nout, &ntot);
     if (rc) return rc;
@@ -3215,6 +3219,7 @@ int mpsort_gpu_newarray_radix(const void* base, const int64_t* nin, int P, void*
                               size_t elsize, void (*radix)(const void* ptr, void* radix, void* arg), size_t rsize,
                               void* arg, unsigned flags) {
     g_err[0] = 0;
+    g_form = MPSORT_GPU_FORM_NONE;
     int64_t ntot = 0;
     int rc = validate_counts(nin, P, nout, &ntot);
     if (rc) return rc;
@@ -3310,6 +3315,7 @@ int mpsort_gpu_last_stats(mpsort_gpu_stats* s) {
     *s = g_last;
     return 0;
 }
+int mpsort_gpu_last_form(void) { return g_form; }
 
 // The reference's timer lines in its order (mpsort-mpi.c:366-602): seconds
 // since the previous line.  Stages that one kernel does together with the
@@ -3855,6 +3861,7 @@ int mpsort_gpu_newarray_learned(const void* base, const int64_t* nin, int P, voi
                                 size_t elsize, const mpsort_key_desc* key, const mpsort_gpu_model* model,
                                 unsigned flags) {
     g_err[0] = 0;
+    g_form = MPSORT_GPU_FORM_NONE;
     if (!model) return fail(MPSORT_ERR_ARG, "model is NULL");
     int64_t ntot = 0;
     int rc = validate_counts(nin, P, nout, &ntot);

@@ -60,8 +60,10 @@ EXPORTS = [
     "mpsort_gpu_segplan_run", "mpsort_gpu_segplan_info", "mpsort_gpu_segplan_free",
     "mpsort_gpu_sort_segments",
     "mpiu_malloc", "mpiu_free", "mpiu_set_malloc", "mpsort_gpu_newarray_noalloc", "mpsort_gpu_set_faults",
-    "mpsort_gpu_segplan_shape",
+    "mpsort_gpu_segplan_shape", "mpsort_gpu_last_form",
 ]
+
+FORM_NONE, FORM_RANKS, FORM_ONE_LAUNCH, FORM_ONE_LEVEL, FORM_TWO_LEVELS = range(5)
 
 SEGPLAN_GRAPH = 1 << 0
 SEGPLAN_TUNE = 1 << 1
@@ -100,6 +102,8 @@ class Stats(ctypes.Structure):
         ("exchange_runs", ctypes.c_int32), ("second_merged", ctypes.c_int32),
     ]
 
+    form = FORM_NONE  # of last_stats: what sorted the records
+
     def as_dict(self):
         d = {}
         for name, _ in self._fields_:
@@ -107,6 +111,7 @@ class Stats(ctypes.Structure):
             if name == "pass_ms":
                 v = [self.pass_ms[i] for i in range(self.npass_ms)]
             d[name] = v
+        d["form"] = self.form
         return d
 
 
@@ -205,6 +210,7 @@ def check(rc):
 def last_stats():
     s = Stats()
     check(lib.mpsort_gpu_last_stats(ctypes.byref(s)))
+    s.form = int(lib.mpsort_gpu_last_form())
     return s
 
 
