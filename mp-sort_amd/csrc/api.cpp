@@ -1649,10 +1649,20 @@ static bool direct_asked(const CallShape& cs) {
 static bool direct_eligible(const CallShape& cs) {
     return direct_asked(cs) && (cs.rw == 2 || cs.rw == 4) && cs.ntot > kSmallRecords && cs.ntot <= kDirectMaxRecords;
 }
-// One workgroup sorts everything, any record size (a packed call's records
-// directly, without packing).
-static bool small_eligible(const CallShape& cs) {
-    return direct_asked(cs) && cs.ntot >= 1 && cs.ntot <= kSmallRecords && cs.elsize <= (1 << 16);
+// One launch, any record size (a packed call's records directly, without
+// packing).  Up to kRankRecords records with input and output apart are placed
+// by workgroups of 16 records, which beats the per-rank form at every size
+// (4096 records of 64 KiB: 327 against 3531 us).  Otherwise one workgroup moves
+// all bytes: 8192 records of 256 bytes take 521 us, of 512 bytes 1657, the
+// per-rank form 550 and 557; where the records or their addresses are not
+// whole words it moves single bytes, and 8192 records of 125 bytes take 525 us,
+// of 189 bytes 728, the per-rank form 587 and 613.
+constexpr int64_t kSmallWordBytes = 2 << 20, kSmallByteBytes = 1 << 20;
+static bool small_eligible(const CallShape& cs, const void* in, const void* out) {
+    if (!direct_asked(cs) || cs.ntot < 1 || cs.ntot > kSmallRecords || cs.elsize > (1 << 16)) return false;
+    if (!cs.general || cs.ntot <= kRankRecords) return true;
+    const bool words = ((cs.elsize | (int64_t)(uintptr_t)in | (int64_t)(uintptr_t)out) & 3) == 0;
+    return cs.ntot * cs.elsize <= (words ? kSmallWordBytes : kSmallByteBytes);
 }
 
 // the rank tables and the counts' device arrays of the two forms
@@ -3033,7 +3043,7 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
     memset(&st, 0, sizeof st);
     remember_key(*c, key, 0, 0);
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
-        if (small_eligible(cs)) return run_small(*c, cs, d_in, d_out, nin, nout, &st);
+        if (small_eligible(cs, d_in, d_out)) return run_small(*c, cs, d_in, d_out, nin, nout, &st);
         if (direct_eligible(cs)) return run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st);
         int r2 = 0;
         if (wide_eligible(cs)) {

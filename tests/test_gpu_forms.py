@@ -37,6 +37,22 @@ def test_form_by_size(n, form):
     assert st.bisect_rounds == 0 and st.first_passes <= 8 and st.second_passes == 0
 
 
+@pytest.mark.parametrize("itemsize, n, form", [
+    (1024, 4096, _lib.FORM_ONE_LAUNCH), (1024, 4097, _lib.FORM_RANKS), (1024, 8192, _lib.FORM_RANKS),
+    (256, 8192, _lib.FORM_ONE_LAUNCH), (260, 8192, _lib.FORM_RANKS), (128, 8192, _lib.FORM_ONE_LAUNCH),
+    (127, 8192, _lib.FORM_ONE_LAUNCH), (129, 8192, _lib.FORM_RANKS), (1023, 4096, _lib.FORM_ONE_LAUNCH),
+    (1023, 4097, _lib.FORM_RANKS), (65536, 17, _lib.FORM_ONE_LAUNCH)])
+def test_form_of_wide_records(itemsize, n, form):
+    """records of more bytes than one workgroup should move are spread over
+    the chip: both sides of 4096 records and of the bounds in bytes"""
+    dt = numpy.dtype({"names": ["key"], "formats": ["<u8"], "offsets": [itemsize // 2], "itemsize": itemsize})
+    g = numpy.random.default_rng(itemsize)
+    a = numpy.frombuffer(g.bytes(itemsize * n), dt).copy()
+    a['key'] >>= 52
+    out, st = check_parity(a, ragged(n, 5, 1), ragged(n, 5, 2), 'key', device=True)
+    assert st.form == form
+
+
 @pytest.mark.parametrize("why", ["ranks", "wide key", "4-byte records", "exchange", "radix FirstSort", "bucket FirstSort"])
 def test_calls_that_keep_the_ranks(why):
     n, P, flags, field = 30000, 65 if why == "ranks" else 4, 0, 'key'
