@@ -13,7 +13,7 @@
 namespace mpsg {
 
 // ---------------------------------------------------------------------------
-// Sample.  Block c takes the keys at positions (2u + 1) n / 2S, u = 1024 c ..
+// Sample.  Block c takes the keys at positions sample_pos(u), u = 1024 c ..
 // 1024 c + 1023, and sorts them: one key per thread, a bitonic network whose
 // strides below 64 are lane exchanges and whose ten larger ones go through
 // LDS.  Block 0 also writes the call's tables and clears its counters (every
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kDirectChunk) void direct_sample_kernel(const uint3
         if (tid < 2 && clear_sums) w.checksum[tid] = 0;
     }
     const int64_t u = (int64_t)blockIdx.x * kDirectChunk + tid;
-    const int64_t pos = ((2 * u + 1) * sh.n) / (2 * (int64_t)sh.S);
+    const int64_t pos = (int64_t)sample_pos((uint32_t)u, (uint32_t)sh.S, (uint64_t)sh.n);
     uint32_t r[RW];
     RecIO<RW>::load(src, pos, r);
     const uint64_t v = bitonic1024(lkey<RW>(r, lk), s_k);

@@ -52,6 +52,22 @@ __device__ __forceinline__ int seg_of_tile(const SegDev& seg, int64_t tile) {
     return upper_index<int64_t>(seg.tile_start, seg.nseg, tile);
 }
 
+// Position of sample u of m among n records (u < m <= n; u < 2^15, n < 2^32):
+// somewhere in the u-th of m equal parts, by a fixed hash of u (the finaliser of
+// Appleby's MurmurHash3).  Even positions meet data of a period that divides
+// n / m, such as records interleaved from several sources or a grid in row
+// order, always at the same phase: 2^21 records of 128 interleaved sources were
+// sampled from one source, and all others fell into two buckets.
+__device__ __forceinline__ uint64_t sample_pos(uint32_t u, uint32_t m, uint64_t n) {
+    uint32_t h = u;
+    h ^= h >> 16;
+    h *= 0x85ebca6bu;
+    h ^= h >> 13;
+    h *= 0xc2b2ae35u;
+    h ^= h >> 16;
+    return ((((uint64_t)u << 16) | (h & 0xffffu)) * n >> 16) / m;
+}
+
 // exclusive scan of B values, one per thread of a B-thread block
 template <int B>
 __device__ __forceinline__ uint32_t scan_block(uint32_t v, uint32_t* s_tmp /*B / 64*/) {

@@ -394,8 +394,8 @@ __global__ __launch_bounds__(256) void wide_offsets_kernel(WideWork w) {
 }
 
 // ---------------------------------------------------------------------------
-// Fine boundaries: up to 4096 keys at even positions of a coarse bucket,
-// sorted in LDS by a bitonic network.
+// Fine boundaries: up to 4096 keys of a coarse bucket, one in each of as many
+// equal parts of it (sample_pos), sorted in LDS by a bitonic network.
 template <int RW, bool SEG>
 __global__ __launch_bounds__(1024) void wide_sample_kernel(const uint32_t* __restrict__ src, LKey lk, WideWork w) {
     constexpr int I = kWideSamples / 1024;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(1024) void wide_sample_kernel(const uint32_t* __res
 #pragma unroll
     for (int k = 0; k < I; k++) {
         const uint32_t u = min((uint32_t)(k * 1024 + tid), m - 1);
-        pos[k] = (uint32_t)(((2 * (uint64_t)u + 1) * n) / (2 * (uint64_t)m));
+        pos[k] = (uint32_t)sample_pos(u, m, n);
         at[k] = w.cbase[c] + pos[k];
     }
     if constexpr (!SEG) {
