@@ -21,7 +21,12 @@ constexpr int kWideSamples = 4096;               // sample keys of a coarse buck
 constexpr int kWideCopy = 4096;                  // records of one copy task
 constexpr int kWideCap = kMergeCap;              // a group of fine buckets sorted by 512 x 6 threads and records
 constexpr int kWideFine = 1024;                  // records per fine bucket while 512 buckets suffice
-constexpr int64_t kWideMaxRecords = (int64_t)1 << 29;
+// The largest call: an average coarse bucket of 7/16 of what kWideRuns tiles
+// hold.  Its boundaries are 32 sample keys apart, so bucket sizes deviate by 18%
+// on average: one call in 100,000 of randomly ordered keys has a bucket above
+// the limit and takes the per-rank form after all, at 400 M records one in 700,
+// at 2^29 nineteen in twenty.
+constexpr int64_t kWideMaxRecords = (int64_t)kWideBuckets * kWideRuns * kWideTile / 16 * 7;
 
 // a group of neighbouring fine buckets [f, fe) and its tiles' runs
 struct WideBucket {

@@ -7,7 +7,7 @@ import sys
 import numpy
 import pytest
 
-from gpu_util import even, gpu_sort
+from gpu_util import even, gpu_sort, gpu_sort_device
 from mpsort import _lib, learned, workloads
 from mpsort._lib import lib
 from test_gpu_direct import ragged
@@ -35,6 +35,21 @@ def test_form_by_size(n, form):
     out, st = check_parity(a, ragged(n, 5, 1), ragged(n, 5, 2), 'key', device=True)
     assert st.form == form
     assert st.bisect_rounds == 0 and st.first_passes <= 8 and st.second_passes == 0
+
+
+@pytest.mark.parametrize("past, form", [(0, _lib.FORM_TWO_LEVELS), (1, _lib.FORM_RANKS)])
+def test_the_largest_two_level_sort(past, form):
+    """sorted, and the same keys: as many of every top 16 bits, and equal sums
+    and exclusive ors"""
+    n, P = 512 * 256 * 6144 // 16 * 7 + past, 3
+    note("two levels at their largest, n=%d" % n)
+    a = numpy.random.default_rng(5).integers(0, 2 ** 64, n, dtype=numpy.uint64)
+    out, st = gpu_sort_device(a, ragged(n, P, 1), ragged(n, P, 2))
+    assert st.form == form
+    assert (out[1:] >= out[:-1]).all()
+    top = lambda x: numpy.bincount((x >> numpy.uint64(48)).astype(numpy.uint16), minlength=1 << 16)
+    assert numpy.array_equal(top(out), top(a))
+    assert out.sum() == a.sum() and numpy.bitwise_xor.reduce(out) == numpy.bitwise_xor.reduce(a)
 
 
 @pytest.mark.parametrize("itemsize, n, form", [
