@@ -42,8 +42,9 @@ int launch_exchange_hist(const void* src, void* dst, int64_t ntot, int rw, const
                          const int64_t* C, int P, const KeySpec& ks, uint32_t* hist, hipStream_t st);
 int launch_pack(const void* in, int64_t n, int64_t elsize, int64_t key_off, int key_bytes,
                 void* out, int rw, int iwords, long long* checksum, hipStream_t st);
+// skip (optional): nothing is written where *skip is set on the device
 int launch_gather(const void* in, int64_t n, int64_t elsize, const void* srec, int rw, int iwords, void* out,
-                  long long* checksum, uint32_t* err, hipStream_t st);
+                  long long* checksum, uint32_t* err, hipStream_t st, const uint32_t* skip = nullptr);
 
 // Workspace of mpsort_gpu_newarray_noalloc: a fixed array in each GPU's
 // memory, held for the life of the process.  Host code never uses this name
@@ -2038,7 +2039,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         int r2 = 0;
         if (cs.general &&
             (r2 = launch_gather(d_in, n, cs.elsize, dst, rw, cs.iwords, d_out, cs.checksum ? d.checksum + 1 : nullptr,
-                                d.err, st)))
+                                d.err, st, w.lists + 5)))
             return r2;
         if ((r2 = launch_wide_counts(rw, dst, a, lk, sh, d, w, res, c.ev[kEvEnd], st))) return r2;
         MPSG_CHECK(hipStreamSynchronize(st));

@@ -852,8 +852,10 @@ __global__ __launch_bounds__(kBlock) void gather_kernel(const uint8_t* __restric
                                                         int64_t elsize, const uint32_t* __restrict__ srec,
                                                         int rw, int iwords, uint8_t* __restrict__ out,
                                                         long long* __restrict__ checksum,
-                                                        uint32_t* __restrict__ error_flag) {
+                                                        uint32_t* __restrict__ error_flag,
+                                                        const uint32_t* __restrict__ skip) {
     __shared__ long long s_sum[kWaves];
+    if (skip && *skip) return;
     long long csum = 0;
     const bool words = (elsize & 3) == 0 && ((uintptr_t)in & 3) == 0 && ((uintptr_t)out & 3) == 0;
     const bool vec = (elsize & 15) == 0 && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0;
@@ -1026,9 +1028,11 @@ __global__ __launch_bounds__(kBlock) void pack32_kernel(const uint4* __restrict_
 __global__ __launch_bounds__(kBlock) void gather32_kernel(const uint4* __restrict__ in, int64_t n,
                                                           const uint2* __restrict__ srec, int iwords,
                                                           uint4* __restrict__ out, long long* __restrict__ checksum,
-                                                          uint32_t* __restrict__ error_flag) {
+                                                          uint32_t* __restrict__ error_flag,
+                                                          const uint32_t* __restrict__ skip) {
     constexpr int U = kRec32Unroll;
     __shared__ long long s_sum[kWaves];
+    if (skip && *skip) return;
     long long csum = 0;
     for (int64_t o0 = (int64_t)blockIdx.x * kBlock * U + threadIdx.x; o0 < n; o0 += (int64_t)gridDim.x * kBlock * U) {
         int64_t at[U];
@@ -1085,18 +1089,18 @@ int launch_pack(const void* in, int64_t n, int64_t elsize, int64_t key_off, int 
 }
 
 int launch_gather(const void* in, int64_t n, int64_t elsize, const void* srec, int rw, int iwords, void* out,
-                  long long* checksum, uint32_t* err, hipStream_t st) {
+                  long long* checksum, uint32_t* err, hipStream_t st, const uint32_t* skip) {
     if (n <= 0) return 0;
     int64_t blocks = (n + kBlock - 1) / kBlock;
     if (blocks > 8192) blocks = 8192;
     if (elsize == 32 && rw == 4 && ((uintptr_t)in & 15) == 0 && ((uintptr_t)out & 15) == 0) {
         hipLaunchKernelGGL(gather32_kernel, dim3(rec32_blocks(n)), dim3(kBlock), 0, st, (const uint4*)in, n,
-                           (const uint2*)srec, iwords, (uint4*)out, checksum, err);
+                           (const uint2*)srec, iwords, (uint4*)out, checksum, err, skip);
         MPSG_CHECK(hipGetLastError());
         return 0;
     }
     hipLaunchKernelGGL(gather_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, st, (const uint8_t*)in,
-                       n, elsize, (const uint32_t*)srec, rw, iwords, (uint8_t*)out, checksum, err);
+                       n, elsize, (const uint32_t*)srec, rw, iwords, (uint8_t*)out, checksum, err, skip);
     MPSG_CHECK(hipGetLastError());
     return 0;
 }
