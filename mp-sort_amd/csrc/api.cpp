@@ -1729,6 +1729,19 @@ static int direct_results(DevCtx& c, const CallShape& cs, const DirectWork& w, c
     return 0;
 }
 
+// A workspace of the partition forms that cannot be had (rc): they hold up to
+// one buffer of records more than the per-rank form, so the call takes that
+// one, which says itself when it is short of memory
+static int short_of_memory(DevCtx& c, int rc, bool* again) {
+    if (rc != MPSORT_ERR_NOMEM) return rc;
+    (void)hipGetLastError();
+    g_err[0] = 0;
+    c.s2.release();
+    c.ltile.release();
+    *again = true;
+    return 0;
+}
+
 static int run_small(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
                      const int64_t* nout, mpsort_gpu_stats* stats) {
     int rc = 0;
@@ -1756,8 +1769,9 @@ static int run_small(DevCtx& c, const CallShape& cs, const void* d_in, void* d_o
     return direct_results(c, cs, w, got, false, MPSORT_GPU_FORM_ONE_LAUNCH, stats);
 }
 
+// *again: nothing was written, the call takes the per-rank form
 static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
-                      const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats) {
+                      const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats, bool* again) {
     hipStream_t st = c.st;
     const int P = cs.P, rw = cs.rw;
     const int64_t n = cs.ntot;
@@ -1794,11 +1808,11 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     };
     Sizer lz;
     lay(lz, [](Sizer& a, auto*& p, size_t k) { a.take<std::remove_reference_t<decltype(*p)>>(k); });
-    if ((rc = c.ltile.ensure(lz.off + 4096))) return rc;
+    if ((rc = c.ltile.ensure(lz.off + 4096)) || (rc = c.s1.ensure((size_t)n * recbytes)) ||
+        (cs.general && ((rc = c.rbuf.ensure((size_t)n * recbytes)) || (rc = c.s0.ensure((size_t)n * recbytes)))))
+        return short_of_memory(c, rc, again);
     Arena la{(char*)c.ltile.p};
     lay(la, [](Arena& a, auto*& p, size_t k) { p = a.take<std::remove_reference_t<decltype(*p)>>(k); });
-    if ((rc = c.s1.ensure((size_t)n * recbytes))) return rc;
-    if (cs.general && ((rc = c.rbuf.ensure((size_t)n * recbytes)) || (rc = c.s0.ensure((size_t)n * recbytes)))) return rc;
     // ---- the sort
     // (the timing events ride on the launches they bracket: an event recorded
     // between two launches costs the GPU about 4.5 us)
@@ -1918,7 +1932,7 @@ static bool wide_eligible(const CallShape& cs) {
 // M: the learned path; the coarse boundaries are the model's quantiles, and
 // its splitters are compared with those read off the result.
 // *again: nothing was written, the call takes another path (the sample, or the
-// model, missed the sizes of the coarse buckets by far)
+// model, missed the sizes of the coarse buckets by far, or memory is short)
 static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
                     const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats, bool* again,
                     const LearnedModel* M = nullptr) {
@@ -1985,8 +1999,9 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     };
     Sizer lz;
     lay(lz, [](Sizer& a, auto*& p, size_t k) { a.take<std::remove_reference_t<decltype(*p)>>(k); });
-    if ((rc = c.ltile.ensure(lz.off + 4096)) || (rc = c.s1.ensure(bytes)) || (rc = c.s2.ensure(bytes))) return rc;
-    if (cs.general && ((rc = c.rbuf.ensure(bytes)) || (rc = c.s0.ensure(bytes)))) return rc;
+    if ((rc = c.ltile.ensure(lz.off + 4096)) || (rc = c.s1.ensure(bytes)) || (rc = c.s2.ensure(bytes)) ||
+        (cs.general && ((rc = c.rbuf.ensure(bytes)) || (rc = c.s0.ensure(bytes)))))
+        return short_of_memory(c, rc, again);
     Arena la{(char*)c.ltile.p};
     lay(la, [](Arena& a, auto*& p, size_t k) { p = a.take<std::remove_reference_t<decltype(*p)>>(k); });
     w.raw = d.raw;
@@ -3045,11 +3060,12 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
     remember_key(*c, key, 0, 0);
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
         if (small_eligible(cs, d_in, d_out)) return run_small(*c, cs, d_in, d_out, nin, nout, &st);
-        if (direct_eligible(cs)) return run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st);
+        const bool one = direct_eligible(cs);
         int r2 = 0;
-        if (wide_eligible(cs)) {
+        if (one || wide_eligible(cs)) {
             bool again = false;
-            r2 = run_wide(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again);
+            r2 = one ? run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again)
+                     : run_wide(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again);
             if (r2 || !again) return r2;
         }
         HistWork w;
@@ -3302,9 +3318,9 @@ int mpsort_gpu_newarray_radix(const void* base, const int64_t* nin, int P, void*
     // the gather's device checksum covers the output; the input sum is the
     // host's (the device sees only the packed records)
     cs.checksum = !(flags & MPSORT_GPU_NO_CHECKSUM);
-    if (direct_eligible(cs)) {
-        rc = run_direct(*c, cs, c->din.p, c->dout.p, nin, nout, packed, &st);
-    } else {
+    bool again = !direct_eligible(cs);
+    if (!again) rc = run_direct(*c, cs, c->din.p, c->dout.p, nin, nout, packed, &st, &again);
+    if (!rc && again) {
         HistWork w;
         rc = histwork_cached(*c, cs, histsort_need(cs, nin, nout, true), &w);
         if (!rc) rc = run_histsort(*c, cs, c->din.p, c->dout.p, nin, nout, packed, &st, w);

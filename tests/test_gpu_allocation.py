@@ -1,5 +1,6 @@
-"""Device allocations that fail, through the allocator hook: a failed call
-leaves the caller's output as it was."""
+"""Device allocations that fail, through the allocator hook: a call that the
+per-rank form has memory for still succeeds, and a failed call leaves the
+caller's output as it was."""
 import ctypes
 
 import numpy
@@ -94,3 +95,27 @@ def test_failed_call_leaves_the_output(itemsize):
             break
         fail += 1
     assert fail > 4
+
+
+@pytest.mark.parametrize("rec, n, P, first", [("rec16", 5000011, 1, _lib.FIRST_RADIX),
+                                              ("rows24", 5000011, 4, _lib.FIRST_BUCKETS)])
+def test_memory_of_the_per_rank_form_suffices(rec, n, P, first):
+    """device memory for what the per-rank form holds (first: the FirstSort
+    it takes at this size), but not for the two-level form's buffers"""
+    g = numpy.random.default_rng(n)
+    a = numpy.zeros(n, [('key', 'u8'), ('v', 'i8')] if rec == "rec16" else [('v', 'i8', 2), ('key', 'u8')])
+    a['key'] = g.integers(0, 1 << 40, n)
+    a['v'] = numpy.arange(a['v'].size).reshape(a['v'].shape)
+    want = a[numpy.argsort(a['key'], kind='stable')].view(numpy.uint8)
+    with Allocator(lambda i, nbytes, held: False) as al:
+        rc, out = sort_into_marked(a, P, flags=first)
+        assert rc == 0 and lib.mpsort_gpu_last_form() == _lib.FORM_RANKS
+        budget = sum(al.sizes.values())
+    with Allocator(lambda i, nbytes, held: held + nbytes > budget) as al:
+        rc, out = sort_into_marked(a, P)
+        note("n=%d: %d bytes held, budget %d, %d allocations failed" % (n, sum(al.sizes.values()), budget, al.failed))
+        assert rc == 0, lib.mpsort_gpu_last_error()
+        assert al.failed and lib.mpsort_gpu_last_form() == _lib.FORM_RANKS
+        assert numpy.array_equal(out, want)
+        rc, out = sort_into_marked(a, P)  # and again, with what the first call left allocated
+        assert rc == 0 and numpy.array_equal(out, want)
