@@ -1851,10 +1851,10 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
                                                  cs.general ? nullptr : c.ev[kEvStart], st)) ||
         (rc = mark(1)) || (rc = launch_direct_count(rw, src, lk, sh, w, cs_in, st)) || (rc = mark(2)) ||
         (rc = launch_lscatter(rw, src, tmp, eq_direct ? dst : tmp, sd, sh.ntiles, w.bkt, w.tables, 0, w.tile_off,
-                              w.err + 1, st, w.tot, n, w.base)) ||
+                              w.err + 1, st, w.tot, n, w.base, cs_out)) ||
         (rc = mark(3)) ||
         (rc = launch_chunk_sort_small(rw, tmp, dst, lk, w.tot, w.base, w.tables, 0, sh.W, w.overflow, w.lists, kLBins,
-                                      w.hard, w.lists + 1, w.medium, w.lists + 2, cs_out, eq_direct, st, nullptr,
+                                      w.hard, w.lists + 1, w.medium, w.lists + 2, cs_out, eq_direct ? kEqSummed : kEqNone, st, nullptr,
                                       (uint32_t)kChunkCap, small_form, c.ev[kEvFirst])) ||
         (rc = mark(4)))
         return rc;

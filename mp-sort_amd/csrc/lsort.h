@@ -81,14 +81,18 @@ int lscatter_tile(int rw);
 // tile_off[tile][b]: offset of the tile's bucket-b run inside its segment
 int launch_ltile_scan(const uint16_t* tile_cnt, const SegDev& sd, const int64_t* bucket_base, uint32_t* tile_off,
                       hipStream_t st);
+// the single-value buckets: sorted as the others, already in dst, already
+// summed as well
+enum { kEqNone = 0, kEqDone = 1, kEqSummed = 2 };
 // records of single-value buckets go to eq_dst, the rest to dst; bkt: the
 // buckets written by launch_lhist.  tot (optional): the segments share one
 // bucket space over records [0, gend) -- tot[b] records in bucket b,
-// tile_off counted from the bucket's start, the starts written to base_out
+// tile_off counted from the bucket's start, the starts written to base_out,
+// the records of single-value buckets added to *eq_sum (may be null)
 int launch_lscatter(int rw, const void* src, void* dst, void* eq_dst, const SegDev& sd, int64_t ntiles,
                     const uint16_t* bkt, const uint64_t* tables, int64_t tstride, const uint32_t* tile_off,
                     uint32_t* err, hipStream_t st, const uint32_t* tot = nullptr, int64_t gend = 0,
-                    int64_t* base_out = nullptr);
+                    int64_t* base_out = nullptr, long long* eq_sum = nullptr);
 // Sorts every bucket (src -> dst, same slots).  eq_done: the scatter already
 // wrote the single-value buckets to dst.  Buckets above kChunkCap go to the
 // overflow list (*noverflow entries of {base, count}); hard (one uint32 per
@@ -173,7 +177,7 @@ int launch_listed_sort(int rw, const void* src, void* dst, const LKey& lk, const
 int launch_chunk_sort_small(int rw, const void* src, void* dst, const LKey& lk, const uint32_t* hist,
                             const int64_t* bucket_base, const uint64_t* tables, int64_t tstride, int64_t nbuckets,
                             int64_t* overflow, uint32_t* noverflow, int max_overflow, uint32_t* hard, uint32_t* nhard,
-                            uint32_t* medium, uint32_t* nmedium, long long* checksum, bool eq_done, hipStream_t st,
+                            uint32_t* medium, uint32_t* nmedium, long long* checksum, int eq_done, hipStream_t st,
                             const EntryOut* eo = nullptr, uint32_t ovf_cap = (uint32_t)kChunkCap, bool small = false, hipEvent_t stop = nullptr);
 // n independent segments (the batched sort) in LDS, one workgroup each, by
 // threads x records a thread (segments_lds_cap records at most) -- 0: 1024 x

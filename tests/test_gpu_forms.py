@@ -2,6 +2,7 @@
 type, and the reference's per-rank steps with the merged SecondSort where the
 FirstSort's form is asked for, on the inputs that strain it.  Every result
 is held to the oracle's bytes and counts."""
+import ctypes
 import sys
 
 import numpy
@@ -66,6 +67,37 @@ def test_form_of_wide_records(itemsize, n, form):
     a['key'] >>= 52
     out, st = check_parity(a, ragged(n, 5, 1), ragged(n, 5, 2), 'key', device=True)
     assert st.form == form
+
+
+@pytest.mark.parametrize("itemsize", [8, 16])
+@pytest.mark.parametrize("P", [1, 64])
+def test_one_key_takes_no_longer(itemsize, P):
+    """4,000,000 records of one key, checksum included, against random keys"""
+    n = 4000000
+    c = (ctypes.c_int64 * P)(*even(n, P))
+    key = _lib.KeyDesc(offset=0, width=8, is_signed=0, nwords=1, reserved=0)
+    d, o = lib.mpsort_gpu_dmalloc(n * itemsize), lib.mpsort_gpu_dmalloc(n * itemsize)
+    ms = []
+    try:
+        for k in (keys("random", n, 1), numpy.full(n, 77, numpy.uint64)):
+            a = numpy.zeros((n, itemsize // 8), numpy.uint64)
+            a[:, -1] = numpy.arange(n)
+            a[:, 0] = k
+            _lib.check(lib.mpsort_gpu_memcpy_h2d(d, a.ctypes.data, a.nbytes))
+            t = []
+            for _ in range(5):
+                _lib.check(lib.mpsort_gpu_newarray(d, c, P, o, c, itemsize, ctypes.byref(key), _lib.DEVICE_PTRS))
+                t.append(_lib.last_stats().t_total_ms)
+            ms.append(min(t))
+            assert _lib.last_stats().form == _lib.FORM_ONE_LEVEL
+            out = numpy.empty_like(a)
+            _lib.check(lib.mpsort_gpu_memcpy_d2h(out.ctypes.data, o, a.nbytes))
+            assert numpy.array_equal(out, a[numpy.argsort(a[:, 0], kind='stable')])
+    finally:
+        lib.mpsort_gpu_dfree(d)
+        lib.mpsort_gpu_dfree(o)
+    note("random keys %.3f ms, one key %.3f ms" % tuple(ms))
+    assert ms[1] < 2 * ms[0]
 
 
 @pytest.mark.parametrize("why", ["ranks", "wide key", "4-byte records", "exchange", "radix FirstSort", "bucket FirstSort"])
