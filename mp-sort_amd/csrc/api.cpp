@@ -1657,13 +1657,15 @@ static bool direct_eligible(const CallShape& cs) {
 // all bytes: 8192 records of 256 bytes take 521 us, of 512 bytes 1657, the
 // per-rank form 550 and 557; where the records or their addresses are not
 // whole words it moves single bytes, and 8192 records of 125 bytes take 525 us,
-// of 189 bytes 728, the per-rank form 587 and 613.
+// of 189 bytes 728, the per-rank form 587 and 613.  For one rank that form is
+// one sort, and the line lies at a quarter: 8192 records of 64 bytes 200
+// against 206 us, of 80 bytes 220 against 208, of 31 odd bytes 207 against 209.
 constexpr int64_t kSmallWordBytes = 2 << 20, kSmallByteBytes = 1 << 20;
 static bool small_eligible(const CallShape& cs, const void* in, const void* out) {
     if (!direct_asked(cs) || cs.ntot < 1 || cs.ntot > kSmallRecords || cs.elsize > (1 << 16)) return false;
     if (!cs.general || cs.ntot <= kRankRecords) return true;
     const bool words = ((cs.elsize | (int64_t)(uintptr_t)in | (int64_t)(uintptr_t)out) & 3) == 0;
-    return cs.ntot * cs.elsize <= (words ? kSmallWordBytes : kSmallByteBytes);
+    return cs.ntot * cs.elsize <= (words ? kSmallWordBytes : kSmallByteBytes) / (cs.P > 1 ? 1 : 4);
 }
 
 // the rank tables and the counts' device arrays of the two forms

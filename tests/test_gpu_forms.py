@@ -53,19 +53,22 @@ def test_the_largest_two_level_sort(past, form):
     assert out.sum() == a.sum() and numpy.bitwise_xor.reduce(out) == numpy.bitwise_xor.reduce(a)
 
 
-@pytest.mark.parametrize("itemsize, n, form", [
-    (1024, 4096, _lib.FORM_ONE_LAUNCH), (1024, 4097, _lib.FORM_RANKS), (1024, 8192, _lib.FORM_RANKS),
-    (256, 8192, _lib.FORM_ONE_LAUNCH), (260, 8192, _lib.FORM_RANKS), (128, 8192, _lib.FORM_ONE_LAUNCH),
-    (127, 8192, _lib.FORM_ONE_LAUNCH), (129, 8192, _lib.FORM_RANKS), (1023, 4096, _lib.FORM_ONE_LAUNCH),
-    (1023, 4097, _lib.FORM_RANKS), (65536, 17, _lib.FORM_ONE_LAUNCH)])
-def test_form_of_wide_records(itemsize, n, form):
+@pytest.mark.parametrize("P, itemsize, n, form", [
+    (5, 1024, 4096, _lib.FORM_ONE_LAUNCH), (5, 1024, 4097, _lib.FORM_RANKS), (5, 1024, 8192, _lib.FORM_RANKS),
+    (5, 256, 8192, _lib.FORM_ONE_LAUNCH), (5, 260, 8192, _lib.FORM_RANKS), (5, 128, 8192, _lib.FORM_ONE_LAUNCH),
+    (5, 127, 8192, _lib.FORM_ONE_LAUNCH), (5, 129, 8192, _lib.FORM_RANKS), (5, 1023, 4096, _lib.FORM_ONE_LAUNCH),
+    (5, 1023, 4097, _lib.FORM_RANKS), (5, 65536, 17, _lib.FORM_ONE_LAUNCH),
+    (1, 64, 8192, _lib.FORM_ONE_LAUNCH), (1, 68, 8192, _lib.FORM_RANKS), (1, 31, 8192, _lib.FORM_ONE_LAUNCH),
+    (1, 33, 8192, _lib.FORM_RANKS), (1, 1023, 4096, _lib.FORM_ONE_LAUNCH)])
+def test_form_of_wide_records(P, itemsize, n, form):
     """records of more bytes than one workgroup should move are spread over
-    the chip: both sides of 4096 records and of the bounds in bytes"""
+    the chip: both sides of 4096 records and of the bounds in
+    bytes"""
     dt = numpy.dtype({"names": ["key"], "formats": ["<u8"], "offsets": [itemsize // 2], "itemsize": itemsize})
     g = numpy.random.default_rng(itemsize)
     a = numpy.frombuffer(g.bytes(itemsize * n), dt).copy()
     a['key'] >>= 52
-    out, st = check_parity(a, ragged(n, 5, 1), ragged(n, 5, 2), 'key', device=True)
+    out, st = check_parity(a, ragged(n, P, 1), ragged(n, P, 2), 'key', device=True)
     assert st.form == form
 
 
