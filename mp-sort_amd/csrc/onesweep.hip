@@ -635,7 +635,8 @@ int seg_passes(const SegSortPlan& pl, const SortBuffers& bufs, hipStream_t st, l
     void* Y = bufs.tmp;
     int rc = 0;
     if (k == 0) {
-        if (src != X) return plan_copy(pl, src, X, cs_out, st);
+        // (in place every record is written back as it was, and summed)
+        if (src != X || cs_out) return plan_copy(pl, src, X, cs_out, st);
         return 0;
     }
     const void* cur = src;
