@@ -592,6 +592,8 @@ __device__ __forceinline__ void lds_count_pass(const uint16_t* s_in, uint16_t* s
     __syncthreads();
 }
 
+constexpr uint32_t kIshOwn = 0x80000000u;  // of an interval's shift: its first key has a bin of its own
+
 // Per bucket: single-value buckets already written (eq_done) only add their
 // checksum; oversized ones go to the overflow list; a bucket of one key value
 // is copied.  Otherwise each record gets a bin, non-decreasing in the key:
@@ -602,6 +604,8 @@ __device__ __forceinline__ void lds_count_pass(const uint16_t* s_in, uint16_t* s
 //             into 65 intervals of about equal counts, each cut into SUB bins:
 //             j = #{samples <= key}, [lo, hi] = interval j,
 //             d = SUB j + min(SUB-1, floor(float((key - lo) >> sh_j) * SUB / (((hi - lo) >> sh_j) + 1)))
+//             (the forms below 512 threads: a key sampled more than once has SUB j - 1, a bin of
+//             its own)
 // Records are grouped by bin with LDS atomics (in any order inside a bin),
 // and a record's final slot is its bin start + #{records of the bin with a
 // smaller key, or an equal key and a smaller position}: the stable order.
@@ -737,10 +741,14 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
     using C = BSort<BLOCK, ITEMS>;
     // one-value long bins placed here (the 512 x 6 form hands them on)
     constexpr bool DUPS = BLOCK != 512 || ITEMS >= 9;
+    // a bin of its own for a key sampled more than once: in the forms with few
+    // bins, where it mostly shares one (42% of 500-record segments with half
+    // their records of one key)
+    constexpr bool OWN = BLOCK < 512;
     __shared__ uint64_t s_gkey[C::CAP + 8];  // key of each bin-order slot (+8: unrolled reads)
     __shared__ uint16_t s_sbin[C::CAP];      // bin of each bin-order slot, then the final
                                              // slot of each bucket position (s_pos)
-    __shared__ uint16_t s_ord[C::CAP];       // bucket position of each bin-order slot
+    __shared__ __attribute__((aligned(4))) uint16_t s_ord[C::CAP];  // bucket position of each bin-order slot
     __shared__ uint64_t s_samp[kSamp];    // the sample, in bucket order
     __shared__ uint64_t s_sorted[kSamp];  // the sample, sorted
     __shared__ int s_crowd;
@@ -755,16 +763,16 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
     __shared__ int s_dup;
     __shared__ int s_defer;
     __shared__ uint32_t s_nlong;
+    __shared__ uint16_t s_lstart[DUPS ? C::NL : 1];  // first slots of the one-value long bins
     uint16_t* s_start = reinterpret_cast<uint16_t*>(s_bins);  // NB u16
     uint32_t* s_fill = s_bins + C::NB / 2;                    // NB u16 counters, two per word
     uint16_t* s_pos = s_sbin;
     // one-value long bins; each array reuses LDS that is free by then
-    static_assert(C::NB <= 32 * 2 * kSamp && (C::W + 1) * C::NL <= C::CAP && C::CAP < 0x8000 && C::NB < 0x8000,
+    static_assert(C::NB <= 32 * 2 * kSamp && C::I * C::W * 64 == C::CAP && C::CAP < 0x8000 && C::NB < 0x8000,
                   "aliased arrays of the one-value long bins");
     uint32_t* s_mix = reinterpret_cast<uint32_t*>(s_samp);   // after the sample sort: long bins of several values
     uint16_t* s_lidx = reinterpret_cast<uint16_t*>(s_fill);  // after the ranking: long bin numbers
-    uint16_t* s_wc = s_ord;                 // after the ranking: their records per wave, one item
-    uint16_t* s_run = s_ord + C::W * C::NL;  // and per long bin, the items before
+    uint16_t* s_wc = s_ord;                  // after the ranking: the records of 64 of them per item and wave
     // one more record in bin d: the count before it
     auto bump = [&](uint32_t d) -> uint32_t {
         const uint32_t sh = (d & 1u) << 4;
@@ -884,7 +892,7 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
         const int bits = 64 - __clzll((long long)(span | 1));
         const int sh = bits > 32 ? bits - 32 : 0;
         s_ilo[j] = lo;
-        s_ish[j] = (uint32_t)sh;
+        s_ish[j] = (uint32_t)sh | (OWN && j >= 2 && s_sorted[j - 2] == lo ? kIshOwn : 0u);
         s_isc[j] = (float)C::SUB / ((float)(uint32_t)(span >> sh) + 1.0f);
         // two neighbouring samples in one plain bin put about count / 64
         // records there: the sampled bins are used
@@ -904,10 +912,17 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
         for (int step = kSamp / 2; step > 0; step >>= 1)
             if (s_sorted[j + step - 1] <= key) j += step;
         if (j == kSamp - 1 && s_sorted[kSamp - 1] <= key) j = kSamp;
-        const uint32_t x = (uint32_t)((key - s_ilo[j]) >> s_ish[j]);
+        const uint64_t off = key - s_ilo[j];
+        const uint32_t sh = s_ish[j];
+        const uint32_t x = (uint32_t)(off >> (sh & 63u));
         uint32_t sub = (uint32_t)((float)x * s_isc[j]);
         sub = sub > (uint32_t)(C::SUB - 1) ? (uint32_t)(C::SUB - 1) : sub;
-        return (uint32_t)j * C::SUB + sub;
+        // a key sampled more than once has the last bin of the interval before
+        // its own, which no other key falls in, so that it is placed by
+        // counting: with its neighbours' it made a bin of several values,
+        // ranked record against record (500 records, half of one key: 115 us)
+        const uint32_t own = OWN && off == 0 && (sh & kIshOwn) ? 1u : 0u;
+        return (uint32_t)j * C::SUB + sub - own;
     };
     uint32_t dbin[C::I];
     uint32_t bmax = 0;  // the fullest bin
@@ -1048,69 +1063,66 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
     __syncthreads();
     if (s_long) return 1;
     if (DUPS && s_defer) {
-        // the records of the one-value long bins, item by item (records
-        // k B .. k B + B - 1, wave by wave): slot = bin start + the bin's
-        // records in earlier items + in earlier waves of this item + in
-        // earlier lanes of this wave.  Long bins are numbered first (in any
-        // order).
-        {
-            constexpr int PER = C::NB / C::B;
+        // the records of the one-value long bins.  Records are numbered item
+        // by item, wave by wave (k B + tid), so slot = bin start + the bin's
+        // records in earlier items and waves + in earlier lanes.  Long bins are
+        // numbered first (in any order) and taken 64 at a time: every wave
+        // counts its records of each of them per item (the lanes of a bin
+        // found by a ballot per bit of its number), and one wave, a lane per
+        // bin, makes the counts a prefix.
+        constexpr int PER = C::NB / C::B;
 #pragma unroll
-            for (int j = 0; j < PER; j++) {
-                const int d = tid * PER + j;
-                const bool lg = d < C::FINE && s_start[d + 1] - s_start[d] > (uint32_t)kLongMin;
-                s_lidx[d] = lg ? (uint16_t)atomicAdd(&s_nlong, 1u) : (uint16_t)0xffffu;
-            }
-            for (int q = tid; q < C::W * C::NL; q += C::B) s_wc[q] = 0;
-            for (int q = tid; q < C::NL; q += C::B) s_run[q] = 0;
+        for (int j = 0; j < PER; j++) {
+            const int d = tid * PER + j;
+            const bool lg = d < C::FINE && s_start[d + 1] - s_start[d] > (uint32_t)kLongMin;
+            const uint32_t L = lg ? atomicAdd(&s_nlong, 1u) : 0xffffu;
+            s_lidx[d] = (uint16_t)L;
+            if (lg) s_lstart[L] = s_start[d];
         }
         __syncthreads();
-        for (int k = 0; k < C::I; k++) {
-            const int i = k * C::B + tid;
-            // this wave's records of each long bin in item k (the lanes of
-            // a bin found by ballots, one bin at a time)
-            {
-                const uint32_t sp = i < count ? s_pos[i] : 0u;
-                const bool def = (sp & 0x8000u) != 0;
-                const uint32_t L = def ? s_lidx[sp & 0x7fffu] : 0xffffu;
-                uint64_t act = __ballot(def);
-                while (act) {
-                    const int ld = __builtin_ctzll(act);
-                    const uint32_t Ll = (uint32_t)__builtin_amdgcn_readlane((int)L, ld);
-                    const uint64_t m = __ballot(L == Ll);
-                    if (lane == ld) s_wc[wave * C::NL + Ll] = (uint16_t)__popcll(m);
-                    act &= ~m;
-                }
-            }
+        const uint32_t nlong = s_nlong;
+        for (uint32_t l0 = 0; l0 < nlong; l0 += 64) {
+            for (int q = tid; q < C::CAP / 2; q += C::B) reinterpret_cast<uint32_t*>(s_wc)[q] = 0;
             __syncthreads();
-            {
+            uint32_t mine = 0;  // the items placed in this round
+#pragma unroll 1
+            for (int k = 0; k * C::B < count; k++) {
+                const int i = k * C::B + tid;
                 const uint32_t sp = i < count ? s_pos[i] : 0u;
-                const bool def = (sp & 0x8000u) != 0;
-                const uint32_t d = sp & 0x7fffu;
-                const uint32_t L = def ? s_lidx[d] : 0xffffu;
-                uint32_t before = 0;
-                if (def) {
-                    before = s_start[d] + s_run[L];
-                    for (int w = 0; w < wave; w++) before += s_wc[w * C::NL + L];
-                }
-                uint64_t act = __ballot(def);
-                while (act) {
-                    const int ld = __builtin_ctzll(act);
-                    const uint32_t Ll = (uint32_t)__builtin_amdgcn_readlane((int)L, ld);
-                    const uint64_t m = __ballot(L == Ll);
-                    if (L == Ll) s_pos[i] = (uint16_t)(before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
-                    act &= ~m;
-                }
-            }
-            __syncthreads();
-            for (int q = tid; q < C::NL; q += C::B) {
-                uint32_t acc = 0;
+                const uint32_t L = (sp & 0x8000u) ? s_lidx[sp & 0x7fffu] - l0 : 0xffffu;
+                uint64_t peers = __ballot(L < 64u);
 #pragma unroll
-                for (int w = 0; w < C::W; w++) {
-                    acc += s_wc[w * C::NL + q];
-                    s_wc[w * C::NL + q] = 0;
+                for (int b = 0; b < 6; b++) {
+                    const bool bit = (L >> b) & 1u;
+                    const uint64_t m = __ballot(bit);
+                    peers &= bit ? m : ~m;
                 }
-                s_run[q] = (uint16_t)(s_run[q] + acc);
+                if (L < 64u) {
+                    const uint32_t rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+                    // until the round's end: the bin's number and the lane's rank
+                    s_pos[i] = (uint16_t)((L << 6) | rank);
+                    mine |= 1u << k;
+                    if (rank == 0) s_wc[(k * C::W + wave) * 64 + L] = (uint16_t)__popcll(peers);
+                }
+            }
+            __syncthreads();
+            if (tid < 64) {
+                uint32_t run = l0 + tid < nlong ? s_lstart[l0 + tid] : 0u;
+#pragma unroll 8
+                for (int q = 0; q < C::I * C::W; q++) {
+                    const uint32_t c = s_wc[q * 64 + tid];
+                    s_wc[q * 64 + tid] = (uint16_t)run;
+                    run += c;
+                }
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (int k = 0; k * C::B < count; k++) {
+                if ((mine >> k) & 1u) {
+                    const int i = k * C::B + tid;
+                    const uint32_t v = s_pos[i];
+                    s_pos[i] = (uint16_t)(s_wc[(k * C::W + wave) * 64 + (v >> 6)] + (v & 63u));
+                }
             }
             __syncthreads();
         }
