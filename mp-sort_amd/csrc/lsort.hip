@@ -592,6 +592,11 @@ __device__ __forceinline__ void lds_count_pass(const uint16_t* s_in, uint16_t* s
     __syncthreads();
 }
 
+// the 512 x 6 form hands a bucket on where a bin holds more than this: ranking 64
+// equal keys costs less than a second sort of the bucket (100 segments of
+// 100,000 x 8 B, each value 24 times: 379 us; with 32 records 576, with 256 the
+// same here and 420 instead of 343 on Zipf keys)
+constexpr int kHandOn = 64;
 constexpr uint32_t kIshOwn = 0x80000000u;  // of an interval's shift: its first key has a bin of its own
 
 // Per bucket: single-value buckets already written (eq_done) only add their
@@ -727,20 +732,21 @@ __device__ __forceinline__ void load_items(const WideSrc<RW>& src, const int (&i
 // Sorts one bucket of count (1 .. BSort<BLOCK>::CAP) records, given by src,
 // into dst[base .. base + count) with a BLOCK-thread workgroup.  Returns 0
 // when sorted; otherwise writes nothing and returns 1 when a bin of several
-// key values is crowded beyond kRunMax, 2 when the bucket is for the
-// 1024-thread form (one-value long bins in the 512 x 6 form, see above).
+// key values is crowded beyond kRunMax, 2 when the bucket is for a larger
+// form (HAND: long bins of keys sampled more than once; placing them takes
+// registers that the merged SecondSort's 512 x 6 form does not have).
 // s_bins: BSort<BLOCK, ITEMS>::BW words of LDS owned by the caller, who may
 // keep data there that src reads while loading.  When
 // bounded, every key lies in [lo, hi] (the bucket's boundaries) and the
 // bucket's minimum and maximum are not computed.
-template <int RW, int BLOCK, class Src, int ITEMS = kCItems>
+template <int RW, int BLOCK, class Src, int ITEMS = kCItems, bool HAND = BLOCK == 512 && ITEMS < 9>
 __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restrict__ dst, int64_t base, int count,
                                                 const LKey& lk, uint32_t* s_bins, long long* __restrict__ checksum_out,
                                                 bool bounded = false, uint64_t lo = 0, uint64_t hi = ~0ull,
                                                 const EntryOut eo = EntryOut{}, int ej = 0, int eb = 0) {
     using C = BSort<BLOCK, ITEMS>;
-    // one-value long bins placed here (the 512 x 6 form hands them on)
-    constexpr bool DUPS = BLOCK != 512 || ITEMS >= 9;
+    // one-value long bins placed here, or the bucket handed on (HAND)
+    constexpr bool DUPS = !HAND;
     // a bin of its own for a key sampled more than once: in the forms with few
     // bins, where it mostly shares one (42% of 500-record segments with half
     // their records of one key)
@@ -972,7 +978,7 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
         mode = 1;
     }
     // one-value long bins are looked for when the sample showed a repeated key
-    const bool any_long = s_dup && bmax > (uint32_t)kLongMin;
+    const bool any_long = s_dup && bmax > (uint32_t)(DUPS ? kLongMin : kHandOn);
     if (!DUPS && any_long) return 2;
     // group by bin: key, bin and bucket position of every bin-order slot
 #pragma unroll
@@ -1939,7 +1945,10 @@ __global__ __launch_bounds__(kMergeBlock, 6) void wide_sort_kernel(const uint32_
     }
     const WideSrc<RW> ws = wide_runs<RW, kMergeBlock>(w, b, recs, s_t, s_scan);
     __builtin_assume(cnt <= (uint32_t)C::CAP && cnt > 0u);
-    const int rc = sort_bucket_lds<RW, kMergeBlock, WideSrc<RW>, kMergeItems>(
+    // groups with long bins of one key: 8-byte records place them here, which
+    // saves their second sort (10,000,019 Zipf keys 647 -> 583 us); 16-byte
+    // records have no registers left for it (2^28: 8.78 -> 9.06 ms)
+    const int rc = sort_bucket_lds<RW, kMergeBlock, WideSrc<RW>, kMergeItems, RW == 4>(
         ws, dst, base, (int)cnt, lk, s_bins, checksum_out);
     if (rc && threadIdx.x == 0) {
         if (rc == 2) {

@@ -107,3 +107,14 @@ def test_small_segments_with_a_heavy_key_take_little_longer(dtype, size, count, 
     ms = plan_ms(records(dtype, k, 1), [size] * count)
     note("distinct %.3f ms, %d%% of one key %.3f ms" % (base, 100 * share, ms))
     assert ms < 2.5 * base
+
+
+def test_large_segments_of_repeated_values_take_little_longer():
+    """100 segments of 100,000 x 8 B, each value 24 times: bins of somewhat
+    more than 32 records are no reason to sort a group twice"""
+    size, count = 100000, 100
+    g = numpy.random.default_rng(1)
+    base = plan_ms(records(workloads.REC8, g.integers(0, 1 << 30, size * count), 1), [size] * count)
+    ms = plan_ms(records(workloads.REC8, g.integers(0, 4096, size * count), 1), [size] * count)
+    note("distinct %.3f ms, 4096 values %.3f ms" % (base, ms))
+    assert ms < 2.1 * base
