@@ -1887,7 +1887,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
             (r2 = launch_gather(d_in, n, cs.elsize, dst, rw, cs.iwords, d_out, cs.checksum ? w.checksum + 1 : nullptr,
                                 w.err, st)))
             return r2;
-        if ((r2 = launch_direct_counts(rw, dst, tmp, lk, sh, w, eq_direct, res, c.ev[kEvEnd], st))) return r2;
+        if ((r2 = launch_direct_counts(rw, dst, tmp, lk, sh, w, res, c.ev[kEvEnd], st))) return r2;
         MPSG_CHECK(hipStreamSynchronize(st));
         return 0;
     };

@@ -72,10 +72,10 @@ int launch_direct_sample(int rw, const void* src, const LKey& lk, const DirectSh
 int launch_direct_count(int rw, const void* src, const LKey& lk, const DirectShape& sh, const DirectWork& w,
                         long long* checksum, hipStream_t st);
 // splitters, counts and layout from the sorted records out and the
-// partitioned ones part (eq_done: their single-value buckets went to out
-// instead), and the call's results into res (pinned host memory)
+// partitioned ones part (whose single-value buckets are not read), and the
+// call's results into res (pinned host memory)
 int launch_direct_counts(int rw, const void* out, const void* part, const LKey& lk, const DirectShape& sh,
-                         const DirectWork& w, bool eq_done, DirectResult* res, hipEvent_t stop, hipStream_t st);
+                         const DirectWork& w, DirectResult* res, hipEvent_t stop, hipStream_t st);
 
 // at most kSmallRecords records sorted by one launch, with the splitters,
 // counts and layout (w: C, myclt, mycle, myC, send, split, pminmax, cross,

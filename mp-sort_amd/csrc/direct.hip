@@ -275,7 +275,7 @@ __global__ __launch_bounds__(1024) void direct_scan_kernel(const uint16_t* __res
 template <int RW>
 __global__ __launch_bounds__(1024) void direct_counts_kernel(const uint32_t* __restrict__ out,
                                                              const uint32_t* __restrict__ part, LKey lk, int P,
-                                                             int64_t n, int64_t ntiles, DirectWork w, int eq_done,
+                                                             int64_t n, int64_t ntiles, DirectWork w,
                                                              DirectResult* __restrict__ res) {
     constexpr int BLOCK = 1024, NW = BLOCK / 64, Q = kDirectMaxP / NW;  // splitters (receivers) per wave
     __shared__ uint64_t s_tab[kLBins];
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(1024) void direct_counts_kernel(const uint32_t* __r
                 r1[q] = ob[b];
                 base[q] = w.base[b];
                 lt[q] = le[q] = s_pref[b];
-                if (eq_done && single_bucket(s_tab, b)) {
+                if (single_bucket(s_tab, b)) {  // the splitter's own key alone: not read
                     le[q] += r1[q] - r0[q];
                     r1[q] = r0[q];
                 }
@@ -884,13 +884,12 @@ int launch_direct_count(int rw, const void* src, const LKey& lk, const DirectSha
 }
 
 int launch_direct_counts(int rw, const void* out, const void* part, const LKey& lk, const DirectShape& sh,
-                         const DirectWork& w, bool eq_done, DirectResult* res, hipEvent_t stop, hipStream_t st) {
+                         const DirectWork& w, DirectResult* res, hipEvent_t stop, hipStream_t st) {
     const uint32_t *o = (const uint32_t*)out, *p = (const uint32_t*)part;
     const dim3 g((unsigned)sh.P), b(1024);
-    const int ed = eq_done ? 1 : 0;
     switch (rw) {
-        case 2: hipExtLaunchKernelGGL(direct_counts_kernel<2>, g, b, 0, st, nullptr, stop, 0, o, p, lk, sh.P, sh.n, sh.ntiles, w, ed, res); break;
-        case 4: hipExtLaunchKernelGGL(direct_counts_kernel<4>, g, b, 0, st, nullptr, stop, 0, o, p, lk, sh.P, sh.n, sh.ntiles, w, ed, res); break;
+        case 2: hipExtLaunchKernelGGL(direct_counts_kernel<2>, g, b, 0, st, nullptr, stop, 0, o, p, lk, sh.P, sh.n, sh.ntiles, w, res); break;
+        case 4: hipExtLaunchKernelGGL(direct_counts_kernel<4>, g, b, 0, st, nullptr, stop, 0, o, p, lk, sh.P, sh.n, sh.ntiles, w, res); break;
         default: return -1;
     }
     MPSG_CHECK(hipGetLastError());
