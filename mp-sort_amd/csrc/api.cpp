@@ -1955,7 +1955,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     DirectShape sh;
     direct_shape(cs, nin, nout, kWideTile, &sh);
     sh.W = (int)std::min<int64_t>(kWideBuckets, std::max<int64_t>(2, (n + kWideCoarse - 1) / kWideCoarse));
-    sh.S = M ? kDirectChunk : std::min(kDirectMaxChunks, (32 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
+    sh.S = M ? 0 : std::min(kDirectMaxChunks, (32 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
 
     // ---- workspace
     DirectWork d;

@@ -21,7 +21,7 @@ constexpr int kDirectMaxBuckets = kLBins;
 struct DirectShape {
     int P;
     int W;            // buckets (2 .. kLBins)
-    int S;            // sample keys (a multiple of kDirectChunk)
+    int S;            // sample keys (a multiple of kDirectChunk; 0: no sample)
     int tile;         // records per tile
     int64_t n;
     int64_t ntiles;   // tiles never cross a rank
@@ -63,7 +63,7 @@ struct DirectResult {
 };
 
 // start / stop (here and below, may be null): events of the launch itself
-// sample and its sort (two launches, one when S == kDirectChunk); also writes
+// sample and its sort (two launches, one up to kDirectChunk keys); also writes
 // the tables of the shape and clears the counters (the checksums too when
 // clear_sums)
 int launch_direct_sample(int rw, const void* src, const LKey& lk, const DirectShape& sh, const DirectWork& w,

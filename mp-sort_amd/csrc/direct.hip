@@ -6,6 +6,8 @@
 // (mpsort-mpi.c:369,571-597) produce that same stable order.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
+
 #include "direct.h"
 #include "layout_dev.h"
 #include "lsort_dev.h"
@@ -64,6 +66,7 @@ __global__ __launch_bounds__(kDirectChunk) void direct_sample_kernel(const uint3
         if (tid < 4) w.err[tid] = 0;
         if (tid < 2 && clear_sums) w.checksum[tid] = 0;
     }
+    if (sh.S == 0) return;  // the boundaries come from elsewhere
     const int64_t u = (int64_t)blockIdx.x * kDirectChunk + tid;
     const int64_t pos = (int64_t)sample_pos((uint32_t)u, (uint32_t)sh.S, (uint64_t)sh.n);
     uint32_t r[RW];
@@ -842,7 +845,7 @@ __global__ __launch_bounds__(1024) void small_sort_kernel(const uint32_t* __rest
 int launch_direct_sample(int rw, const void* src, const LKey& lk, const DirectShape& sh, const DirectWork& w,
                          bool clear_sums, hipEvent_t start, hipStream_t st) {
     const uint32_t* s = (const uint32_t*)src;
-    const unsigned g = (unsigned)(sh.S / kDirectChunk);
+    const unsigned g = (unsigned)std::max(1, sh.S / kDirectChunk);
     switch (rw) {
         case 2: hipExtLaunchKernelGGL(direct_sample_kernel<2>, dim3(g), dim3(kDirectChunk), 0, st, start, nullptr, 0, s, lk, sh, w, clear_sums ? 1 : 0); break;
         case 4: hipExtLaunchKernelGGL(direct_sample_kernel<4>, dim3(g), dim3(kDirectChunk), 0, st, start, nullptr, 0, s, lk, sh, w, clear_sums ? 1 : 0); break;
