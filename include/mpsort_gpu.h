@@ -220,11 +220,17 @@ int mpsort_gpu_last_form(void);
  *       the key of one record is flipped between FirstSort and SecondSort
  *       (plain path, more than one rank, key not filling the record), else
  *       the recorded input sum is changed; the call then fails with
- *       MPSORT_ERR_CHECKSUM (unless MPSORT_GPU_NO_CHECKSUM) */
+ *       MPSORT_ERR_CHECKSUM (unless MPSORT_GPU_NO_CHECKSUM)
+ *   MPSORT_GPU_FAULT_KEEP_FORM   with the other hooks, calls keep the form
+ *       that they take without them instead of MPSORT_GPU_FORM_RANKS;
+ *       BUCKET_CAP then also applies to the plain path's buckets, CORRUPT flips
+ *       its byte between two steps of the partition, and SPLITTERS and PLAIN
+ *       have nothing to change there */
 #define MPSORT_GPU_FAULT_SPLITTERS (1u << 0)
 #define MPSORT_GPU_FAULT_BUCKET_CAP (1u << 1)
 #define MPSORT_GPU_FAULT_PLAIN (1u << 2)
 #define MPSORT_GPU_FAULT_CORRUPT (1u << 3)
+#define MPSORT_GPU_FAULT_KEEP_FORM (1u << 4)
 int mpsort_gpu_set_faults(unsigned faults, int64_t bucket_cap);
 
 /* Prints the phase times of the last call in the reference's format

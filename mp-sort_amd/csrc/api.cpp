@@ -1652,7 +1652,8 @@ constexpr int64_t kDirectAvg = 2048;   // records per bucket while kLBins bucket
 constexpr int kDirectKeys = 16, kDirectManyKeys = 20;
 constexpr int64_t kDirectMany = (int64_t)kLBins * 3500;
 static bool direct_asked(const CallShape& cs) {
-    return !g_faults && !cs.exchange && cs.first_mode == 0 && cs.P <= kDirectMaxP && cs.ks.key_bytes <= 8;
+    return (!g_faults || (g_faults & MPSORT_GPU_FAULT_KEEP_FORM)) && !cs.exchange && cs.first_mode == 0 &&
+           cs.P <= kDirectMaxP && cs.ks.key_bytes <= 8;
 }
 static bool direct_eligible(const CallShape& cs) {
     return direct_asked(cs) && (cs.rw == 2 || cs.rw == 4) && cs.ntot > kSmallRecords && cs.ntot <= kDirectMaxRecords;
@@ -1772,7 +1773,8 @@ static int run_small(DevCtx& c, const CallShape& cs, const void* d_in, void* d_o
                                 cs.key_bytes_user, sh, w, cs.checksum, apart, res, c.ev[kEvStart], c.ev[kEvEnd], c.st)))
         return rc;
     MPSG_CHECK(hipStreamSynchronize(c.st));
-    const DirectResult got = *res;
+    DirectResult got = *res;
+    if (g_faults & MPSORT_GPU_FAULT_CORRUPT) got.sums[0]++;
     stats->first_passes = (int32_t)got.lists[3];
     stats->t_first_sort_ms = stats->t_total_ms = ev_ms(c.ev[kEvStart], c.ev[kEvEnd]);
     return direct_results(c, cs, w, got, false, MPSORT_GPU_FORM_ONE_LAUNCH, stats);
@@ -1847,10 +1849,14 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     long long* cs_in = cs_direct ? w.checksum : nullptr;
     long long* cs_out = cs_direct ? w.checksum + 1 : nullptr;
     void* tmp = c.s1.p;
+    // the corruption fault hook changes the last byte of a scattered record,
+    // else the recorded input sum
+    const bool corrupt = (g_faults & MPSORT_GPU_FAULT_CORRUPT) != 0;
+    const bool corrupt_record = corrupt && !cs.general && cs.ks.key_off + cs.ks.key_bytes < rw * 4;
     // single-value buckets go straight to the output unless it overlaps the
     // records still to be read
     const char *sa = (const char*)src, *da = (const char*)dst;
-    const bool eq_direct = sa >= da + (size_t)n * recbytes || da >= sa + (size_t)n * recbytes;
+    const bool eq_direct = !corrupt_record && (sa >= da + (size_t)n * recbytes || da >= sa + (size_t)n * recbytes);
     hipEvent_t* pe = cs.timing ? c.pass_ev[0] : nullptr;
     auto mark = [&](int i) -> int {
         if (pe) MPSG_CHECK(hipEventRecord(pe[i], st));
@@ -1862,10 +1868,10 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         (rc = mark(1)) || (rc = launch_direct_count(rw, src, lk, sh, w, cs_in, st)) || (rc = mark(2)) ||
         (rc = launch_lscatter(rw, src, tmp, eq_direct ? dst : tmp, sd, sh.ntiles, w.bkt, w.tables, 0, w.tile_off,
                               w.err + 1, st, w.tot, n, w.base, cs_out)) ||
-        (rc = mark(3)) ||
+        (corrupt_record && (rc = launch_fault_corrupt((char*)tmp + recbytes - 1, nullptr, st))) || (rc = mark(3)) ||
         (rc = launch_chunk_sort_small(rw, tmp, dst, lk, w.tot, w.base, w.tables, 0, sh.W, w.overflow, w.lists, kLBins,
                                       w.hard, w.lists + 1, w.medium, w.lists + 2, cs_out, eq_direct ? kEqSummed : kEqNone, st, nullptr,
-                                      (uint32_t)kChunkCap, small_form, c.ev[kEvFirst])) ||
+                                      fault_cap(), small_form, c.ev[kEvFirst])) ||
         (rc = mark(4)))
         return rc;
     // The buckets above 4608 records (lists[2]) and the crowded ones: enqueued
@@ -1919,6 +1925,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         got = *res;
     }
 
+    if (corrupt && !corrupt_record) got.sums[0]++;
     stats->buckets = sh.W;
     stats->buckets_overflow = stats->buckets_overflow_first = (int32_t)got.lists[0];
     stats->buckets_lds_radix = (int32_t)got.lists[1];
@@ -1973,7 +1980,8 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     w.nfine = n / w.avg + w.W;
     w.ngrid = wide_grid(n, w.W);
     w.ncopy = n / kWideCopy + w.nfine;
-    w.max_overflow = (int)(n / kChunkCap + 1);
+    w.cap = fault_cap();
+    w.max_overflow = (int)std::min<int64_t>(n / w.cap + 1, w.nfine);
     uint64_t* prop = nullptr;
     auto lay = [&](auto& a, auto take) {
         take(a, d.begin, (size_t)P);
@@ -2055,7 +2063,11 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
             (rc = launch_model_proposals(md, d.C, n, P, prop, st)))
             return rc;
     }
-    if ((rc = mark(1)) || (rc = launch_wide_level1(rw, src, a, lk, sd, w, cs_in, st)) || (rc = mark(2)) ||
+    // (the corruption fault hook, as in run_direct)
+    const bool corrupt = (g_faults & MPSORT_GPU_FAULT_CORRUPT) != 0;
+    const bool corrupt_record = corrupt && !cs.general && cs.ks.key_off + cs.ks.key_bytes < rw * 4;
+    if ((rc = mark(1)) || (rc = launch_wide_level1(rw, src, a, lk, sd, w, cs_in, st)) ||
+        (corrupt_record && (rc = launch_fault_corrupt((char*)a + rw * 4 - 1, nullptr, st))) || (rc = mark(2)) ||
         (rc = launch_wide_level2(rw, a, b, dst, lk, w, cs_out, st)) || (rc = mark(3)) ||
         (rc = launch_wide_sort(rw, b, dst, lk, w, cs_out, st)) || (rc = mark(4)))
         return rc;
@@ -2101,6 +2113,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         got = *res;
     }
 
+    if (corrupt && !corrupt_record) got.sums[0]++;
     stats->buckets = (int32_t)got.buckets;
     stats->buckets_overflow = stats->buckets_overflow_first = (int32_t)got.lists[0];
     stats->buckets_lds_radix = (int32_t)got.lists[1];
@@ -2578,6 +2591,7 @@ static int seg_group_wide(SegGroup& G, const std::vector<int64_t>& cnt, const st
     w.nt2 = ctile[n];
     w.ngrid = wide_grid(w.n, w.W);
     w.ncopy = w.n / kWideCopy + w.nfine;
+    w.cap = (uint32_t)kChunkCap;
     w.max_overflow = (int)(w.n / kChunkCap + 1);
     uint32_t* d_tile_c = nullptr;
     auto lay = [&](auto& a, auto take) {
@@ -3501,7 +3515,7 @@ static void parse_env_options(void) {
 }
 int mpsort_gpu_set_faults(unsigned faults, int64_t bucket_cap) {
     const unsigned known = MPSORT_GPU_FAULT_SPLITTERS | MPSORT_GPU_FAULT_BUCKET_CAP | MPSORT_GPU_FAULT_PLAIN |
-                           MPSORT_GPU_FAULT_CORRUPT;
+                           MPSORT_GPU_FAULT_CORRUPT | MPSORT_GPU_FAULT_KEEP_FORM;
     if (faults & ~known) return fail(MPSORT_ERR_ARG, "unknown fault bits 0x%x", faults & ~known);
     if ((faults & MPSORT_GPU_FAULT_BUCKET_CAP) && (bucket_cap < 1 || bucket_cap > kChunkCap))
         return fail(MPSORT_ERR_ARG, "bucket_cap %lld outside [1, %d]", (long long)bucket_cap, kChunkCap);

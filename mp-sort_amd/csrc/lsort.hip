@@ -1938,7 +1938,7 @@ __global__ __launch_bounds__(kMergeBlock, 6) void wide_sort_kernel(const uint32_
     const uint32_t cnt = w.fcnt[id];
     const int64_t base = w.fbase[id];
     const WideBucket b = w.desc[id];
-    if (cnt == 0 || cnt > (uint32_t)kChunkCap) return;
+    if (cnt == 0 || cnt > w.cap) return;
     if (cnt > (uint32_t)C::CAP) {
         if (threadIdx.x == 0) w.medium[atomicAdd(&w.lists[2], 1u)] = id;
         return;
@@ -2040,7 +2040,7 @@ __global__ __launch_bounds__(kMergeBlock) void wide_copy_kernel(const uint32_t* 
             const int i = (int)task.y + k * kMergeBlock + (int)threadIdx.x;
             if (i < cnt) {
                 RecIO<RW>::store(dst, base + i, r[k]);
-                if (checksum_out && cnt > kChunkCap) {
+                if (checksum_out && cnt > (int)w.cap) {
 #pragma unroll
                     for (int v = 0; v < RW; v++) csum += sbyte_sum(r[k][v]);
                 }

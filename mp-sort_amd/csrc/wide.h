@@ -40,6 +40,7 @@ struct WideWork {
     int64_t n, nt, ntpad;      // records, level 1 tiles, entries of a row of off and loc
     int64_t nt2, nfine;        // level 2 tiles and fine buckets, at most
     int64_t ngrid;             // groups sorted by one workgroup each (wide_grid); those past it are listed
+    uint32_t cap;              // largest group sorted in LDS (kChunkCap, less by the capacity fault hook)
     const uint64_t* raw;       // W - 1 sample keys at the coarse boundaries
     uint64_t* tables;          // kWideBuckets coarse boundaries
     uint64_t* tables2;         // W rows of kWideBuckets fine boundaries

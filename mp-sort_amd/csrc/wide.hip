@@ -511,7 +511,8 @@ __global__ __launch_bounds__(kWideBuckets) void wide_fine_kernel(WideWork w) {
     }
     const uint32_t pre = scan_block<kWideBuckets>(sum, s_tmp);
     const bool single = f < nw && wide_single(w.tables2 + (int64_t)c * kWideBuckets, f, nw - 1);
-    const bool alone = sum > (uint32_t)kWideCap || (single && sum > kWideAlone);
+    const uint32_t most = min((uint32_t)kWideCap, w.cap);  // records of a group of several
+    const bool alone = sum > most || (single && sum > kWideAlone);
     const uint64_t am = __ballot(alone);
     if (lane == 0) s_alone[wave] = am;
     s_pref[f] = pre;
@@ -533,11 +534,11 @@ __global__ __launch_bounds__(kWideBuckets) void wide_fine_kernel(WideWork w) {
                 break;
             }
         }
-        // the largest fe <= stop with pref[fe] - pref[f] <= kWideCap
+        // the largest fe <= stop with pref[fe] - pref[f] <= most
         int lo = f + 1, hi = stop;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
-            if (s_pref[mid] - pre <= (uint32_t)kWideCap) lo = mid; else hi = mid - 1;
+            if (s_pref[mid] - pre <= most) lo = mid; else hi = mid - 1;
         }
         fe = lo;
     }
@@ -563,8 +564,8 @@ __global__ __launch_bounds__(kWideBuckets) void wide_fine_kernel(WideWork w) {
     w.fbase[id] = base;
     w.desc[id] = WideBucket{t0, w.cbase[c], (uint16_t)nt, (uint16_t)f, (uint16_t)fe, 0};
     // (many one-value groups) sorted with the listed ones
-    if (id >= (uint32_t)w.ngrid && cnt <= (uint32_t)kChunkCap) w.medium[atomicAdd(&w.lists[2], 1u)] = id;
-    if (cnt > (uint32_t)kChunkCap) {
+    if (id >= (uint32_t)w.ngrid && cnt <= w.cap) w.medium[atomicAdd(&w.lists[2], 1u)] = id;
+    if (cnt > w.cap) {
         if (!single) {
             const uint32_t slot = atomicAdd(&w.lists[0], 1u);
             if ((int)slot < w.max_overflow) {

@@ -38,6 +38,7 @@ FAULT_SPLITTERS = 1 << 0
 FAULT_BUCKET_CAP = 1 << 1
 FAULT_PLAIN = 1 << 2
 FAULT_CORRUPT = 1 << 3
+FAULT_KEEP_FORM = 1 << 4
 
 # mpsort.h:17-20
 MPSORT_DISABLE_SPARSE_ALLTOALLV = 1 << 1
