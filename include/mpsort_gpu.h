@@ -309,14 +309,18 @@ int mpsort_gpu_newarray_learned(const void *base, const int64_t *nin, int P, voi
  * threshold, then the workgroup shape of the in-LDS segments (the waves that
  * share a CU), on the first run and caches the choice per (record size, key
  * width, size class) in memory and in $MPSORT_GPU_TUNE_CACHE (default
- * ~/.cache/mpsort_gpu_segsort.tune). */
+ * ~/.cache/mpsort_gpu_segsort.tune; choices made for other plans, by another
+ * version of the library, are not read). */
 typedef struct mpsort_gpu_segplan_s mpsort_gpu_segplan;
 #define MPSORT_GPU_SEGPLAN_GRAPH (1u << 0)
 #define MPSORT_GPU_SEGPLAN_TUNE (1u << 1)
-/* the workgroup shape of the segments sorted in LDS when not tuned (default:
- * 1024 threads x 9 records, one workgroup per CU): 512 x 9 (two per CU,
- * segments up to 4608 records) or 512 x 6 (three per CU, up to 3072); larger
- * ones below the threshold take the 1024-thread form */
+/* The workgroup shape of the segments sorted in LDS when not tuned.  Segments
+ * of at most 768 and 1536 records take workgroups of 128 and 256 threads x 6
+ * records (eleven and six per CU); the shape chosen takes those up to its
+ * capacity -- 512 threads x 9 records (the default; two per CU, up to 4608
+ * records) or 512 x 6 (three per CU, up to 3072) -- and 1024 threads x 9 records
+ * the larger ones.  With MPSORT_GPU_SEGPLAN_EACH the default is 1024 x 9 for
+ * all, and a shape chosen takes all up to its capacity. */
 #define MPSORT_GPU_SEGPLAN_SMALL_512x9 (1u << 2)
 #define MPSORT_GPU_SEGPLAN_SMALL_512x6 (1u << 3)
 /* every segment sorted by launches of its own, one segment after the other
@@ -329,11 +333,13 @@ int mpsort_gpu_segplan_add(mpsort_gpu_segplan *plan, const void *d_in, void *d_o
                            int nseg, size_t elsize, const mpsort_key_desc *key);
 /* stats (may be NULL): t_total_ms and nrecords are filled */
 int mpsort_gpu_segplan_run(mpsort_gpu_segplan *plan, mpsort_gpu_stats *stats);
-/* the tuning a group runs with: segments sorted in LDS / by onesweep, tile */
+/* the tuning a group runs with: segments sorted in LDS, and larger ones (by a
+ * partition level up to 943,616 records of 8 or 16 bytes, else by onesweep), tile */
 int mpsort_gpu_segplan_info(const mpsort_gpu_segplan *plan, int group, int *nsmall, int *nlarge, int *block,
                             int *items, int *threshold);
-/* the workgroup shape of a group's in-LDS segments (0: 1024 x 9, 1: 512 x 9,
- * 2: 512 x 6) and the waves that then share a CU */
+/* the workgroup shape of a group's in-LDS segments (0: the default, 1: 512 x 9,
+ * 2: 512 x 6, see MPSORT_GPU_SEGPLAN_SMALL_512x9) and the waves of the shape that
+ * then share a CU */
 int mpsort_gpu_segplan_shape(const mpsort_gpu_segplan *plan, int group, int *form, int *waves_per_cu);
 int mpsort_gpu_segplan_free(mpsort_gpu_segplan *plan);
 /* one group, no graph: create + add + run + free */

@@ -2458,14 +2458,15 @@ using namespace mpsg;
 // Thousands of independent stable sorts of one record type, segments back to
 // back in one buffer.  Segments of at most `threshold` records are sorted by
 // one workgroup each in LDS (the bucket-sort kernels of the learned path, with
-// the segment as the bucket); the larger ones by the segmented onesweep over
-// just those segments.  Every launch of a group depends only on device data,
+// the segment as the bucket); the larger ones by one partition level (wide.hip)
+// or the segmented onesweep over just those segments.  Every launch of a group depends only on device data,
 // so the whole batch can be captured once in a hipGraph and replayed.
-// tile: the onesweep tile of the large segments; threshold: the largest
-// segment sorted in LDS; form: the workgroup shape of those, which sets how
-// many share a CU (0: 1024 x 9, one per CU, 16 waves; 1: 512 x 9, two per
-// CU, 16 waves; 2: 512 x 6, three per CU, 24 waves), the segments above its
-// capacity going to the 1024-thread form
+// tile: the tile of the onesweep; threshold: the largest segment sorted in LDS;
+// form: the workgroup shape of those above 1536 records up to its capacity, which
+// sets how many share a CU (0, 1: 512 x 9, two per CU, 16 waves; 2: 512 x 6, three
+// per CU, 24 waves).  Smaller ones take 128 and 256 threads, larger ones 1024 x 9.
+// One segment at a time (each), the form takes all up to its capacity, and 0 is
+// 1024 x 9.
 struct SegTune {
     TileCfg tile;
     int threshold;
@@ -2514,6 +2515,11 @@ static std::map<std::string, SegTune>& seg_tune_cache() {
     return m;
 }
 
+// Tuned choices hold for one set of plans: this number goes up when a group's
+// segments are sorted by other kernels, and choices of another are not read
+// (2: the partition level and the workgroup sizes by segment).
+constexpr int kSegPlans = 2;
+
 // size class: log2 of the median segment length
 static std::string seg_tune_key(const SegGroup& G) {
     std::vector<int64_t> c(G.count);
@@ -2522,7 +2528,7 @@ static std::string seg_tune_key(const SegGroup& G) {
     int cls = 0;
     while ((int64_t(1) << (cls + 1)) <= med) cls++;
     char k[96];
-    snprintf(k, sizeof k, "rw=%d keybytes=%d class=%d", G.rw, G.ks.key_bytes, cls);
+    snprintf(k, sizeof k, "plans=%d rw=%d keybytes=%d class=%d", kSegPlans, G.rw, G.ks.key_bytes, cls);
     return k;
 }
 
@@ -2543,12 +2549,12 @@ static void seg_tune_load() {
     if (!fp) return;
     char line[256];
     while (fgets(line, sizeof line, fp)) {
-        int rw, kb, cls, blk, items, thr, form = 0;
-        const int got = sscanf(line, "rw=%d keybytes=%d class=%d block=%d items=%d threshold=%d form=%d", &rw, &kb,
-                               &cls, &blk, &items, &thr, &form);
-        if (got >= 6) {
+        int plans, rw, kb, cls, blk, items, thr, form = 0;
+        const int got = sscanf(line, "plans=%d rw=%d keybytes=%d class=%d block=%d items=%d threshold=%d form=%d",
+                               &plans, &rw, &kb, &cls, &blk, &items, &thr, &form);
+        if (got >= 7 && plans == kSegPlans) {
             char k[96];
-            snprintf(k, sizeof k, "rw=%d keybytes=%d class=%d", rw, kb, cls);
+            snprintf(k, sizeof k, "plans=%d rw=%d keybytes=%d class=%d", plans, rw, kb, cls);
             SegTune t{{blk, items}, thr, form};
             if (tile_supported(rw, t.tile) && thr >= 0 && thr <= kChunkCap && form >= 0 && form <= 2)
                 seg_tune_cache()[k] = t;
@@ -2954,10 +2960,11 @@ static int seg_group_tune(SegGroup& G, DevCtx& c) {
         }
     }
     // then the workgroup shape of the segments sorted in LDS (how many
-    // workgroups and waves share a CU), with that tile and threshold
+    // workgroups and waves share a CU), with that tile and threshold (shapes
+    // 0 and 1 make one plan, except one segment at a time)
     const bool lds_ok = (G.rw == 2 || G.rw == 4) && G.ks.key_bytes <= 8;
     if (lds_ok && pick.threshold > 0) {
-        for (int form = 1; form <= 2; form++) {
+        for (int form = G.each ? 1 : 2; form <= 2; form++) {
             G.tune = SegTune{pick.tile, pick.threshold, form};
             if ((rc = seg_group_prepare(G, c.st))) return rc;
             if (!G.nsmall) break;

@@ -17,9 +17,12 @@ class SegmentPlan(object):
     segments back to back.  ``graph=True`` captures the whole plan in a
     hipGraph on the first run and replays it afterwards; ``tune=True`` picks
     the tile shape, the in-LDS threshold and the workgroup shape of the
-    in-LDS segments by timing them on the first run.  ``small_form`` sets that
-    shape without tuning: 0 (1024 threads x 9 records, one workgroup per CU),
-    1 (512 x 9, two per CU) or 2 (512 x 6, three per CU)."""
+    in-LDS segments by timing them on the first run.  ``small_form`` sets the
+    shape of the segments above 1536 records without tuning: 0 and 1 (512
+    threads x 9 records, two workgroups per CU) or 2 (512 x 6, three per CU);
+    smaller segments take workgroups of 128 and 256 threads, those above the
+    shape's capacity 1024.  With ``each=True`` the shape takes all segments up
+    to its capacity, and 0 is 1024 threads x 9 records."""
 
     def __init__(self, graph=False, tune=False, small_form=0, each=False):
         flags = (_lib.SEGPLAN_GRAPH if graph else 0) | (_lib.SEGPLAN_TUNE if tune else 0)
