@@ -1639,7 +1639,8 @@ static int plain_bucket_first(DevCtx& c, const CallShape& cs, const SegSortPlan&
 // ---- the sort without per-rank local sorts (direct.hip) ----------------------
 // Taken by the allocating plain path when nothing asks for another form (an
 // exchange, a FirstSort form, a fault hook): up to kDirectMaxP ranks, 8- or
-// 16-byte sort records with keys of at most 8 bytes.  One partition pass has
+// 16-byte sort records with keys of at most 8 bytes (4-byte records, bare keys,
+// have no kernels in these forms and keep the per-rank one).  One partition pass has
 // at most kLBins buckets, each at most about the in-LDS capacity of 4608
 // records: kDirectMaxRecords.
 constexpr int64_t kDirectMaxRecords = (int64_t)kLBins * 4200;
@@ -1794,7 +1795,6 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     sh.W = (int)std::min<int64_t>(kLBins, std::max<int64_t>(2, (n + kDirectAvg - 1) / kDirectAvg));
     const int keys = n > kDirectMany ? kDirectManyKeys : kDirectKeys;
     sh.S = std::min(kDirectMaxChunks, (keys * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
-    const bool small_form = false;
 
     // ---- workspace
     DirectWork w;
@@ -1871,7 +1871,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         (corrupt_record && (rc = launch_fault_corrupt((char*)tmp + recbytes - 1, nullptr, st))) || (rc = mark(3)) ||
         (rc = launch_chunk_sort_small(rw, tmp, dst, lk, w.tot, w.base, w.tables, 0, sh.W, w.overflow, w.lists, kLBins,
                                       w.hard, w.lists + 1, w.medium, w.lists + 2, cs_out, eq_direct ? kEqSummed : kEqNone, st, nullptr,
-                                      fault_cap(), small_form, c.ev[kEvFirst])) ||
+                                      fault_cap(), c.ev[kEvFirst])) ||
         (rc = mark(4)))
         return rc;
     // The buckets above 4608 records (lists[2]) and the crowded ones: enqueued
@@ -1951,7 +1951,7 @@ static bool wide_eligible(const CallShape& cs) {
 // *again: nothing was written, the call takes another path (the sample, or the
 // model, missed the sizes of the coarse buckets by far, or memory is short)
 static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_out, const int64_t* nin,
-                    const int64_t* nout, const void* packed_host, mpsort_gpu_stats* stats, bool* again,
+                    const int64_t* nout, mpsort_gpu_stats* stats, bool* again,
                     const LearnedModel* M = nullptr) {
     hipStream_t st = c.st;
     const int P = cs.P, rw = cs.rw;
@@ -2033,13 +2033,10 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         MPSG_CHECK(hipEventRecord(c.ev[kEvStart], st));
         src = c.rbuf.p;
         dst = c.s0.p;
-        if (packed_host) {
-            MPSG_CHECK(hipMemcpyAsync(c.rbuf.p, packed_host, bytes, hipMemcpyHostToDevice, st));
-        } else if ((rc = launch_fill_u32((uint32_t*)d.checksum, 0u, 4, st)) ||
-                   (rc = launch_pack(d_in, n, cs.elsize, cs.key_off_user, cs.key_bytes_user, c.rbuf.p, rw, cs.iwords,
-                                     cs.checksum ? d.checksum : nullptr, st))) {
+        if ((rc = launch_fill_u32((uint32_t*)d.checksum, 0u, 4, st)) ||
+            (rc = launch_pack(d_in, n, cs.elsize, cs.key_off_user, cs.key_bytes_user, c.rbuf.p, rw, cs.iwords,
+                              cs.checksum ? d.checksum : nullptr, st)))
             return rc;
-        }
     }
     const bool cs_direct = cs.checksum && !cs.general;
     long long* cs_in = cs_direct ? d.checksum : nullptr;
@@ -2052,7 +2049,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
     };
     const SegDev sd{d.begin, d.count, d.tile_start, P, 0};
     if ((rc = mark(0)) ||
-        (rc = launch_direct_sample(rw, src, lk, sh, d, !(cs.general && !packed_host),
+        (rc = launch_direct_sample(rw, src, lk, sh, d, !cs.general,
                                    cs.general ? nullptr : c.ev[kEvStart], st)))
         return rc;
     if (M) {
@@ -2130,7 +2127,7 @@ static int run_wide(DevCtx& c, const CallShape& cs, const void* d_in, void* d_ou
         stats->splitters_exact = P > 1 ? (int32_t)got.exact : 0;
         stats->splitters_repaired = P > 1 ? P - 1 - stats->splitters_exact : 0;
     }
-    return direct_results(c, cs, d, got, packed_host != nullptr, MPSORT_GPU_FORM_TWO_LEVELS, stats);
+    return direct_results(c, cs, d, got, false, MPSORT_GPU_FORM_TWO_LEVELS, stats);
 }
 
 // The learned path by two partition levels: per-rank bucket sorts, bounds and
@@ -3075,8 +3072,10 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
     if (!cs.general && cs.rw == 8 && cs.ks.key_bytes <= 8 && !cs.exchange && cs.first_mode != 1 &&
         ntot >= kFirstMinAvg * P) {
         // 32-byte records of large ranks: sorted as packed {key, index}
-        // records, so that the bucket FirstSort and the merged SecondSort
-        // take them (a quarter of the radix passes' traffic, gather included)
+        // records (a quarter of the radix passes' traffic, gather included).
+        // The line at 2^18 records a rank is the bucket FirstSort's; the one-
+        // and two-level forms do not need it, but calls of smaller ranks have
+        // not been measured in them and keep the per-rank form.
         if ((rc = shape_for(key, elsize, flags | MPSORT_GPU_FORCE_GENERAL, devptr ? base : nullptr,
                             devptr ? out : nullptr, ntot, &cs)))
             return rc;
@@ -3096,7 +3095,7 @@ int mpsort_gpu_newarray(const void* base, const int64_t* nin, int P, void* out, 
         if (one || wide_eligible(cs)) {
             bool again = false;
             r2 = one ? run_direct(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again)
-                     : run_wide(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again);
+                     : run_wide(*c, cs, d_in, d_out, nin, nout, &st, &again);
             if (r2 || !again) return r2;
         }
         HistWork w;
@@ -3948,7 +3947,7 @@ int mpsort_gpu_newarray_learned(const void* base, const int64_t* nin, int P, voi
     rc = staged_call(c, cs, base, out, devptr, P, &st, [&](const void* d_in, void* d_out) {
         if (learned_wide_eligible(cs)) {
             bool again = false;
-            const int r2 = run_wide(*c, cs, d_in, d_out, nin, nout, nullptr, &st, &again, &model->m);
+            const int r2 = run_wide(*c, cs, d_in, d_out, nin, nout, &st, &again, &model->m);
             if (r2 || !again) return r2;
         }
         return run_histsort_learned(*c, cs, d_in, d_out, nin, nout, model->m, &st);

@@ -15,7 +15,6 @@ constexpr int kSmallRecords = 8192;     // sorted by one launch
 constexpr int kRankRecords = 4096;      // of those, by counting every record's rank
 constexpr int kDirectChunk = 1024;      // sample keys sorted by one workgroup
 constexpr int kDirectMaxChunks = 20;    // sample chunks
-constexpr int kDirectMaxBuckets = kLBins;
 
 // the host tables of one call, passed by value (no upload)
 struct DirectShape {

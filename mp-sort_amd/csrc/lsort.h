@@ -170,15 +170,15 @@ int launch_listed_sort(int rw, const void* src, void* dst, const LKey& lk, const
                        const uint32_t* hist, const int64_t* bucket_base, const uint64_t* tables, int nbins,
                        int64_t tstride, uint32_t* hard, uint32_t* nhard, long long* checksum, hipStream_t st,
                        const EntryOut* eo = nullptr, const uint32_t* d_nlist = nullptr);
-// launch_chunk_sort with 512-thread workgroups: two per CU, or with small
-// three (buckets up to kMergeCap records); larger buckets (up to kChunkCap)
-// are listed in medium (*nmedium entries) for launch_listed_sort; no LDS
-// radix pass is launched
+// launch_chunk_sort with 512-thread workgroups, two per CU: buckets above
+// 4608 records (up to kChunkCap) are listed in medium (*nmedium entries) for
+// launch_listed_sort; no LDS radix pass is launched.  stop (may be null): an
+// event of the launch itself
 int launch_chunk_sort_small(int rw, const void* src, void* dst, const LKey& lk, const uint32_t* hist,
                             const int64_t* bucket_base, const uint64_t* tables, int64_t tstride, int64_t nbuckets,
                             int64_t* overflow, uint32_t* noverflow, int max_overflow, uint32_t* hard, uint32_t* nhard,
                             uint32_t* medium, uint32_t* nmedium, long long* checksum, int eq_done, hipStream_t st,
-                            const EntryOut* eo = nullptr, uint32_t ovf_cap = (uint32_t)kChunkCap, bool small = false, hipEvent_t stop = nullptr);
+                            const EntryOut* eo = nullptr, uint32_t ovf_cap = (uint32_t)kChunkCap, hipEvent_t stop = nullptr);
 // n independent segments (the batched sort) in LDS, one workgroup each, by
 // threads x records a thread (segments_lds_cap records at most) -- 0: 1024 x
 // 9 (one workgroup per CU), 1: 512 x 9 (two per CU), 2: 512 x 6 (three per

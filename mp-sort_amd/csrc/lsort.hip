@@ -2450,21 +2450,19 @@ int launch_chunk_sort_small(int rw, const void* src, void* dst, const LKey& lk, 
                             const int64_t* bucket_base, const uint64_t* tables, int64_t tstride, int64_t nbuckets,
                             int64_t* overflow, uint32_t* noverflow, int max_overflow, uint32_t* hard, uint32_t* nhard,
                             uint32_t* medium, uint32_t* nmedium, long long* checksum, int eq_done, hipStream_t st,
-                            const EntryOut* eop, uint32_t ovf_cap, bool small, hipEvent_t stop) {
+                            const EntryOut* eop, uint32_t ovf_cap, hipEvent_t stop) {
     if (nbuckets <= 0) return 0;
     const EntryOut eo = eop ? *eop : EntryOut{};
     const uint32_t* s = (const uint32_t*)src;
     uint32_t* d = (uint32_t*)dst;
     const unsigned grid = (unsigned)nbuckets;
-#define MPSG_CHUNKFORM(R, I) \
-    hipExtLaunchKernelGGL((interp_sort_kernel<R, kMergeBlock, I>), dim3(grid), dim3(kMergeBlock), 0, st, nullptr, stop, 0, s, d, lk, hist, \
-                       bucket_base, tables, tstride, nbuckets, overflow, noverflow, max_overflow, hard, nhard, medium, \
-                       nmedium, checksum, eq_done, eo, ovf_cap)
-    switch (rw * 2 + (small ? 1 : 0)) {
-        case 4: MPSG_CHUNKFORM(2, kSmallItems); break;
-        case 5: MPSG_CHUNKFORM(2, kMergeItems); break;
-        case 8: MPSG_CHUNKFORM(4, kSmallItems); break;
-        case 9: MPSG_CHUNKFORM(4, kMergeItems); break;
+#define MPSG_CHUNKFORM(R) \
+    hipExtLaunchKernelGGL((interp_sort_kernel<R, kMergeBlock, kSmallItems>), dim3(grid), dim3(kMergeBlock), 0, st, \
+                          nullptr, stop, 0, s, d, lk, hist, bucket_base, tables, tstride, nbuckets, overflow, noverflow, \
+                          max_overflow, hard, nhard, medium, nmedium, checksum, eq_done, eo, ovf_cap)
+    switch (rw) {
+        case 2: MPSG_CHUNKFORM(2); break;
+        case 4: MPSG_CHUNKFORM(4); break;
         default: return -1;
     }
 #undef MPSG_CHUNKFORM

@@ -68,7 +68,8 @@ struct WideWork {
 };
 
 // level 1 of [0, n) (ranks: sd): src -> dst tile by tile, the coarse counts
-// and offsets, and the coarse buckets' samples.  clears lists and tally
+// and offsets, and the coarse buckets' samples.  clears tally; lists are zero
+// before (launch_direct_sample)
 int launch_wide_level1(int rw, const void* src, void* dst, const LKey& lk, const SegDev& sd, const WideWork& w,
                        long long* checksum, hipStream_t st);
 // fine boundaries and level 2: src (level 1's dst) -> dst tile by tile, the
