@@ -1645,13 +1645,6 @@ static int plain_bucket_first(DevCtx& c, const CallShape& cs, const SegSortPlan&
 // records: kDirectMaxRecords.
 constexpr int64_t kDirectMaxRecords = (int64_t)kLBins * 4200;
 constexpr int64_t kDirectAvg = 2048;   // records per bucket while kLBins buckets suffice
-// Sample keys per bucket.  A bucket above 9216 records costs the call a wait, the
-// radix path and second counts, 370 instead of 270 us at 4.2 M records.  With
-// 16 keys it happens to one call in 1400 at kDirectMany records, one in 43 at
-// 4.0 M, one in 9 at the largest size; 20 keys, 2 to 7 us more, make it one in
-// 350 and 50 (24 keys: 10 us more).
-constexpr int kDirectKeys = 16, kDirectManyKeys = 20;
-constexpr int64_t kDirectMany = (int64_t)kLBins * 3500;
 static bool direct_asked(const CallShape& cs) {
     return (!g_faults || (g_faults & MPSORT_GPU_FAULT_KEEP_FORM)) && !cs.exchange && cs.first_mode == 0 &&
            cs.P <= kDirectMaxP && cs.ks.key_bytes <= 8;
@@ -1793,8 +1786,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
     DirectShape sh;
     direct_shape(cs, nin, nout, lscatter_tile(rw), &sh);
     sh.W = (int)std::min<int64_t>(kLBins, std::max<int64_t>(2, (n + kDirectAvg - 1) / kDirectAvg));
-    const int keys = n > kDirectMany ? kDirectManyKeys : kDirectKeys;
-    sh.S = std::min(kDirectMaxChunks, (keys * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
+    sh.S = std::min(kDirectMaxChunks, (16 * sh.W + kDirectChunk - 1) / kDirectChunk) * kDirectChunk;
 
     // ---- workspace
     DirectWork w;
@@ -1876,7 +1868,7 @@ static int run_direct(DevCtx& c, const CallShape& cs, const void* d_in, void* d_
         return rc;
     // The buckets above 4608 records (lists[2]) and the crowded ones: enqueued
     // with the rest where some are likely.  A bucket's size is estimated from
-    // 16 or 20 sample keys (a deviation of a quarter): at 2500 records on average
+    // 16 sample keys (a deviation of a quarter): at 2500 records on average
     // one bucket in a thousand is above, at 3900 one in five.  Waiting for
     // their number and counting a second time took 40 us of 289 (4,000,000 x
     // 16 B); where none are listed the two launches take 8.

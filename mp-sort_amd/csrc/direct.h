@@ -14,7 +14,7 @@ constexpr int kDirectMaxP = 64;         // ranks: one lane each
 constexpr int kSmallRecords = 8192;     // sorted by one launch
 constexpr int kRankRecords = 4096;      // of those, by counting every record's rank
 constexpr int kDirectChunk = 1024;      // sample keys sorted by one workgroup
-constexpr int kDirectMaxChunks = 20;    // sample chunks
+constexpr int kDirectMaxChunks = 16;    // sample chunks
 
 // the host tables of one call, passed by value (no upload)
 struct DirectShape {

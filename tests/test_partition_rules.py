@@ -1,6 +1,6 @@
-"""The sizes up to which a call takes the partition forms, and their samples,
-against the distribution of the sampled buckets (CPU only; the constants are
-read from the sources)."""
+"""The sizes up to which a call takes the two-level partition, against the
+distribution of its sampled buckets (CPU only; the constants are read from the
+sources)."""
 import os
 import re
 
@@ -15,12 +15,11 @@ def constants():
     for name in ("lsort.h", "direct.h", "wide.h", "api.cpp"):
         text = open(os.path.join(CSRC, name)).read()
         for k, v in re.findall(r"^constexpr \w+ (k\w+) = ([^;]+);", text, re.M):
-            for k, v in re.findall(r"(k\w+) = ([^,]+)", k + " = " + v):
-                v = re.sub(r"\(\w+_t\)", "", v).replace("/", "//")
-                try:
-                    c[k] = eval(v, {"__builtins__": {}}, dict(c))
-                except (NameError, SyntaxError):
-                    pass
+            v = re.sub(r"\(\w+_t\)", "", v).replace("/", "//")
+            try:
+                c[k] = eval(v, {"__builtins__": {}}, dict(c))
+            except (NameError, SyntaxError):
+                pass
     return c
 
 
@@ -48,20 +47,3 @@ def test_the_two_level_sort_reaches_its_largest_size(share):
 def test_the_chance_is_not_small_beyond():
     assert chance_of_a_missed_bucket(400000000) > 1e-3
     assert chance_of_a_missed_bucket(1 << 29) > 0.9
-
-
-def chance_of_an_oversized_bucket(n):
-    """of a one-level call with randomly ordered distinct keys: an upper bound
-    of the chance that some bucket is above the in-LDS capacity"""
-    W = min(C["kLBins"], max(2, -(-n // C["kDirectAvg"])))
-    keys = C["kDirectManyKeys"] if n > C["kDirectMany"] else C["kDirectKeys"]
-    S = min(C["kDirectMaxChunks"], -(-keys * W // C["kDirectChunk"])) * C["kDirectChunk"]
-    s = S // W
-    return W * beta.sf(C["kChunkCap"] / n, s, S - s + 1)
-
-
-def test_few_one_level_calls_have_an_oversized_bucket():
-    assert chance_of_an_oversized_bucket(C["kDirectMaxRecords"]) < 0.025
-    assert chance_of_an_oversized_bucket(4000000) < 4e-3
-    assert chance_of_an_oversized_bucket(C["kDirectMany"]) < 2e-3
-    assert chance_of_an_oversized_bucket(2000000) < 1e-9
