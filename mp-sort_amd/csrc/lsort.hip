@@ -592,10 +592,10 @@ __device__ __forceinline__ void lds_count_pass(const uint16_t* s_in, uint16_t* s
     __syncthreads();
 }
 
-// the 512 x 6 form hands a bucket on where a bin holds more than this: ranking 64
-// equal keys costs less than a second sort of the bucket (100 segments of
-// 100,000 x 8 B, each value 24 times: 379 us; with 32 records 576, with 256 the
-// same here and 420 instead of 343 on Zipf keys)
+// a form that hands buckets on (HAND) does so where a bin holds more than this:
+// ranking 64 equal keys costs less than a second sort of the bucket (16-byte
+// records, 800 segments of up to 30,000 with 1000 values: 531 us, with 32 671;
+// 100 segments of 100,000 Zipf keys: 395 us, with 256 459)
 constexpr int kHandOn = 64;
 constexpr uint32_t kIshOwn = 0x80000000u;  // of an interval's shift: its first key has a bin of its own
 
@@ -614,12 +614,12 @@ constexpr uint32_t kIshOwn = 0x80000000u;  // of an interval's shift: its first 
 // Records are grouped by bin with LDS atomics (in any order inside a bin),
 // and a record's final slot is its bin start + #{records of the bin with a
 // smaller key, or an equal key and a smaller position}: the stable order.
-// In the 9-record forms, a bin of more than kLongMin records that all hold
-// one key value (a duplicate-heavy key) is placed by counting instead:
-// slot = bin start + #{its records before this one in the bucket}, item by
-// item; the 512 x 6 form, whose registers are all in use, hands a bucket with
-// such bins to the 1024-thread form (result 2) when the sample holds a
-// repeated key.
+// A bin of more than kLongMin records that all hold one key value (a
+// duplicate-heavy key; looked for when the sample repeats one) is placed by
+// counting instead: slot = bin start + #{its records before this one in the
+// bucket}.  The 512 x 6 form of 16-byte records and of the merged SecondSort,
+// whose registers are all in use, hands a bucket on (result 2) when the sample
+// repeats a key and a bin holds more than kHandOn records.
 // Buckets with a bin above kRunMax records of several key values go to the
 // list for lsd_sort_kernel (result 1).  Record i of the bucket is item
 // i / BLOCK of thread i % BLOCK.
@@ -1090,7 +1090,7 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
         for (uint32_t l0 = 0; l0 < nlong; l0 += 64) {
             for (int q = tid; q < C::CAP / 2; q += C::B) reinterpret_cast<uint32_t*>(s_wc)[q] = 0;
             __syncthreads();
-            uint32_t mine = 0;  // the items placed in this round
+            uint32_t mine = 0;  // the items whose bins are among these 64
 #pragma unroll 1
             for (int k = 0; k * C::B < count; k++) {
                 const int i = k * C::B + tid;
@@ -1105,7 +1105,7 @@ __device__ __forceinline__ int sort_bucket_lds(const Src& src, uint32_t* __restr
                 }
                 if (L < 64u) {
                     const uint32_t rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
-                    // until the round's end: the bin's number and the lane's rank
+                    // until the counts are a prefix: the bin's number and the lane's rank
                     s_pos[i] = (uint16_t)((L << 6) | rank);
                     mine |= 1u << k;
                     if (rank == 0) s_wc[(k * C::W + wave) * 64 + L] = (uint16_t)__popcll(peers);
